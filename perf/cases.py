@@ -99,6 +99,7 @@ def draw(rng):
 # ------------------------------------------------------------------ what a program keeps
 _CTX = None
 _RULES = {}
+_STREAM = None
 
 
 def _context():
@@ -106,6 +107,15 @@ def _context():
     if _CTX is None:
         _CTX = S.Context(torch.cuda.current_device())
     return _CTX
+
+
+def _stream():
+    """The stream of every grids_step_noalloc call: calls on several streams would share its scratch array at once,
+    which its contract rules out."""
+    global _STREAM
+    if _STREAM is None:
+        _STREAM = torch.cuda.Stream()
+    return _STREAM
 
 
 def _rules(name):
@@ -221,7 +231,7 @@ def prepare(case, seed):
     draws = torch.bucketize(torch.rand(at, generator=gen, device="cuda"), edges, right=True)
     init = torch.tensor(ids, dtype=torch.int32, device="cuda")[draws].contiguous()
     arena = torch.zeros((2, at), dtype=torch.int32, device="cuda")
-    return dict(case=case, grids=grids, init=init, arena=arena, stream=torch.cuda.Stream(), rules=_rules(case["rules"]))
+    return dict(case=case, grids=grids, init=init, arena=arena, stream=_stream(), rules=_rules(case["rules"]))
 
 
 def run(state):
