@@ -116,8 +116,10 @@ int se_world_push_modification(se_world* w, const se_modification* m);
  * one step with that frame (frame 1 clears); queued modifications apply to the
  * first of them and are then cleared.  Plain kernel: one pass over HBM per step. */
 int se_world_step(se_world* w, uint32_t nsteps);
-/* Same result as se_world_step, advanced by the LDS temporal-blocked kernel in
- * launches of up to `sub` sub-steps (0 = autotuned choice). */
+/* Same result as se_world_step, advanced in launches of up to `sub` sub-steps (0 =
+ * autotuned choice): by the sliced kernels (bit planes, 32 blocks to a word) for
+ * longer runs of rule sets that have that form, else by the LDS temporal-blocked
+ * kernel. */
 int se_world_step_blocked(se_world* w, uint32_t nsteps, uint32_t sub);
 /* Kernel variant selection (no reference counterpart; the autotuner drives it):
  * plain_variant indexes the plain-kernel instantiations (rows per wavefront x
@@ -126,7 +128,9 @@ int se_world_step_blocked(se_world* w, uint32_t nsteps, uint32_t sub);
  * b=tile h, c=max sub-steps * 1000 + threads per workgroup; kind 2: a=the LDS
  * variant se_world_step_blocked uses for `index` sub-steps per launch; kind 3:
  * a=workgroups of LDS variant `index` resident at once on the device (the
- * batch's persistent launch shape), b=its LDS bytes per workgroup). */
+ * batch's persistent launch shape), b=its LDS bytes per workgroup).  The last
+ * LDS index of a rule set with a sliced form (bit planes, se_world_step_blocked's
+ * choice for longer runs) names those kernels: LDS bytes 0, single worlds only. */
 int se_world_set_variant(se_world* w, int32_t plain_variant, int32_t lds_variant);
 /* Tile sleeping of se_world_step_blocked (no reference counterpart; on by
  * default): an LDS tile whose cells, halo included, all hold one material whose

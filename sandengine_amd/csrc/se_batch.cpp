@@ -237,7 +237,7 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
             }
         }
         if (la < 0) la = t != b->tuned.end() ? (int)t->second.persistent : 0;
-        if (vi < 0 || vi >= (int)mod->lds.size()) return fail(SE_ERR_ARG, "LDS variant out of range");
+        if (vi < 0 || vi >= (int)mod->lds.size() || mod->lds[vi].first.sliced) return fail(SE_ERR_ARG, "LDS variant out of range");
         plans.emplace_back(new Plan());
         plans.back()->persistent = la == 1;
         int rc = make_plan(ctx, mod, vi, kk, g.second, *plans.back());
@@ -425,6 +425,7 @@ int se_batch_autotune(se_batch* b, uint32_t rounds, int32_t* best_variant, uint3
         uint32_t bk = 0;
         bool bp = false;
         for (int vi = 0; vi < (int)mod->lds.size(); vi++) {
+            if (mod->lds[vi].first.sliced) continue;  // single worlds only
             const int hb = mod->lds[vi].first.hb;
             for (uint32_t kk : {(uint32_t)hb, (uint32_t)std::max(2, hb / 2)})
             for (int la = 0; la < 2; la++) {

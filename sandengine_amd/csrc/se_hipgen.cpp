@@ -1,5 +1,7 @@
 #include "se_hipgen.hpp"
 
+#include "se_net.hpp"
+
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -15,6 +17,9 @@ namespace se {
 
 static const char* kKernelTemplates =
 #include "se_kernels_src.inc"
+    ;
+static const char* kSlicedTemplates =
+#include "se_sliced_src.inc"
     ;
 
 namespace {
@@ -915,13 +920,373 @@ std::string hip_rules_source(const ParsingResult& r, HipGenInfo* info, bool allo
     return o.str();
 }
 
+// ------------------------------------------------------------------ sliced form
+// The rule chain over bit planes: a cell is `planes` words whose bit i belongs to
+// block i, a condition is a word, an action a select under that word.  One
+// evaluation advances 32 blocks.
+namespace {
+
+constexpr int kSlicedMaxMaterials = 16, kSlicedMaxClasses = 8;
+
+struct NotSliced {};  // the rule set reads something that has no word form
+
+class Slicer {
+public:
+    Slicer(const Ctx& ctx, int planes, const std::vector<int>& code) : ctx_(ctx), K_(planes), code_(code) {
+        for (int c = 0; c < 4; c++)
+            for (int k = 0; k < K_; k++) cell_[c].push_back(net.input());
+    }
+    Net net;
+    std::vector<std::pair<int, uint32_t>> classes;  // inputs after the cells, in order of first use
+    std::vector<Net::Lit> class_lit;
+
+    Net::Lit below(int lane, int64_t t) {  // hash lane <= t
+        if (t < 0) return Net::kZero;
+        if (t >= 0xFFFFFFFFll) return Net::kOne;
+        for (size_t i = 0; i < classes.size(); i++)
+            if (classes[i] == std::make_pair(lane, (uint32_t)t)) return class_lit[i];
+        classes.push_back({lane, (uint32_t)t});
+        class_lit.push_back(net.input());
+        return class_lit.back();
+    }
+
+    // simulate() after the cell reads (falling_sand.glsl:61-118), as se_block_h
+    std::vector<Net::Lit> chain(const ParsingResult& r) {
+        std::vector<bool> fixed(ctx_.nmat);
+        for (int i = 0; i < ctx_.nmat; i++) fixed[i] = ctx_.mat_type[i] == 1 || ctx_.mat_type[i] == 2;
+        fixed_of_ = fixed;
+        State in;
+        for (int c = 0; c < 4; c++) {
+            in.cell[c] = cell_[c];
+            in.fixed[c] = holds(in.cell[c], fixed);
+        }
+        State s = in;
+        const Net::Lit mirror = below(0, rand_threshold(0.5f, false));
+        swap(s, 0, 1, mirror);
+        swap(s, 2, 3, mirror);
+        for (auto& rl : r.rules)
+            if (rl.used && rl.ruletype == RuleType::Mirrored) rule(rl, Net::kOne, s);
+        swap(s, 0, 1, mirror);
+        swap(s, 2, 3, mirror);
+        for (auto& rl : r.rules)
+            if (rl.used && rl.ruletype != RuleType::Mirrored) rule(rl, Net::inv(mirror), s);
+        std::vector<Net::Lit> out;
+        for (int c = 0; c < 4; c++) out.insert(out.end(), s.cell[c].begin(), s.cell[c].end());
+        // a block of four EMPTY cells stays as it is (falling_sand.glsl:77-79): kept
+        // out of the network where the rules leave it alone anyway
+        std::vector<uint32_t> words(net.inputs(), 0u), got;
+        for (int c = 0; c < 4; c++)
+            for (int k = 0; k < K_; k++) words[c * K_ + k] = (code_[0] >> k) & 1 ? ~0u : 0u;
+        bool stays = true;
+        for (uint32_t m = 0; m < (1u << classes.size()); m += 32) {
+            for (size_t j = 0; j < classes.size(); j++) {
+                uint32_t w = 0;
+                for (uint32_t i = 0; i < 32; i++) w |= (((m + i) >> j) & 1u) << i;
+                words[4 * K_ + j] = w;
+            }
+            net.eval(words, out, got);
+            for (size_t i = 0; i < out.size(); i++) stays = stays && got[i] == words[i];
+        }
+        if (!stays) {
+            std::vector<bool> empty(ctx_.nmat);
+            empty[0] = true;
+            Net::Lit all = Net::kOne;
+            for (int c = 0; c < 4; c++) all = net.land(all, holds(in.cell[c], empty));
+            for (int c = 0; c < 4; c++)
+                for (int k = 0; k < K_; k++) out[c * K_ + k] = net.mux(all, in.cell[c][k], out[c * K_ + k]);
+        }
+        return out;
+    }
+
+private:
+    using Cell = std::vector<Net::Lit>;
+    struct State {
+        Cell cell[4];
+        Net::Lit fixed[4];  // the cell refuses swaps; a swap never moves such a cell
+    };
+    const Ctx& ctx_;
+    int K_;
+    std::vector<int> code_;
+    Cell cell_[4];
+    std::vector<bool> fixed_of_;
+
+    template <class F>  // f(material id) over the codes of one cell
+    Net::Lit table(const Cell& c, F f) {
+        std::vector<char> tt((size_t)1 << K_, 2);
+        for (int m = 0; m < ctx_.nmat; m++) tt[code_[m]] = (char)f(m);
+        return net.func(c, tt);
+    }
+    Net::Lit holds(const Cell& c, const std::vector<bool>& set) {
+        return table(c, [&](int m) { return set[m] ? 1 : 0; });
+    }
+    // a cell's code with equal densities sharing the lowest of their codes (codes
+    // ascend with the density wherever ranks are compared)
+    Cell rank(const Cell& c) {
+        Cell r;
+        for (int k = 0; k < K_; k++)
+            r.push_back(table(c, [&](int m) {
+                int low = code_[m];
+                for (int o = 0; o < ctx_.nmat; o++)
+                    if (ctx_.dens[o] == ctx_.dens[m]) low = std::min(low, code_[o]);
+                return (low >> k) & 1;
+            }));
+        return r;
+    }
+    Net::Lit less(const Cell& a, const Cell& b) {
+        Net::Lit r = Net::kZero;
+        for (int k = 0; k < K_; k++) r = net.mux(net.lxor(a[k], b[k]), b[k], r);
+        return r;
+    }
+    Net::Lit equal(const Cell& a, const Cell& b) {
+        Net::Lit r = Net::kOne;
+        for (int k = 0; k < K_; k++) r = net.land(r, Net::inv(net.lxor(a[k], b[k])));
+        return r;
+    }
+
+    Net::Lit cond(const Ex& e, const State& s) {
+        const unsigned cm = cells_used(e);
+        const bool rnd = uses_rand(e);
+        if (!rnd && cm == 0) {
+            Env v{};
+            return eval_bool(e, v, ctx_) ? Net::kOne : Net::kZero;
+        }
+        if (!rnd && (cm & (cm - 1)) == 0) {
+            const int k = __builtin_ctz(cm);
+            return table(s.cell[k], [&](int m) {
+                Env v{};
+                v.c[k] = m;
+                return eval_bool(e, v, ctx_) ? 1 : 0;
+            });
+        }
+        switch (e.k) {
+            case Ex::And: { const Net::Lit a = cond(*e.a, s); return net.land(a, cond(*e.b, s)); }
+            case Ex::Or: { const Net::Lit a = cond(*e.a, s); return net.lor(a, cond(*e.b, s)); }
+            case Ex::Not: return Net::inv(cond(*e.a, s));
+            case Ex::Cmp: return compare(e, s);
+            default: gen_error("internal: unexpected boolean node");
+        }
+    }
+    Net::Lit compare(const Ex& e, const State& s) {
+        if (e.a->ty == Ty::Bool) {
+            const Net::Lit x = cond(*e.a, s), d = net.lxor(x, cond(*e.b, s));
+            return e.op == 4 ? Net::inv(d) : d;
+        }
+        if (e.a->ty == Ty::Mat) {  // two cells (a cell against a constant is a table of one cell)
+            const Net::Lit q = equal(s.cell[e.a->cell], s.cell[e.b->cell]);
+            return e.op == 4 ? q : Net::inv(q);
+        }
+        if (e.a->k == Ex::Dens && e.b->k == Ex::Dens) {
+            const Cell a = rank(s.cell[e.a->cell]), b = rank(s.cell[e.b->cell]);
+            switch (e.op) {
+                case 0: return less(a, b);
+                case 1: return Net::inv(less(b, a));
+                case 2: return less(b, a);
+                case 3: return Net::inv(less(a, b));
+                case 4: return equal(a, b);
+                default: return Net::inv(equal(a, b));
+            }
+        }
+        if (!uses_rand(e)) {  // any other compare of two cells' numbers: a table over both codes
+            const unsigned cm = cells_used(e);
+            const int x = __builtin_ctz(cm), y = 31 - __builtin_clz(cm);
+            if (__builtin_popcount(cm) != 2) throw NotSliced();
+            Cell both = s.cell[x];
+            both.insert(both.end(), s.cell[y].begin(), s.cell[y].end());
+            std::vector<char> tt((size_t)1 << (2 * K_), 2);
+            for (int a = 0; a < ctx_.nmat; a++)
+                for (int b = 0; b < ctx_.nmat; b++) {
+                    Env v{};
+                    v.c[x] = a;
+                    v.c[y] = b;
+                    tt[(size_t)code_[a] | ((size_t)code_[b] << K_)] = eval_bool(e, v, ctx_) ? 1 : 0;
+                }
+            return net.func(both, tt);
+        }
+        const Ex* rn = nullptr;
+        const Ex* cst = nullptr;
+        int op = e.op;
+        if (e.a->k == Ex::Rand && !uses_rand(*e.b) && cells_used(*e.b) == 0) { rn = e.a.get(); cst = e.b.get(); }
+        else if (e.b->k == Ex::Rand && !uses_rand(*e.a) && cells_used(*e.a) == 0) {
+            rn = e.b.get(); cst = e.a.get();
+            static const int flip[] = {2, 3, 0, 1, 4, 5};
+            op = flip[op];
+        }
+        if (!rn) throw NotSliced();
+        Env v{};
+        const float c = eval_num(*cst, v, ctx_);
+        if (std::isnan(c)) return op == 5 ? Net::kOne : Net::kZero;
+        const int64_t tle = rand_threshold(c, true), tlt = rand_threshold(c, false);
+        const int l = rn->lane;
+        switch (op) {
+            case 0: return below(l, tlt);
+            case 1: return below(l, tle);
+            case 2: return Net::inv(below(l, tle));
+            case 3: return Net::inv(below(l, tlt));
+            case 4: return net.land(Net::inv(below(l, tlt)), below(l, tle));
+            default: return Net::inv(net.land(Net::inv(below(l, tlt)), below(l, tle)));
+        }
+    }
+
+    // guarded swap (operations.glsl:16-23) where `m` holds
+    void swap(State& s, int a, int b, Net::Lit m) {
+        const Net::Lit ok = net.land(m, net.land(Net::inv(s.fixed[a]), Net::inv(s.fixed[b])));
+        for (int k = 0; k < K_; k++) {
+            const Net::Lit x = s.cell[a][k], y = s.cell[b][k];
+            s.cell[a][k] = net.mux(ok, y, x);
+            s.cell[b][k] = net.mux(ok, x, y);
+        }
+    }
+    void set(State& s, int a, int mat, Net::Lit m) {
+        for (int k = 0; k < K_; k++)
+            s.cell[a][k] = net.mux(m, (code_[mat] >> k) & 1 ? Net::kOne : Net::kZero, s.cell[a][k]);
+        s.fixed[a] = net.mux(m, fixed_of_[mat] ? Net::kOne : Net::kZero, s.fixed[a]);
+    }
+    // the action lines of emit_actions, under the word m
+    void actions(const std::string& text, State& s, Net::Lit m) {
+        std::istringstream is(emit_actions(text, ctx_, ""));
+        std::string line;
+        while (std::getline(is, line)) {
+            int a = 0, b = 0;
+            if (std::sscanf(line.c_str(), "SE_GSWAP(c%d, c%d);", &a, &b) == 2) swap(s, a, b, m);
+            else if (std::sscanf(line.c_str(), "c%d = %du;", &a, &b) == 2) set(s, a, b, m);
+            else gen_error("internal: action '" + line + "'");
+        }
+    }
+    // One rule where `on` holds.  The levels exclude each other, so every level's
+    // condition reads the cells as the rule found them.
+    void rule(const SandRule& r, Net::Lit on, State& s) {
+        const State in = s;
+        Net::Lit rest = on;
+        if (r.precondition) rest = net.land(rest, cond(*ExprParser(*r.precondition, ctx_).parse(), in));
+        std::vector<Level> lv;
+        std::string fin;
+        bool has_fin;
+        levels_of(r, lv, &fin, &has_fin);
+        for (auto& l : lv) {
+            const std::string text = (l.p == 1.0f ? std::string() : "rand.y <= " + fmt_f32(l.p) + " && ") + l.cond;
+            const Net::Lit c = cond(*ExprParser(text, ctx_).parse(), in);
+            actions(l.act, s, net.land(rest, c));
+            rest = net.land(rest, Net::inv(c));
+        }
+        if (has_fin) actions(fin, s, rest);
+    }
+};
+
+}  // namespace
+
+std::string hip_sliced_source(const ParsingResult& r, SlicedInfo& out) {
+    out = SlicedInfo();
+    const Ctx ctx = build_ctx(r);
+    const int n = ctx.nmat;
+    if (n > kSlicedMaxMaterials || n < 3) return "";
+    for (float d : ctx.dens)
+        if (std::isnan(d)) return "";
+    int K = 1;
+    while ((1 << K) < n) K++;
+    // codes ascend with the density (ties by id), so that comparing densities
+    // compares codes; id order where no rule compares them (no remapping then)
+    Emitter em(ctx);
+    for (auto& rl : r.rules)
+        if (rl.used) emit_rule(rl, ctx, em);
+    std::vector<int> by(n), code(n);
+    for (int i = 0; i < n; i++) by[i] = i;
+    if (em.rank_used)
+        std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return ctx.dens[a] < ctx.dens[b]; });
+    for (int i = 0; i < n; i++) code[by[i]] = i;
+    Slicer sl(ctx, K, code);
+    std::vector<Net::Lit> outs;
+    try {
+        outs = sl.chain(r);
+    } catch (const NotSliced&) {
+        return "";
+    }
+    const int P = (int)sl.classes.size();
+    if (P > kSlicedMaxClasses) return "";
+    // does any block change a WALL cell?  (every tuple of codes, every class word)
+    bool kept = true;
+    {
+        std::vector<uint32_t> in(sl.net.inputs()), got;
+        for (int t = 0; t < n * n * n * n && kept; t++) {
+            const int id[4] = {t % n, t / n % n, t / n / n % n, t / n / n / n};
+            bool wall = false;
+            for (int c = 0; c < 4; c++) {
+                wall |= id[c] == 2;
+                for (int k = 0; k < K; k++) in[c * K + k] = (code[id[c]] >> k) & 1 ? ~0u : 0u;
+            }
+            if (!wall) continue;
+            for (uint32_t m = 0; m < (1u << P); m += 32) {
+                for (int j = 0; j < P; j++) {
+                    uint32_t w = 0;
+                    for (uint32_t i = 0; i < 32; i++) w |= (((m + i) >> j) & 1u) << i;
+                    in[4 * K + j] = w;
+                }
+                sl.net.eval(in, outs, got);
+                for (int c = 0; c < 4; c++)
+                    for (int k = 0; k < K && id[c] == 2; k++) kept = kept && got[c * K + k] == in[c * K + k];
+            }
+        }
+    }
+    out.ok = true;
+    out.planes = K;
+    out.code = code;
+    out.classes = sl.classes;
+    out.wall_kept = kept;
+    std::vector<std::string> in_names, out_names;
+    for (int c = 0; c < 4; c++)
+        for (int k = 0; k < K; k++) {
+            in_names.push_back("c" + std::to_string(c) + "[" + std::to_string(k) + "]");
+            out_names.push_back("n" + std::to_string(c) + "_" + std::to_string(k));
+        }
+    for (int j = 0; j < P; j++) in_names.push_back("h[" + std::to_string(j) + "]");
+    std::string body;
+    out.tables = sl.net.emit(outs, in_names, [&] {
+        std::vector<std::string> decl;
+        for (auto& o : out_names) decl.push_back("const unsigned int " + o);
+        return decl;
+    }(), "    ", body);
+    std::ostringstream o;
+    o << "// ---- sliced form: " << K << " bit planes per cell, " << P << " hash planes, " << out.tables
+      << " tables per 32 blocks\n";
+    o << "template <int TT>\n__device__ __forceinline__ unsigned int se_lut3(unsigned int a, unsigned int b, unsigned int "
+         "c) {\n    return __builtin_amdgcn_bitop3_b32(a, b, c, TT);\n}\n";
+    o << "#define SE_SL_K " << K << "\n#define SE_SL_P " << P << "\n#define SE_SL_KEEP " << (kept ? 1 : 0) << "\n";
+    o << "#define SE_SL_REMAP " << (em.rank_used ? 1 : 0) << "\n";
+    o << "#define SE_SL_EMPTY " << code[0] << "u\n#define SE_SL_NULL " << code[1] << "u\n#define SE_SL_WALL " << code[2]
+      << "u\n";
+    // code of id i and id of code i as bytes of four words
+    for (int dir = 0; dir < 2; dir++) {
+        uint32_t w[4] = {0, 0, 0, 0};
+        for (int i = 0; i < 16; i++) {
+            const int v = i < n ? (dir == 0 ? code[i] : by[i]) : (dir == 0 ? code[1] : 1);
+            w[i / 4] |= (uint32_t)v << (8 * (i & 3));
+        }
+        for (int j = 0; j < 4; j++) o << "#define SE_SL_" << (dir == 0 ? "CODE" : "ID") << j << " " << hex_u32(w[j]) << "\n";
+    }
+    // hash planes: lane of each, and per lane its thresholds
+    o << "__device__ __forceinline__ void se_sliced_classes(const unsigned int* h, bool* c) {\n";
+    for (int j = 0; j < P; j++)
+        o << "    c[" << j << "] = h[" << sl.classes[j].first << "] <= " << hex_u32(sl.classes[j].second) << ";\n";
+    o << "}\n";
+    o << "__device__ __forceinline__ constexpr bool se_sliced_lane(int l) {\n    return false";
+    for (int l = 0; l < 4; l++)
+        for (auto& c : sl.classes)
+            if (c.first == l) { o << " || l == " << l; break; }
+    o << ";\n}\n";
+    o << "__device__ __forceinline__ void se_sliced_block(unsigned int* c0, unsigned int* c1, unsigned int* c2, "
+         "unsigned int* c3, const unsigned int* h) {\n" << body;
+    for (int c = 0; c < 4; c++)
+        for (int k = 0; k < K; k++) o << "    " << in_names[c * K + k] << " = " << out_names[c * K + k] << ";\n";
+    o << "}\n";
+    return o.str();
+}
+
 std::string lds_kernel_name(const LdsVariant& v) {
     return "se_step_lds_" + std::to_string(v.tw) + "x" + std::to_string(v.th) + "_h" + std::to_string(v.hb) + "_t" +
            std::to_string(v.nt);
 }
 
 std::string hip_program_source(const ParsingResult& r, const std::vector<LdsVariant>& lds, bool allow_ctable,
-                               uint64_t ct_x_words) {
+                               uint64_t ct_x_words, SlicedInfo* sliced) {
     std::string s = hip_rules_source(r, nullptr, allow_ctable, ct_x_words);
     s += "\n";
     s += kKernelTemplates;
@@ -929,6 +1294,12 @@ std::string hip_program_source(const ParsingResult& r, const std::vector<LdsVari
     for (auto& v : lds)
         s += "SE_LDS_KERNEL(" + std::to_string(v.tw) + ", " + std::to_string(v.th) + ", " + std::to_string(v.hb) + ", " +
              std::to_string(v.nt) + ")\n";
+    if (!lds.empty()) {  // not in the small module that only enumerates the coded table
+        SlicedInfo local;
+        SlicedInfo& sl = sliced ? *sliced : local;
+        const std::string rules = hip_sliced_source(r, sl);
+        if (sl.ok) s += rules + kSlicedTemplates;
+    }
     return s;
 }
 

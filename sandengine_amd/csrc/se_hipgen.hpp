@@ -21,6 +21,18 @@ namespace se {
 
 struct LdsVariant {
     int tw, th, hb, nt;  // tile width/height, halo (= max sub-steps), threads per workgroup
+    bool sliced = false; // the sliced kernels (se_sliced.hip), not an LDS instantiation
+};
+
+// The sliced form of a rule set: cells as bit planes, 32 blocks to a word, the
+// rule chain as a Boolean network over them (se_sliced.hip).
+struct SlicedInfo {
+    bool ok = false;      // at most 16 materials, rand only in threshold compares
+    int planes = 0;       // bit planes of a cell code
+    int tables = 0;       // three-input tables of the network (instructions per word of 32 blocks)
+    std::vector<int> code;                          // material id -> code
+    std::vector<std::pair<int, uint32_t>> classes;  // hash planes: bit set when the lane is <= the threshold
+    bool wall_kept = false;                         // no block changes a WALL cell
 };
 
 struct HipGenInfo {
@@ -32,6 +44,7 @@ struct HipGenInfo {
     bool ctable = false; // coded-table candidate (SE_TBL 2): fit checked when the rule set is loaded
     int ct_D = 0;        // materials the coded table covers (all but NULL and WALL)
     int ct_R = 0;        // classes of hash lanes 1..3
+    SlicedInfo sliced;   // filled by hip_program_source
 };
 
 // Generated device code for the rule set (SE_NMAT, se_fixed, se_block, ...).
@@ -40,9 +53,14 @@ struct HipGenInfo {
 std::string hip_rules_source(const ParsingResult& r, HipGenInfo* info = nullptr, bool allow_ctable = true,
                              uint64_t ct_x_words = 0);
 
-// Full translation unit: rules + kernel templates + LDS instantiations.
+// The sliced form of the rule set (out.ok false where it has none) and its device
+// code: constants, the code tables and se_sliced_block.
+std::string hip_sliced_source(const ParsingResult& r, SlicedInfo& out);
+
+// Full translation unit: rules + kernel templates + LDS instantiations + the
+// sliced form and its kernels.
 std::string hip_program_source(const ParsingResult& r, const std::vector<LdsVariant>& lds, bool allow_ctable = true,
-                               uint64_t ct_x_words = 0);
+                               uint64_t ct_x_words = 0, SlicedInfo* sliced = nullptr);
 
 // Name of an LDS kernel instantiation.
 std::string lds_kernel_name(const LdsVariant& v);

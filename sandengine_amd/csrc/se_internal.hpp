@@ -55,6 +55,14 @@ struct DeviceGuard {
     }
 };
 
+// The sliced kernels of a module (se_sliced.hip); ok false where the rule set has
+// no sliced form.
+struct SlicedKernels {
+    bool ok = false;
+    int planes = 0, classes = 0;  // bit planes of a cell, hash planes of a frame
+    hipFunction_t pack = nullptr, unpack = nullptr, hash = nullptr;
+    hipFunction_t step[3] = {};   // words x rows of a lane: 2x2, 4x2, 4x4
+};
 
 }  // namespace se_rt
 
@@ -76,6 +84,7 @@ struct se_module {
     hipFunction_t plain_v[6] = {};  // se_step_plain_r{1,2,4}_nt{0,1}
     std::vector<std::pair<se::LdsVariant, hipFunction_t>> lds;
     std::vector<hipFunction_t> batch;  // se_batch_lds_* parallel to `lds`
+    se_rt::SlicedKernels sliced;
     int device = 0;
     ~se_module() {
         if (mod) {
@@ -100,6 +109,12 @@ struct se_ctx {
     void* staging = nullptr;
     hipEvent_t staging_done = nullptr;
     std::mutex staging_mu;
+    // packed grids and hash planes of the sliced kernels (se_sliced.cpp), as large
+    // as the largest call needed; freed with the context's last world
+    std::mutex sliced_mu;
+    void* sliced_mem = nullptr;
+    size_t sliced_bytes = 0;
+    int worlds = 0;  // live worlds made by se_world_create (under sliced_mu)
 };
 
 struct se_ruleset {

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "se_internal.hpp"
+#include "se_sliced.hpp"
 
 namespace {
 thread_local std::string g_err;
@@ -126,7 +127,7 @@ int gen_source(const se::ParsingResult& pr, std::string& src, se::HipGenInfo* in
         se::hip_rules_source(pr, &gi, allow_ctable, ct_x_words);
         src = se::hip_program_source(pr, with_lds ? variants_for(table_words_of(gi, ct_x_words))
                                                   : std::vector<se::LdsVariant>(),
-                                     allow_ctable, ct_x_words);
+                                     allow_ctable, ct_x_words, &gi.sliced);
     } catch (const se::LangError& e) {
         return fail(SE_ERR_CODEGEN, e.what());
     } catch (const std::exception& e) {
@@ -412,6 +413,27 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         else if (!enough && !d_enough && m->lds_waves[i] > m->lds_waves[d]) m->default_lds = (int)i;
     }
     if (m->default_lds < 0) m->default_lds = 0;
+    if (info.sliced.ok) {
+        se_rt::SlicedKernels& K = m->sliced;
+        HIPCHECK(hipModuleGetFunction(&K.pack, m->mod, "se_sl_pack"));
+        HIPCHECK(hipModuleGetFunction(&K.unpack, m->mod, "se_sl_unpack"));
+        HIPCHECK(hipModuleGetFunction(&K.hash, m->mod, "se_sl_hash"));
+        HIPCHECK(hipModuleGetFunction(&K.step[0], m->mod, "se_sl_step_2x2"));
+        HIPCHECK(hipModuleGetFunction(&K.step[1], m->mod, "se_sl_step_4x2"));
+        HIPCHECK(hipModuleGetFunction(&K.step[2], m->mod, "se_sl_step_4x4"));
+        K.planes = info.sliced.planes;
+        K.classes = (int)info.sliced.classes.size();
+        K.ok = true;
+        // listed after the LDS instantiations (never the default among them)
+        m->lds.push_back({{128, 128, 32, 64, true}, K.step[0]});
+        m->batch.push_back(nullptr);
+        m->lds_bytes.push_back(0);
+        int per_cu = 0, cus = 0;
+        HIPCHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, K.step[0], 64, 0));
+        HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+        m->lds_grid.push_back(std::max(8, (std::max(per_cu, 1) * cus) & ~7));
+        m->lds_waves.push_back(std::max(per_cu, 1));
+    }
     std::lock_guard<std::mutex> lk(ctx->mu);
     ctx->cache[key] = {src, m};
     out = m;
@@ -526,7 +548,7 @@ const std::pair<se::LdsVariant, hipFunction_t>* pick_lds(se_world* w, uint32_t s
     }
     const std::pair<se::LdsVariant, hipFunction_t>* best = nullptr;
     for (auto& p : L) {
-        if (sub != 0 && (uint32_t)p.first.hb < sub) continue;
+        if (p.first.sliced || (sub != 0 && (uint32_t)p.first.hb < sub)) continue;
         if (!best || p.first.hb < best->first.hb) best = &p;
     }
     return best;
@@ -584,6 +606,22 @@ int blocked_steps(se_world* w, uint32_t nsteps, uint32_t sub) {
     }
     auto* v = pick_lds(w, sub);
     if (!v) return fail(SE_ERR_ARG, "no LDS variant supports " + std::to_string(sub) + " sub-steps");
+    if (v->first.sliced || (w->lds_variant < 0 && se_rt::sliced_pays(w, nsteps))) {
+        // the sliced kernels take neither the clearing frame nor modifications: the
+        // step that carries them is a plain one
+        if (nsteps && (w->frame + 1 == 1 || !w->pending.empty())) {
+            int rc = plain_step(w);
+            if (rc) return rc;
+            nsteps--;
+        }
+        bool done = nsteps == 0;
+        int rc = done ? SE_OK : se_rt::sliced_steps(w, nsteps, sub, &done);
+        if (rc || done) return rc;
+        if (v->first.sliced) {  // no memory for them: the default LDS tile
+            v = &w->mod->lds[w->mod->default_lds];
+            sub = std::min(sub, (uint32_t)v->first.hb);
+        }
+    }
     uint32_t k = sub ? sub : (uint32_t)v->first.hb;
     // a world inside one tile keeps its WALL border in LDS: no halo limit on k
     const bool single = w->W <= (uint32_t)v->first.tw && w->H <= (uint32_t)v->first.th;
@@ -702,6 +740,7 @@ void se_ctx_destroy(se_ctx* ctx) {
             hipEventDestroy(ctx->staging_done);
         }
         if (ctx->staging) hipHostFree(ctx->staging);
+        hipFree(ctx->sliced_mem);
     }
     delete ctx;
 }
@@ -799,6 +838,10 @@ int se_world_create(se_ctx* ctx, const se_ruleset* rs, uint32_t w, uint32_t h, s
         hipGetLastError();
         return fail(SE_ERR_OOM, "hipMalloc of " + std::to_string(2 * bytes) + " bytes failed");
     }
+    {
+        std::lock_guard<std::mutex> lk(ctx->sliced_mu);
+        ctx->worlds++;
+    }
     int rc = launch_fill(W, W->buf[0], 0u);
     if (!rc) rc = launch_fill(W, W->buf[1], 0u);
     if (rc) {
@@ -825,6 +868,12 @@ void se_world_destroy(se_world* w) {
         hipFree(w->noise);
         hipFree(w->d_sleep[0]);
         hipFree(w->d_sleep[1]);
+        std::lock_guard<std::mutex> lk(w->ctx->sliced_mu);
+        if (w->owns && --w->ctx->worlds == 0) {
+            hipFree(w->ctx->sliced_mem);
+            w->ctx->sliced_mem = nullptr;
+            w->ctx->sliced_bytes = 0;
+        }
     }
     delete w;
 }
