@@ -1262,11 +1262,15 @@ std::string hip_sliced_source(const ParsingResult& r, SlicedInfo& out) {
         }
         for (int j = 0; j < 4; j++) o << "#define SE_SL_" << (dir == 0 ? "CODE" : "ID") << j << " " << hex_u32(w[j]) << "\n";
     }
-    // hash planes: lane of each, and per lane its thresholds
-    o << "__device__ __forceinline__ void se_sliced_classes(const unsigned int* h, bool* c) {\n";
-    for (int j = 0; j < P; j++)
-        o << "    c[" << j << "] = h[" << sl.classes[j].first << "] <= " << hex_u32(sl.classes[j].second) << ";\n";
-    o << "}\n";
+    // hash planes: the lane and the threshold of each
+    for (int part = 0; part < 2; part++) {
+        o << "__device__ __forceinline__ constexpr unsigned int se_sliced_class_" << (part == 0 ? "lane" : "max")
+          << "(int p) {\n    return ";
+        for (int j = 0; j + 1 < P; j++)
+            o << "p == " << j << " ? " << (part == 0 ? std::to_string(sl.classes[j].first) + "u" : hex_u32(sl.classes[j].second))
+              << " : ";
+        o << (part == 0 ? std::to_string(sl.classes[P - 1].first) + "u" : hex_u32(sl.classes[P - 1].second)) << ";\n}\n";
+    }
     o << "__device__ __forceinline__ constexpr bool se_sliced_lane(int l) {\n    return false";
     for (int l = 0; l < 4; l++)
         for (auto& c : sl.classes)

@@ -61,7 +61,7 @@ struct SlicedKernels {
     bool ok = false;
     int planes = 0, classes = 0;  // bit planes of a cell, hash planes of a frame
     hipFunction_t pack = nullptr, unpack = nullptr, hash = nullptr;
-    hipFunction_t step[3] = {};   // words x rows of a lane: 2x2, 4x2, 4x4
+    hipFunction_t step[2] = {};   // words x rows of a lane: 2x2, 4x2
 };
 
 }  // namespace se_rt

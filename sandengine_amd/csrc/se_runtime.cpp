@@ -420,7 +420,6 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         HIPCHECK(hipModuleGetFunction(&K.hash, m->mod, "se_sl_hash"));
         HIPCHECK(hipModuleGetFunction(&K.step[0], m->mod, "se_sl_step_2x2"));
         HIPCHECK(hipModuleGetFunction(&K.step[1], m->mod, "se_sl_step_4x2"));
-        HIPCHECK(hipModuleGetFunction(&K.step[2], m->mod, "se_sl_step_4x4"));
         K.planes = info.sliced.planes;
         K.classes = (int)info.sliced.classes.size();
         K.ok = true;

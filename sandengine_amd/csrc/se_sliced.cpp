@@ -20,7 +20,7 @@ constexpr size_t kHashBudget = 128u << 20;  // hash planes made ahead, unless on
 struct Tile {
     int nw, r;
 };
-constexpr Tile kTiles[3] = {{2, 2}, {4, 2}, {4, 4}};  // as instantiated in se_sliced.hip
+constexpr Tile kTiles[2] = {{2, 2}, {4, 2}};  // as instantiated in se_sliced.hip
 
 template <typename... A>
 int launch2(hipFunction_t f, unsigned gx, unsigned gy, unsigned block, hipStream_t s, A... args) {
@@ -49,10 +49,10 @@ se_rt::SlicedShape se_rt::sliced_shape(uint32_t W, uint32_t H, uint32_t sub) {
     // The tile and the depth of a launch, by how many 2x2 tiles (64 useful columns and
     // rows at 32 sub-steps) the world makes.  Up to one a SIMD the launches are a
     // serial chain of sub-steps: the smallest tile and the deepest launch
-    // (1000x700: 162 us for 200 steps, 249 with 4x2, 178 with 16 sub-steps).  Beyond
+    // (1000x700: 133 us for 200 steps, 206 with 4x2, 153 with 16 sub-steps).  Beyond
     // that the rows given up count, and from 8 a SIMD on the columns too
-    // (4096^2, 200 steps: 541 us with 2x2 and 16, 563 with either 4x2 or 32;
-    // 16384^2, 100 steps: 3.35 ms with 4x2 and 16, 3.52 with 2x2).
+    // (4096^2, 200 steps: 512 us with 2x2 and 16, 531 with 4x2, 534 with 32;
+    // 16384^2, 100 steps: 1.65 ms with 4x2 and 16, 2.04 with 2x2, 1.97 with 32).
     const size_t few = (size_t)((W + 63) / 64) * ((H + 63) / 64);
     const int i = few > 8192 ? 1 : 0;
     const uint32_t deep = few > 1024 ? 16 : 32;
@@ -78,24 +78,59 @@ void se_rt::sliced_geometry(const SlicedShape& s, uint32_t W, uint32_t H, Sliced
     }
     g.hcols = (s.tiles_x - 1) * (2 * s.nw - 2) + 2 * s.nw;
     g.rows = ((s.tiles_y - 1) * (64 * s.r - 2 * s.halo) + 64 * s.r + 63) & ~63;
-    g.wcols = g.hcols / 2;
     g.brows = g.rows / 2;
 }
 
 size_t se_rt::sliced_packed_bytes(const SlicedGrid& g, int planes) {
     return ((size_t)g.hcols * g.rows * 2 * planes * sizeof(uint16_t) + 255) & ~(size_t)255;
 }
-size_t se_rt::sliced_frame_bytes(const SlicedGrid& g, int classes) {
-    return (size_t)g.wcols * g.brows * classes * sizeof(uint32_t);
+
+size_t se_rt::sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int classes) {
+    const int wcols = g.hcols / 2;
+    g.hash_frame0 = frame0;
+    // shared form: the range of n of each parity over the frames, and the words of b
+    // that cover it (one more than a tile's last word, for the shifted read)
+    int64_t lo[2] = {0, 0}, hi[2] = {-1, -1};
+    for (uint32_t i = 0; i < nf; i++) {
+        const int64_t f = (int64_t)frame0 + i;
+        const int ox = (int)(f & 1), oy = (f & 3) == 1 || (f & 3) == 2;
+        const int64_t n = 461ll * (-ox - g.xpad) + 2131ll * (oy - g.ypad) + 4541161ll * f;
+        const int c = (int)((ox + oy + f) & 1);
+        if (hi[c] < lo[c]) lo[c] = hi[c] = n;
+        lo[c] = std::min(lo[c], n);
+        hi[c] = std::max(hi[c], n);
+    }
+    int64_t words = 0;
+    for (int c = 0; c < 2; c++) {
+        const int64_t m = (hi[c] - lo[c]) / 2 + 2131ll * g.brows + 461ll * 32 * (wcols + 1);
+        words = std::max(words, (m / 461 + 2144) / 32 + 2);
+        g.hash_n0[c] = (uint32_t)lo[c];
+    }
+    // The shared form where it hashes less: its sets hold every n between the first
+    // and the last, 4.5 M more with each frame, used or not.  16384^2 (67 M blocks a
+    // frame) takes 1.6 us a frame and 21 direct, 8192^2 with twelve materials (17 M) 4
+    // and 13; at 4096^2 (4.2 M) the direct form hashes less.
+    const int64_t shared = 2 * words * 464, direct = (int64_t)nf * wcols * g.brows;
+    g.hash_shared = shared < direct && words * 464 < (1ll << 26) ? 1 : 0;
+    g.hash_pitch = g.hash_shared ? 464 : g.brows;
+    g.hash_words = (int)(g.hash_shared ? words * 464 : (int64_t)wcols * g.brows);
+    // The step kernel loads up to four frames past the last one and a word past a
+    // row's last: 4 * 4541161 / 2 / 461 bits further on, or four more frames.
+    const size_t sets = g.hash_shared ? 2 : nf;
+    const size_t past = g.hash_shared ? (size_t)(4 * 4541161 / 2 / 461 / 32 + 70) * 464
+                                      : 4 * (size_t)g.hash_words + g.brows;
+    return (sets * g.hash_words + past) * classes * sizeof(uint32_t);
 }
 
 // Packing, hashing and unpacking cost three launches more than the LDS kernels
-// have, and from the largest worlds a pass over the grid: the LDS kernels stay for
-// short runs (measured per call, LDS against sliced: 256^2 8 steps 23 and 20 us, 12
-// steps 37 and 24; 4096^2 8 steps 46 and 56, 12 steps 82 and 67; 16384^2 16 steps
-// 836 and 921, 24 steps 1208 and 1146).
+// have, and from the largest worlds a pass over the grid.  The LDS kernels' default
+// tile advances 8 steps in one launch and stays for those; the generated chain,
+// where no table fits, does a step in the time of ten (measured per call, LDS
+// against sliced, us: four materials 256^2 8 steps 22 and 19, 12 steps 37 and 20;
+// 4096^2 46 and 55, 83 and 64; 16384^2 427 and 567, 831 and 607; twelve at 8192^2
+// 226 and 223, 368 and 261; feature rules 4096^2 2 steps 52 and 53, 4 steps 88 and 66).
 bool se_rt::sliced_pays(const se_world* w, uint32_t n) {
-    return w->mod->sliced.ok && n >= ((size_t)w->W * w->H > (64u << 20) ? 24u : 12u);
+    return w->mod->sliced.ok && n >= (w->mod->table_form == 0 ? 4u : 9u);
 }
 
 int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
@@ -105,12 +140,18 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     SlicedGrid g;
     sliced_geometry(shape, w->W, w->H, g);
     g.pitch = (int)w->pitch;
-    const size_t packed = sliced_packed_bytes(g, K.planes), frame = sliced_frame_bytes(g, K.classes);
+    const size_t packed = sliced_packed_bytes(g, K.planes);
     const uint32_t per_launch = std::min(shape.max_sub, n);
-    // frames hashed at a time: whole launches within the budget
-    uint32_t ahead = (uint32_t)std::min<size_t>(n, std::max<size_t>(1, kHashBudget / frame));
-    if (shape.halo) ahead = std::min(n, std::max(ahead / per_launch, 1u) * per_launch);
-    const size_t bytes = 2 * packed + ahead * frame;
+    // frames hashed at a time: as many whole launches as the budget holds
+    uint32_t ahead = n;
+    size_t hash = sliced_hash_layout(g, w->frame + 1, ahead, K.classes);
+    while (hash > kHashBudget && ahead > (shape.halo ? per_launch : 1u)) {
+        ahead = ahead / 2;
+        if (shape.halo) ahead = std::max(ahead / per_launch, 1u) * per_launch;
+        hash = sliced_hash_layout(g, w->frame + 1, ahead, K.classes);
+    }
+    // later chunks start at another phase of the cycle: a word or two more
+    const size_t bytes = 2 * packed + hash + (size_t)64 * 464 * K.classes;
 
     // The scratch belongs to the context: its worlds share one stream, and the
     // launches of one call are enqueued together under the lock.
@@ -139,11 +180,17 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     int from = 0;
     for (uint32_t at = 0; at < n && !rc;) {
         const uint32_t nf = std::min(ahead, n - at);
-        g.hash_frame0 = w->frame + 1 + (int)at;
-        rc = launch2(K.hash, (unsigned)(g.brows + 255) / 256, std::min(nf * (uint32_t)g.wcols, 65535u), 256, w->stream,
-                     g, (int)nf);
+        const size_t need = sliced_hash_layout(g, w->frame + 1 + (int)at, nf, K.classes);
+        if (2 * packed + need > ctx->sliced_bytes) return fail(SE_ERR_STATE, "internal: hash planes exceed their scratch");
+        rc = launch2(K.hash, (unsigned)(g.hash_words + 255) / 256, g.hash_shared ? 2u : nf, 256, w->stream, g);
         for (uint32_t d = 0; d < nf && !rc;) {
-            const uint32_t m = std::min(shape.max_sub, nf - d);
+            // a launch after the first starts at the head of a cycle where that costs
+            // no further launch
+            const uint32_t lead = (uint32_t)(g.hash_frame0 + (int)d + (int)shape.max_sub) & 3u;
+            uint32_t m = std::min(shape.max_sub, nf - d);
+            if (m < nf - d && lead < m && (nf - d - (m - lead) + shape.max_sub - 1) / shape.max_sub ==
+                                              (nf - d - m + shape.max_sub - 1) / shape.max_sub)
+                m -= lead;
             rc = launch2(K.step[shape.kernel], (unsigned)(shape.tiles_x * shape.tiles_y), 1, 64, w->stream, g, from,
                          shape.tiles_x, g.hash_frame0 + (int)d, (int)m, shape.halo);
             from ^= 1;

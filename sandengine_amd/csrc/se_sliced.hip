@@ -13,9 +13,19 @@
 // row m of it are the world's x = c - xpad and y = m - ypad; everything around
 // the world is WALL.
 //
-// Hash planes: u32 [frame][plane][word column][block row]; bit i of word w is the
-// block whose columns at an even x offset are 64w + 2i and 64w + 2i + 1.  At an
-// odd offset bit i is the block one column to the left, and at an odd y offset
+// Hash planes: bits of blocks, 32 blocks of a block row to a word.  The hash input of
+// the block with origin (x, y) in frame f depends on n = 461 x + 2131 y + 2131^2 f
+// alone.  The planes come in one of two forms:
+//   direct: a set of planes per frame, u32 [b / 32][a][plane], bit b % 32, with a the
+//     block row and b the block column.
+//   shared: two sets, one per parity of n.  Within a set the n used are n0 + 2 m, and
+//     m = 2131 a + 461 b with 0 <= a < 461 names each n once; the same layout with
+//     these a and b.  A block row is a run along b, the row below it is a + 1 at the
+//     same b (from a = 461 on: a - 461, b + 2131), and another frame is another
+//     start: four frames on, a + 113 and b + 9 * 2131.  Blocks of different rows and
+//     frames with the same n, most of them in a large world, are hashed once.
+// At an even x offset the block at bit i of word w is that of columns 64w + 2i and
+// 64w + 2i + 1, at an odd offset the block one column to the left; at an odd y offset
 // block row j is one row further down (rows 2j + 1 and 2j + 2).
 // ---------------------------------------------------------------------------
 typedef unsigned short u16;
@@ -28,11 +38,11 @@ struct se_slgrid {  // == SlicedGrid (se_sliced.hpp)
     u32* hash;      // hash planes of frames hash_frame0 ...
     int W, H, pitch;
     int xpad, ypad, hcols, rows;  // packed geometry: columns of 32 cells, rows (a multiple of 64)
-    int wcols, brows;             // hash planes: word columns, block rows (even)
-    int hash_frame0;
+    int brows;                    // block rows (even)
+    int hash_frame0, hash_shared;
+    int hash_pitch, hash_words;   // values of a, words of a plane
+    u32 hash_n0[2];               // shared: n0 of the sets of even and of odd n
 };
-
-__device__ __forceinline__ u32 se_sl_alignbit(u32 hi, u32 lo, int n) { return __builtin_amdgcn_alignbit(hi, lo, n); }
 
 // Codes of four ids < SE_NMAT packed in bytes, and ids of four codes.
 __device__ __forceinline__ u32 se_sl_map(u32 q, u32 t0, u32 t1, u32 t2, u32 t3) {
@@ -251,44 +261,58 @@ extern "C" __global__ __launch_bounds__(256) void se_sl_unpack(se_slgrid g, int 
 }
 
 // ---------------------------------------------------------------------------
-// Hash planes of `nf` frames from hash_frame0 on.  A thread makes the words of one
-// (frame, word column, block row): lanes are consecutive block rows, so the
-// stores are contiguous, and a thread steps its hash inputs along x by a constant.
-// Bound by VALU issue: per block and hash lane two 32-bit multiplies and three
-// shifted exclusive ors, and two instructions per plane (compare, shift it in).
+// Hash planes.  A thread makes one word of every plane: lanes are consecutive block
+// rows (values of a), so the stores are contiguous, and a thread steps its hash
+// inputs along the block row by a constant.  Bound by VALU issue: per block and hash
+// lane two 32-bit multiplies, three shifted exclusive ors and the step, and two
+// instructions per plane (compare, shift the bit in).  16384^2 and one plane: 1.6 us a
+// frame in the shared form, 21 in the direct one; 4096^2 1.0 us (direct).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void se_sl_hash_word(const se_slgrid& g, int fi, int wc, int j) {
-    const u32 f = (u32)(g.hash_frame0 + fi);
-    int ox, oy;
-    se_offset(f, ox, oy);
-    const int y = 2 * j + oy - g.ypad, x = 64 * wc + 62 - ox - g.xpad;  // block of bit 31
+#define SE_SL_B0 2144  // keeps b >= 0; a multiple of 32
+__device__ __forceinline__ constexpr u32 se_sl_mult(int l) {
+    return l == 0 ? 213u : l == 1 ? 2131u : l == 2 ? 21313u : 213132u;
+}
+
+// acc = acc << 1 | (h <= t): the compare's carry shifted in
+__device__ __forceinline__ void se_sl_push(u32& acc, u32 h, u32 t) {
+    __asm__("v_cmp_ge_u32 vcc, %2, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(acc) : "v"(h), "s"(t) : "vcc");
+}
+
+// grid: x over the words of a plane, y over the sets
+extern "C" __global__ __launch_bounds__(256) void se_sl_hash(se_slgrid g) {
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x, set = (int)blockIdx.y;
+    if (i >= g.hash_words) return;
+    const int u = i / g.hash_pitch, a = i - u * g.hash_pitch;
+    u32 n;  // of the block at bit 31
+    if (g.hash_shared) {
+        n = g.hash_n0[set] + 2u * (2131u * (u32)a + 461u * (u32)(32 * u + 31 - SE_SL_B0));
+    } else {
+        const u32 f = (u32)(g.hash_frame0 + set);
+        int ox, oy;
+        se_offset(f, ox, oy);
+        n = 461u * (u32)(64 * u + 62 - ox - g.xpad) + 2131u * (u32)(2 * a + oy - g.ypad) + 4541161u * f;
+    }
     u32 in[4], acc[SE_SL_P];
 #pragma unroll
-    for (int l = 0; l < 4; l++)
-        in[l] = (u32)x * se_hash_ka(l) + (u32)y * se_hash_kb(l) + f * se_hash_kf(l);
+    for (int l = 0; l < 4; l++) in[l] = n * se_sl_mult(l);
 #pragma unroll
     for (int p = 0; p < SE_SL_P; p++) acc[p] = 0u;
 #pragma unroll 4
-    for (int i = 0; i < 32; i++) {
+    for (int k = 0; k < 32; k++) {
         u32 h[4];
-        bool c[SE_SL_P];
 #pragma unroll
-        for (int l = 0; l < 4; l++) h[l] = se_sliced_lane(l) ? se_lowbias(in[l]) : 0u;
-        se_sliced_classes(h, c);
+        for (int l = 0; l < 4; l++) {
+            h[l] = 0u;
+            if (!se_sliced_lane(l)) continue;
+            h[l] = se_lowbias(in[l]);
+            in[l] -= 922u * se_sl_mult(l);
+        }
 #pragma unroll
-        for (int p = 0; p < SE_SL_P; p++) acc[p] = acc[p] + acc[p] + (c[p] ? 1u : 0u);
-#pragma unroll
-        for (int l = 0; l < 4; l++) in[l] -= 2u * se_hash_ka(l);
+        for (int p = 0; p < SE_SL_P; p++) se_sl_push(acc[p], h[se_sliced_class_lane(p)], se_sliced_class_max(p));
     }
+    u32* out = g.hash + ((size_t)set * g.hash_words + i) * SE_SL_P;
 #pragma unroll
-    for (int p = 0; p < SE_SL_P; p++)
-        g.hash[(((size_t)fi * SE_SL_P + p) * g.wcols + wc) * g.brows + j] = acc[p];
-}
-
-extern "C" __global__ __launch_bounds__(256) void se_sl_hash(se_slgrid g, int nf) {
-    const int j = (int)blockIdx.x * 256 + (int)threadIdx.x;
-    if (j >= g.brows) return;
-    for (int c = (int)blockIdx.y; c < nf * g.wcols; c += (int)gridDim.y) se_sl_hash_word(g, c / g.wcols, c % g.wcols, j);
+    for (int p = 0; p < SE_SL_P; p++) out[p] = acc[p];
 }
 
 // ---------------------------------------------------------------------------
@@ -356,97 +380,212 @@ __device__ __forceinline__ void se_sl_rows_down(se_sltile<NW, R>& t) {
         }
 }
 
+// Where the lane's block rows find their hash words: a and b of the tile's first
+// block, for one phase of the cycle; stepping four frames on stays in the phase.
 template <int NW, int R>
-__device__ __forceinline__ void se_sl_hash_load(const se_slgrid& g, int fi, int wc0, int j0,
-                                                u32 (&h)[NW][R / 2][SE_SL_P]) {
+struct se_slwords {  // raw words: a row's bits start at any bit of the first
+    u32 v[R / 2][NW + 1][SE_SL_P], shift[R / 2];
+};
+
+template <int R>
+struct se_slplace {
+    u32 a[R / 2], b[R / 2];
+    u32 set;  // word offset of the set (direct: of the frame's planes)
+};
+
+template <int R>
+__device__ __forceinline__ se_slplace<R> se_sl_place(const se_slgrid& g, u32 f, int blk0, int j0) {
+    int ox, oy;
+    se_offset(f, ox, oy);
+    const u32 parity = (u32)(ox + oy + (int)f) & 1u;
+    const u32 m = (461u * (u32)(-ox - g.xpad) + 2131u * (u32)(oy - g.ypad) + 4541161u * f - g.hash_n0[parity]) >> 1;
+    const u32 a0 = m % 461u * 204u % 461u;  // 204 * 2131 = 1 mod 461
+    const u32 b0 = (m + 461u * SE_SL_B0 - 2131u * a0) / 461u;
+    const bool sh = g.hash_shared != 0;
+    se_slplace<R> q;
+    q.set = (sh ? parity : f - (u32)g.hash_frame0) * (u32)g.hash_words;
 #pragma unroll
-    for (int p = 0; p < SE_SL_P; p++)
+    for (int i = 0; i < R / 2; i++) {
+        const u32 a = (sh ? a0 : 0u) + (u32)(j0 + i), wrap = sh ? a / 461u : 0u;
+        q.a[i] = a - 461u * wrap;
+        q.b[i] = (sh ? b0 : 0u) + (u32)blk0 + 2131u * wrap;
+    }
+    return q;
+}
+
+// Loads at the place; the words are shifted into line only where they are used
+// (se_sl_hash_of), so nothing waits here.
+template <int NW, int R>
+__device__ __forceinline__ void se_sl_hash_load(const se_slgrid& g, const se_slplace<R>& q, se_slwords<NW, R>& h) {
 #pragma unroll
-        for (int w = 0; w < NW; w++) {
-            const u32* s = g.hash + (((size_t)fi * SE_SL_P + p) * g.wcols + wc0 + w) * g.brows + j0;
+    for (int i = 0; i < R / 2; i++) {
+        const u32 at = (q.set + (q.b[i] >> 5) * (u32)g.hash_pitch + q.a[i]) * (u32)SE_SL_P;
+        h.shift[i] = q.b[i];  // alignbit takes it modulo 32
 #pragma unroll
-            for (int b = 0; b < R / 2; b++) h[w][b][p] = s[b];
+        for (int w = 0; w <= NW; w++) {
+            const u32* s = g.hash + (size_t)w * (size_t)(g.hash_pitch * SE_SL_P);
+#pragma unroll
+            for (int p = 0; p < SE_SL_P; p++) h.v[i][w][p] = s[at + (u32)p];
         }
+    }
+}
+
+template <int R>
+__device__ __forceinline__ void se_sl_next_cycle(const se_slgrid& g, se_slplace<R>& q) {
+    const u32 da = g.hash_shared ? 113u : 0u, db = g.hash_shared ? 9u * 2131u : 0u;
+    const u32 mod = g.hash_shared ? 461u : 0x7fffffffu;
+    q.set += g.hash_shared ? 0u : 4u * (u32)g.hash_words;
+#pragma unroll
+    for (int i = 0; i < R / 2; i++) {
+        const u32 a = q.a[i] + da;
+        const bool c = a >= mod;
+        q.a[i] = c ? a - mod : a;
+        q.b[i] += c ? db + 2131u : db;
+    }
 }
 
 template <int NW, int R>
-__device__ __forceinline__ void se_sl_advance(se_sltile<NW, R>& t, const se_slgrid& g, int wc0, int row0, int lane,
-                                              int frame0, int nsub) {
-    const int j0 = row0 / 2 + (R / 2) * lane;
-    int ysh = 0;
-    u32 h[NW][R / 2][SE_SL_P];
-    se_sl_hash_load<NW, R>(g, frame0 - g.hash_frame0, wc0, j0, h);
-#if !SE_SL_KEEP
-    const bool edge = 64 * wc0 < g.xpad || 64 * (wc0 + NW) > g.xpad + g.W || row0 < g.ypad ||
-                      row0 + 64 * R > g.ypad + g.H;
-#endif
-    for (int s = 0; s < nsub; s++) {
-        int ox, oy;
-        se_offset((u32)(frame0 + s), ox, oy);
-        u32 hn[NW][R / 2][SE_SL_P];  // the next sub-step's hash planes are in flight during this one
-        se_sl_hash_load<NW, R>(g, frame0 - g.hash_frame0 + min(s + 1, nsub - 1), wc0, j0, hn);
-        if (oy != ysh) {
-            if (oy) se_sl_rows_up(t);
-            else se_sl_rows_down(t);
-            ysh = oy;
-        }
-        if (ox) {
+__device__ __forceinline__ void se_sl_hash_of(const se_slwords<NW, R>& r, u32 (&h)[R / 2][NW][SE_SL_P]) {
 #pragma unroll
-            for (int r = 0; r < R; r++)
-#pragma unroll
-                for (int k = 0; k < SE_SL_K; k++)
-#pragma unroll
-                    for (int w = NW - 1; w >= 0; w--)
-                        t.o[r][w][k] = se_sl_alignbit(t.o[r][w][k], w ? t.o[r][w - 1][k] : se_sl_wall(k), 31);
-#pragma unroll
-            for (int w = 0; w < NW; w++)
-#pragma unroll
-                for (int b = 0; b < R / 2; b++)
-                    se_sliced_block(t.o[2 * b][w], t.e[2 * b][w], t.o[2 * b + 1][w], t.e[2 * b + 1][w], h[w][b]);
-#pragma unroll
-            for (int r = 0; r < R; r++)
-#pragma unroll
-                for (int k = 0; k < SE_SL_K; k++)
-#pragma unroll
-                    for (int w = 0; w < NW; w++)
-                        t.o[r][w][k] = se_sl_alignbit(w + 1 < NW ? t.o[r][w + 1][k] : se_sl_wall(k), t.o[r][w][k], 1);
-        } else {
-#pragma unroll
-            for (int w = 0; w < NW; w++)
-#pragma unroll
-                for (int b = 0; b < R / 2; b++)
-                    se_sliced_block(t.e[2 * b][w], t.o[2 * b][w], t.e[2 * b + 1][w], t.o[2 * b + 1][w], h[w][b]);
-        }
-#if !SE_SL_KEEP
-        if (edge) {  // rules may change the WALL outside the world: it is put back
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int y = row0 + R * lane + r + ysh - g.ypad;
-                const u32 rm = y >= 0 && y < g.H ? 0xffffffffu : 0u;
-#pragma unroll
-                for (int w = 0; w < NW; w++) {
-                    const int x0 = 64 * (wc0 + w) - g.xpad;  // column of bit 0 of E
-                    const int lo = x0 < 0 ? (-x0 + 1) / 2 : 0, lo1 = x0 < 0 ? -x0 / 2 : 0;
-                    const int hi = min(32, max(0, (g.W - x0 + 1) / 2)), hi1 = min(32, max(0, (g.W - x0) / 2));
-                    const u32 me = (u32)((1ull << hi) - 1ull) & ~(u32)((1ull << min(lo, 32)) - 1ull) & rm;
-                    const u32 mo = (u32)((1ull << hi1) - 1ull) & ~(u32)((1ull << min(lo1, 32)) - 1ull) & rm;
-#pragma unroll
-                    for (int k = 0; k < SE_SL_K; k++) {
-                        t.e[r][w][k] = (t.e[r][w][k] & me) | (se_sl_wall(k) & ~me);
-                        t.o[r][w][k] = (t.o[r][w][k] & mo) | (se_sl_wall(k) & ~mo);
-                    }
-                }
-            }
-        }
-#endif
+    for (int i = 0; i < R / 2; i++)
 #pragma unroll
         for (int w = 0; w < NW; w++)
 #pragma unroll
-            for (int b = 0; b < R / 2; b++)
+            for (int p = 0; p < SE_SL_P; p++)
+                h[i][w][p] = __builtin_amdgcn_alignbit(r.v[i][w + 1][p], r.v[i][w][p], r.shift[i]);
+}
+
+#if !SE_SL_KEEP
+// Puts back the WALL outside the world (rules may change it); ysh: rows moved up.
+template <int NW, int R>
+__device__ __forceinline__ void se_sl_keep_wall(se_sltile<NW, R>& t, const se_slgrid& g, int wc0, int y0) {
 #pragma unroll
-                for (int p = 0; p < SE_SL_P; p++) h[w][b][p] = hn[w][b][p];
+    for (int r = 0; r < R; r++) {
+        const u32 rm = y0 + r >= 0 && y0 + r < g.H ? 0xffffffffu : 0u;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const int x0 = 64 * (wc0 + w) - g.xpad;  // column of bit 0 of E
+            const int lo = x0 < 0 ? (-x0 + 1) / 2 : 0, lo1 = x0 < 0 ? -x0 / 2 : 0;
+            const int hi = min(32, max(0, (g.W - x0 + 1) / 2)), hi1 = min(32, max(0, (g.W - x0) / 2));
+            const u32 me = (u32)((1ull << hi) - 1ull) & ~(u32)((1ull << min(lo, 32)) - 1ull) & rm;
+            const u32 mo = (u32)((1ull << hi1) - 1ull) & ~(u32)((1ull << min(lo1, 32)) - 1ull) & rm;
+#pragma unroll
+            for (int k = 0; k < SE_SL_K; k++) {
+                t.e[r][w][k] = (t.e[r][w][k] & me) | (se_sl_wall(k) & ~me);
+                t.o[r][w][k] = (t.o[r][w][k] & mo) | (se_sl_wall(k) & ~mo);
+            }
+        }
     }
-    if (ysh) se_sl_rows_down(t);
+}
+#endif
+
+// One sub-step at x offset OX with the rows already paired (y offset applied).
+template <int NW, int R, bool OX>
+__device__ __forceinline__ void se_sl_substep(se_sltile<NW, R>& t, const se_slwords<NW, R>& raw) {
+    u32 h[R / 2][NW][SE_SL_P];
+    se_sl_hash_of<NW, R>(raw, h);
+    if (OX) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int k = 0; k < SE_SL_K; k++)
+#pragma unroll
+                for (int w = NW - 1; w >= 0; w--)
+                    t.o[r][w][k] = __builtin_amdgcn_alignbit(t.o[r][w][k], w ? t.o[r][w - 1][k] : se_sl_wall(k), 31);
+    }
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+        for (int b = 0; b < R / 2; b++) {
+            if (OX) se_sliced_block(t.o[2 * b][w], t.e[2 * b][w], t.o[2 * b + 1][w], t.e[2 * b + 1][w], h[b][w]);
+            else se_sliced_block(t.e[2 * b][w], t.o[2 * b][w], t.e[2 * b + 1][w], t.o[2 * b + 1][w], h[b][w]);
+        }
+    if (OX) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int k = 0; k < SE_SL_K; k++)
+#pragma unroll
+                for (int w = 0; w < NW; w++)
+                    t.o[r][w][k] = __builtin_amdgcn_alignbit(w + 1 < NW ? t.o[r][w + 1][k] : se_sl_wall(k),
+                                                             t.o[r][w][k], 1);
+    }
+}
+
+// Whole cycles of four frames run in a loop of their own: every offset is a
+// constant there, the rows move up once and down once and the moves are register
+// names.  Up to three frames before and after them take the general step.  The
+// hash words are loaded AHEAD frames before their use: a 2x2 tile's sub-step takes
+// 0.3 us, and the words come from beyond the L2.
+template <int NW, int R, int AHEAD>
+__device__ __forceinline__ void se_sl_advance(se_sltile<NW, R>& t, const se_slgrid& g, int blk0, int row0, int lane,
+                                              int frame0, int nsub) {
+    static_assert(AHEAD == 2 || AHEAD == 4, "sets of words by phase");
+    const int j0 = row0 / 2 + (R / 2) * lane;
+    u32 f = (u32)frame0;
+    const u32 end = f + (u32)nsub, first = (f + 3u) & ~3u;
+#if !SE_SL_KEEP
+    const int wc0 = blk0 / 32;
+    const bool edge = 64 * wc0 < g.xpad || 64 * (wc0 + NW) > g.xpad + g.W || row0 < g.ypad ||
+                      row0 + 64 * R > g.ypad + g.H;
+    const int y0 = row0 + R * lane - g.ypad;
+#define SE_SL_FIX(up) if (edge) se_sl_keep_wall<NW, R>(t, g, wc0, y0 + (up))
+#else
+#define SE_SL_FIX(up)
+#endif
+    auto general = [&](u32 fr, const se_slwords<NW, R>& h) {
+        int ox, oy;
+        se_offset(fr, ox, oy);
+        if (oy) se_sl_rows_up(t);
+        if (ox) se_sl_substep<NW, R, true>(t, h);
+        else se_sl_substep<NW, R, false>(t, h);
+        SE_SL_FIX(oy);
+        if (oy) se_sl_rows_down(t);
+    };
+    for (; f < end && f < first; f++) {
+        se_slwords<NW, R> h;
+        se_sl_hash_load<NW, R>(g, se_sl_place<R>(g, f, blk0, j0), h);
+        general(f, h);
+    }
+    if (f + 4u <= end) {
+        se_slplace<R> q[4];
+        se_slwords<NW, R> h[AHEAD];
+#pragma unroll
+        for (u32 p = 0; p < 4; p++) q[p] = se_sl_place<R>(g, f + p, blk0, j0);
+#pragma unroll
+        for (int p = 0; p < AHEAD; p++) se_sl_hash_load<NW, R>(g, q[p], h[p]);
+#pragma unroll
+        for (int p = 0; p < AHEAD; p++) se_sl_next_cycle<R>(g, q[p]);
+        // (the last cycle's loads run on into the frames after the last: the planes
+        // have room for them)
+        do {
+            se_sl_substep<NW, R, false>(t, h[0]);          // offsets (0, 0)
+            SE_SL_FIX(0);
+            se_sl_hash_load<NW, R>(g, q[AHEAD & 3], h[0]);
+            se_sl_next_cycle<R>(g, q[AHEAD & 3]);
+            se_sl_rows_up(t);
+            se_sl_substep<NW, R, true>(t, h[1]);           // (1, 1)
+            SE_SL_FIX(1);
+            se_sl_hash_load<NW, R>(g, q[(AHEAD + 1) & 3], h[1]);
+            se_sl_next_cycle<R>(g, q[(AHEAD + 1) & 3]);
+            se_sl_substep<NW, R, false>(t, h[2 % AHEAD]);  // (0, 1)
+            SE_SL_FIX(1);
+            se_sl_hash_load<NW, R>(g, q[(AHEAD + 2) & 3], h[2 % AHEAD]);
+            se_sl_next_cycle<R>(g, q[(AHEAD + 2) & 3]);
+            se_sl_rows_down(t);
+            se_sl_substep<NW, R, true>(t, h[3 % AHEAD]);   // (1, 0)
+            SE_SL_FIX(0);
+            se_sl_hash_load<NW, R>(g, q[(AHEAD + 3) & 3], h[3 % AHEAD]);
+            se_sl_next_cycle<R>(g, q[(AHEAD + 3) & 3]);
+            f += 4u;
+        } while (f + 4u <= end);
+    }
+    for (; f < end; f++) {
+        se_slwords<NW, R> h;
+        se_sl_hash_load<NW, R>(g, se_sl_place<R>(g, f, blk0, j0), h);
+        general(f, h);
+    }
+#undef SE_SL_FIX
 }
 
 // Rows of two neighbouring half columns <-> words (R rows x 2K planes each).
@@ -502,7 +641,7 @@ __device__ __forceinline__ void se_sl_store(const se_sltile<NW, R>& t, u16* pk, 
 
 // `from`: the packed grid read, the other is written.  halo 0: the world fits the
 // one tile, all of which is stored.
-template <int NW, int R>
+template <int NW, int R, int AHEAD>
 __device__ __forceinline__ void se_sl_tile(const se_slgrid& g, int from, int tx, int ty, int frame0, int nsub,
                                            int halo) {
     const int lane = (int)(threadIdx.x & 63);
@@ -510,18 +649,17 @@ __device__ __forceinline__ void se_sl_tile(const se_slgrid& g, int from, int tx,
     const int row = row0 + R * lane;
     se_sltile<NW, R> t;
     se_sl_load<NW, R>(t, g.pk[from], g, hc0, row);
-    se_sl_advance<NW, R>(t, g, hc0 / 2, row0, lane, frame0, nsub);
+    se_sl_advance<NW, R, AHEAD>(t, g, 16 * hc0, row0, lane, frame0, nsub);
     if (R * lane < halo || R * lane >= 64 * R - halo) return;
     if (halo == 0) se_sl_store<NW, R>(t, g.pk[from ^ 1], g, hc0, row, 0, 2 * NW - 1);
     else se_sl_store<NW, R>(t, g.pk[from ^ 1], g, hc0, row, 1, 2 * NW - 2);
 }
 
-#define SE_SL_STEP(NW, R)                                                                                     \
+#define SE_SL_STEP(NW, R, AHEAD)                                                                                     \
     extern "C" __global__ __launch_bounds__(64) void se_sl_step_##NW##x##R(se_slgrid g, int from, int tiles_x, \
                                                                            int frame0, int nsub, int halo) {   \
         const int tile = se_xcd_tile((int)blockIdx.x, (int)gridDim.x);                                         \
-        se_sl_tile<NW, R>(g, from, tile % tiles_x, tile / tiles_x, frame0, nsub, halo);                        \
+        se_sl_tile<NW, R, AHEAD>(g, from, tile % tiles_x, tile / tiles_x, frame0, nsub, halo);                        \
     }
-SE_SL_STEP(2, 2)
-SE_SL_STEP(4, 2)
-SE_SL_STEP(4, 4)
+SE_SL_STEP(2, 2, 4)
+SE_SL_STEP(4, 2, 2)

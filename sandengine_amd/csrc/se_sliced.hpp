@@ -15,10 +15,12 @@ struct SlicedGrid {
     uint32_t* hash = nullptr;
     int W = 0, H = 0, pitch = 0;
     int xpad = 0, ypad = 0, hcols = 0, rows = 0;
-    int wcols = 0, brows = 0;
-    int hash_frame0 = 0;
+    int brows = 0;
+    int hash_frame0 = 0, hash_shared = 0;
+    int hash_pitch = 0, hash_words = 0;
+    uint32_t hash_n0[2] = {0, 0};
 };
-static_assert(sizeof(SlicedGrid) == 80, "se_slgrid layout");
+static_assert(sizeof(SlicedGrid) == 96, "se_slgrid layout");
 
 // How a world is cut into tiles of one step kernel.
 struct SlicedShape {
@@ -34,7 +36,10 @@ SlicedShape sliced_shape(uint32_t W, uint32_t H, uint32_t sub);
 // Fills the geometry fields of g for that shape.
 void sliced_geometry(const SlicedShape& s, uint32_t W, uint32_t H, SlicedGrid& g);
 size_t sliced_packed_bytes(const SlicedGrid& g, int planes);  // of one packed grid
-size_t sliced_frame_bytes(const SlicedGrid& g, int classes);  // hash planes of one frame
+// Sets up the hash planes of frames [frame0, frame0 + nf) in g (all but the pointer):
+// the form and its sizes; returns their bytes, with room for the words that the step
+// kernel loads ahead.
+size_t sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int classes);
 
 // Is the sliced path taken for n steps of a world whose caller chose no variant?
 bool sliced_pays(const se_world* w, uint32_t n);

@@ -63,6 +63,26 @@ def test_sliced_equals_plain(name, size):
     b.close()
 
 
+@pytest.mark.parametrize("name", ["four_materials", "twelve_materials"])
+@pytest.mark.parametrize("size,first,steps", [((5003, 4999), 3, 45), ((9001, 2801), 2147483000, 38)],
+                         ids=["5003x4999", "9001x2801_late"])
+def test_sliced_shared_hash_planes(name, size, first, steps):
+    """Worlds large enough to share hash planes between block rows and frames (rows
+    past 461 wrap); a start near the last frame, where the hash inputs wrap."""
+    print(f"\n[gpu] sliced {name} {size} from frame {first}", flush=True)
+    r, (W, H) = rs(name), size
+    a, b = S.World(_ctx, r, W, H), S.World(_ctx, r, W, H)
+    for w in (a, b):
+        w.fill_seeded(3, *FILL[name])
+        w.frame = first
+    a.step(steps)
+    b.step_blocked(steps)
+    assert a.frame == b.frame == first + steps
+    np.testing.assert_array_equal(a.download(), b.download())
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("name", list(FILL))
 def test_sliced_equals_oracle(name):
     print(f"\n[gpu] sliced {name} against the oracle", flush=True)

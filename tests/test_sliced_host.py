@@ -37,11 +37,9 @@ int main(int argc, char** argv) {
                 for (int k = 0; k < SE_SL_K; k++)
                     c[j][k] = ((cw[id[j] / 4] >> (8 * (id[j] & 3)) >> k) & 1) ? ~0u : 0u;
             for (int p = 0; p < SE_SL_P; p++) h[p] = 0;
-            for (size_t k = k0; k < nh && k < k0 + 32; k++) {
-                bool b[SE_SL_P];
-                se_sliced_classes(hs + 4 * k, b);
-                for (int p = 0; p < SE_SL_P; p++) h[p] |= (unsigned)b[p] << (k - k0);
-            }
+            for (size_t k = k0; k < nh && k < k0 + 32; k++)
+                for (int p = 0; p < SE_SL_P; p++)
+                    h[p] |= (unsigned)(hs[4 * k + se_sliced_class_lane(p)] <= se_sliced_class_max(p)) << (k - k0);
             se_sliced_block(c[0], c[1], c[2], c[3], h);
             for (size_t k = k0; k < nh && k < k0 + 32; k++)
                 for (int j = 0; j < 4; j++) {
