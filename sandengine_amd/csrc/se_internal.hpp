@@ -55,6 +55,12 @@ struct DeviceGuard {
     }
 };
 
+struct FillSpec {  // == se_fillspec in se_kernels.hip
+    int n, stone_rows;
+    uint32_t stone_id, pad;
+    uint32_t ids[16], thr[16];
+};
+
 // The sliced kernels of a module (se_sliced.hip); ok false where the rule set has
 // no sliced form.
 struct SlicedKernels {

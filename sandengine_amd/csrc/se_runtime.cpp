@@ -1180,17 +1180,29 @@ int se_world_fill_seeded(se_world* w, uint64_t seed, const uint32_t* ids, const 
     if (!w || !ids || !thresholds || n < 1 || n > 64) return fail(SE_ERR_ARG, "bad fill arguments");
     DeviceGuard dg(w->ctx->device);
     se_rt::sleep_reset(w);
-    // ids and thresholds are staged in the world's modification buffer (8 KiB)
-    void* d = w->d_mods;
-    uint32_t host[128] = {0};
-    std::memcpy(host, ids, n * 4);
-    std::memcpy(host + 64, thresholds, n * 4);
-    HIPCHECK(hipMemcpyAsync(d, host, sizeof host, hipMemcpyHostToDevice, w->stream));
     size_t cells = (size_t)w->W * w->H;
     unsigned blocks = (unsigned)std::min<size_t>((cells + 255) / 256, 1u << 16);
-    int rc = launch(w->mod->fill_seeded, blocks, w->stream, w->buf[w->cur], (int)w->W, (int)w->H, (int)w->pitch,
+    int rc;
+    if (n <= 16) {
+        se_rt::FillSpec fs{};
+        fs.n = n;
+        fs.stone_rows = (int)stone_rows;
+        fs.stone_id = stone_id;
+        std::memcpy(fs.ids, ids, n * 4);
+        std::memcpy(fs.thr, thresholds, n * 4);
+        rc = launch(w->mod->fill_spec, blocks, w->stream, w->buf[w->cur], (int)w->W, (int)w->H, (int)w->pitch,
+                    (unsigned long long)seed, fs);
+    } else {
+        // ids and thresholds are staged in the world's modification buffer (8 KiB)
+        void* d = w->d_mods;
+        uint32_t host[128] = {0};
+        std::memcpy(host, ids, n * 4);
+        std::memcpy(host + 64, thresholds, n * 4);
+        HIPCHECK(hipMemcpyAsync(d, host, sizeof host, hipMemcpyHostToDevice, w->stream));
+        rc = launch(w->mod->fill_seeded, blocks, w->stream, w->buf[w->cur], (int)w->W, (int)w->H, (int)w->pitch,
                     (unsigned long long)seed, (const uint32_t*)d, (const uint32_t*)d + 64, n, (int)stone_rows,
                     stone_id);
+    }
     hipError_t e2 = hipStreamSynchronize(w->stream);
     if (rc) return rc;
     if (e2 != hipSuccess) return fail(SE_ERR_HIP, std::string("fill sync: ") + hipGetErrorString(e2));

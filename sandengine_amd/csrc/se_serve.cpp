@@ -97,12 +97,6 @@ struct Arena {
     }
 };
 
-struct FillSpec {  // == se_fillspec in se_kernels.hip
-    int n, stone_rows;
-    uint32_t stone_id, pad;
-    uint32_t ids[16], thr[16];
-};
-
 struct BWorld {  // == se_bworld in se_kernels.hip
     uint32_t* buf[2];
     int W, H, pitch, tiles_x, ntiles;
@@ -322,7 +316,7 @@ uint64_t fnv64(const uint32_t* p, size_t n) {
 struct se_serve {
     se_ctx* ctx = nullptr;
     std::vector<const se_ruleset*> rs;
-    std::vector<FillSpec> fills;
+    std::vector<se_rt::FillSpec> fills;
     se_serve_config cfg{};
     std::vector<Request> reqs;
     bool ran = false;
@@ -399,7 +393,7 @@ int admit(se_serve* S, Request& r, Arena& A) {
     r.off = off;
     r.bytes = need;
     r.state = 1;
-    const FillSpec& fs = S->fills[r.rs];
+    const se_rt::FillSpec& fs = S->fills[r.rs];
     size_t cells = (size_t)r.side * r.side;
     unsigned blocks = (unsigned)std::min<size_t>((cells + 255) / 256, 1u << 16);
     return launch(w->mod->fill_spec, blocks, w->stream, w->buf[0], (int)r.side, (int)r.side, (int)pitch,
@@ -666,7 +660,7 @@ int se_serve_create(se_ctx* ctx, const se_ruleset* const* rulesets, int n_rulese
             return fail(SE_ERR_ARG, "rule set missing or from another context");
         }
         S->rs.push_back(rulesets[i]);
-        FillSpec f{};
+        se_rt::FillSpec f{};
         f.n = 1;
         f.ids[0] = 0;
         S->fills.push_back(f);
@@ -685,7 +679,7 @@ void se_serve_destroy(se_serve* S) {
 int se_serve_set_fill(se_serve* S, int rs, const uint32_t* ids, const uint32_t* thresholds, int n) {
     if (!S || rs < 0 || rs >= (int)S->rs.size() || !ids || !thresholds || n < 1 || n > 16)
         return fail(SE_ERR_ARG, "bad fill");
-    FillSpec f{};
+    se_rt::FillSpec f{};
     f.n = n;
     for (int i = 0; i < n; i++) {
         f.ids[i] = ids[i];
