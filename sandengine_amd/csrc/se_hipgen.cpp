@@ -932,7 +932,9 @@ struct NotSliced {};  // the rule set reads something that has no word form
 
 class Slicer {
 public:
-    Slicer(const Ctx& ctx, int planes, const std::vector<int>& code) : ctx_(ctx), K_(planes), code_(code) {
+    // code: of a material; order: ascending with the density where rules compare it
+    Slicer(const Ctx& ctx, int planes, const std::vector<int>& code, const std::vector<int>& order)
+        : ctx_(ctx), K_(planes), code_(code), order_(order) {
         for (int c = 0; c < 4; c++)
             for (int k = 0; k < K_; k++) cell_[c].push_back(net.input());
     }
@@ -1006,7 +1008,7 @@ private:
     };
     const Ctx& ctx_;
     int K_;
-    std::vector<int> code_;
+    std::vector<int> code_, order_;
     Cell cell_[4];
     std::vector<bool> fixed_of_;
 
@@ -1019,15 +1021,14 @@ private:
     Net::Lit holds(const Cell& c, const std::vector<bool>& set) {
         return table(c, [&](int m) { return set[m] ? 1 : 0; });
     }
-    // a cell's code with equal densities sharing the lowest of their codes (codes
-    // ascend with the density wherever ranks are compared)
+    // a cell's order with equal densities sharing the lowest of theirs
     Cell rank(const Cell& c) {
         Cell r;
         for (int k = 0; k < K_; k++)
             r.push_back(table(c, [&](int m) {
-                int low = code_[m];
+                int low = order_[m];
                 for (int o = 0; o < ctx_.nmat; o++)
-                    if (ctx_.dens[o] == ctx_.dens[m]) low = std::min(low, code_[o]);
+                    if (ctx_.dens[o] == ctx_.dens[m]) low = std::min(low, order_[o]);
                 return (low >> k) & 1;
             }));
         return r;
@@ -1183,17 +1184,23 @@ std::string hip_sliced_source(const ParsingResult& r, SlicedInfo& out) {
         if (std::isnan(d)) return "";
     int K = 1;
     while ((1 << K) < n) K++;
-    // codes ascend with the density (ties by id), so that comparing densities
-    // compares codes; id order where no rule compares them (no remapping then)
+    // Codes ascend with the density (ties by id) where rules compare it, so that
+    // comparing densities compares codes, up to an exclusive or that makes WALL 0:
+    // the planes that come in from outside a tile are then 0, which the wave shifts
+    // give for nothing.
     Emitter em(ctx);
     for (auto& rl : r.rules)
         if (rl.used) emit_rule(rl, ctx, em);
-    std::vector<int> by(n), code(n);
+    std::vector<int> by(n), order(n), code(n), id_of(16, 2);
     for (int i = 0; i < n; i++) by[i] = i;
     if (em.rank_used)
         std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return ctx.dens[a] < ctx.dens[b]; });
-    for (int i = 0; i < n; i++) code[by[i]] = i;
-    Slicer sl(ctx, K, code);
+    for (int i = 0; i < n; i++) order[by[i]] = i;
+    for (int i = 0; i < n; i++) {
+        code[i] = order[i] ^ order[2];
+        id_of[code[i]] = i;
+    }
+    Slicer sl(ctx, K, code, order);
     std::vector<Net::Lit> outs;
     try {
         outs = sl.chain(r);
@@ -1250,14 +1257,11 @@ std::string hip_sliced_source(const ParsingResult& r, SlicedInfo& out) {
     o << "template <int TT>\n__device__ __forceinline__ unsigned int se_lut3(unsigned int a, unsigned int b, unsigned int "
          "c) {\n    return __builtin_amdgcn_bitop3_b32(a, b, c, TT);\n}\n";
     o << "#define SE_SL_K " << K << "\n#define SE_SL_P " << P << "\n#define SE_SL_KEEP " << (kept ? 1 : 0) << "\n";
-    o << "#define SE_SL_REMAP " << (em.rank_used ? 1 : 0) << "\n";
-    o << "#define SE_SL_EMPTY " << code[0] << "u\n#define SE_SL_NULL " << code[1] << "u\n#define SE_SL_WALL " << code[2]
-      << "u\n";
     // code of id i and id of code i as bytes of four words
     for (int dir = 0; dir < 2; dir++) {
         uint32_t w[4] = {0, 0, 0, 0};
         for (int i = 0; i < 16; i++) {
-            const int v = i < n ? (dir == 0 ? code[i] : by[i]) : (dir == 0 ? code[1] : 1);
+            const int v = dir == 0 ? (i < n ? code[i] : code[1]) : id_of[i];
             w[i / 4] |= (uint32_t)v << (8 * (i & 3));
         }
         for (int j = 0; j < 4; j++) o << "#define SE_SL_" << (dir == 0 ? "CODE" : "ID") << j << " " << hex_u32(w[j]) << "\n";

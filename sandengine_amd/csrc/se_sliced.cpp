@@ -49,20 +49,25 @@ se_rt::SlicedShape se_rt::sliced_shape(uint32_t W, uint32_t H, uint32_t sub) {
     // The tile and the depth of a launch, by how many 2x2 tiles (64 useful columns and
     // rows at 32 sub-steps) the world makes.  Up to one a SIMD the launches are a
     // serial chain of sub-steps: the smallest tile and the deepest launch
-    // (1000x700: 133 us for 200 steps, 206 with 4x2, 153 with 16 sub-steps).  Beyond
-    // that the rows given up count, and from 8 a SIMD on the columns too
-    // (4096^2, 200 steps: 512 us with 2x2 and 16, 531 with 4x2, 534 with 32;
-    // 16384^2, 100 steps: 1.65 ms with 4x2 and 16, 2.04 with 2x2, 1.97 with 32).
+    // (1000x700: 132 us for 200 steps, 214 with 4x2, 155 with 16 sub-steps).  Beyond
+    // that the rows and columns given up count (16 columns a side up to 16
+    // sub-steps, 32 beyond), and from 8 a SIMD on the wider tile pays (4096^2, 200
+    // steps: 456 us with 2x2 and 16, 494 with 4x2, 526 with 32; 16384^2, 100 steps:
+    // 1.45 ms with 4x2 and 12, 1.55 with 16, 1.56 with 2x2; twelve materials at
+    // 8192^2, 64 steps: 761, 800 and 770 us).
     const size_t few = (size_t)((W + 63) / 64) * ((H + 63) / 64);
     const int i = few > 8192 ? 1 : 0;
-    const uint32_t deep = few > 1024 ? 16 : 32;
+    const uint32_t deep = few > 8192 ? 12 : few > 1024 ? 16 : 32;
+
     s.kernel = i;
     s.nw = kTiles[i].nw;
     s.r = kTiles[i].r;
     s.max_sub = sub ? std::min(sub, deep) : deep;
     s.halo = (int)(s.max_sub + 3) & ~3;
-    s.tiles_x = (int)(W + 64 * s.nw - 65) / (64 * s.nw - 64);
-    s.tiles_y = (int)(H + 64 * s.r - 2 * s.halo - 1) / (64 * s.r - 2 * s.halo);
+    s.side = s.max_sub > 16 ? 2 : 1;
+    const uint32_t ux = 64u * s.nw - 32u * s.side, uy = 64u * s.r - 2u * s.halo;  // useful columns and rows of a tile
+    s.tiles_x = (int)((W + ux - 1) / ux);
+    s.tiles_y = (int)((H + uy - 1) / uy);
     return s;
 }
 
@@ -73,20 +78,20 @@ void se_rt::sliced_geometry(const SlicedShape& s, uint32_t W, uint32_t H, Sliced
         g.xpad = 4;  // keeps the 16-byte loads of ids aligned
         g.ypad = 2;
     } else {
-        g.xpad = 32;
+        g.xpad = 16 * s.side;
         g.ypad = s.halo;
     }
-    g.hcols = (s.tiles_x - 1) * (2 * s.nw - 2) + 2 * s.nw;
+    g.bcols = (s.tiles_x - 1) * (4 * s.nw - 2 * s.side) + 4 * s.nw;
     g.rows = ((s.tiles_y - 1) * (64 * s.r - 2 * s.halo) + 64 * s.r + 63) & ~63;
     g.brows = g.rows / 2;
 }
 
-size_t se_rt::sliced_packed_bytes(const SlicedGrid& g, int planes) {
-    return ((size_t)g.hcols * g.rows * 2 * planes * sizeof(uint16_t) + 255) & ~(size_t)255;
+size_t se_rt::sliced_packed_bytes(const SlicedGrid& g) {
+    return ((size_t)g.bcols * g.rows * 8 + 255) & ~(size_t)255;
 }
 
 size_t se_rt::sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int classes) {
-    const int wcols = g.hcols / 2;
+    const int wcols = (g.bcols + 3) / 4;
     g.hash_frame0 = frame0;
     // shared form: the range of n of each parity over the frames, and the words of b
     // that cover it (one more than a tile's last word, for the shifted read)
@@ -140,7 +145,7 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     SlicedGrid g;
     sliced_geometry(shape, w->W, w->H, g);
     g.pitch = (int)w->pitch;
-    const size_t packed = sliced_packed_bytes(g, K.planes);
+    const size_t packed = sliced_packed_bytes(g);
     const uint32_t per_launch = std::min(shape.max_sub, n);
     // frames hashed at a time: as many whole launches as the budget holds
     uint32_t ahead = n;
@@ -171,12 +176,14 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     *done = true;
     g.in = w->buf[w->cur];
     g.out = w->buf[w->cur ^ 1];
-    g.pk[0] = (uint16_t*)ctx->sliced_mem;
-    g.pk[1] = (uint16_t*)((char*)ctx->sliced_mem + packed);
+    g.pk[0] = ctx->sliced_mem;
+    g.pk[1] = (char*)ctx->sliced_mem + packed;
     g.hash = (uint32_t*)((char*)ctx->sliced_mem + 2 * packed);
 
-    const int wtiles = g.hcols / 2, ctiles = wtiles * (g.rows / 64);
-    int rc = launch2(K.pack, (unsigned)(ctiles + 3) / 4, 1, 256, w->stream, g, wtiles, ctiles);
+    // 64 columns x 64 rows a wavefront; packing also covers the margins
+    const int pcols = 1 + (g.bcols - g.xpad / 16 + 3) / 4, ptiles = pcols * (g.rows / 64);
+    const int ucols = (int)(w->W + (g.xpad & 15) + 63) / 64, utiles = ucols * (g.rows / 64);
+    int rc = launch2(K.pack, (unsigned)(ptiles + 3) / 4, 1, 256, w->stream, g, pcols, ptiles);
     int from = 0;
     for (uint32_t at = 0; at < n && !rc;) {
         const uint32_t nf = std::min(ahead, n - at);
@@ -192,13 +199,13 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
                                               (nf - d - m + shape.max_sub - 1) / shape.max_sub)
                 m -= lead;
             rc = launch2(K.step[shape.kernel], (unsigned)(shape.tiles_x * shape.tiles_y), 1, 64, w->stream, g, from,
-                         shape.tiles_x, g.hash_frame0 + (int)d, (int)m, shape.halo);
+                         shape.tiles_x, g.hash_frame0 + (int)d, (int)m, shape.side, shape.halo);
             from ^= 1;
             d += m;
         }
         at += nf;
     }
-    if (!rc) rc = launch2(K.unpack, (unsigned)(ctiles + 3) / 4, 1, 256, w->stream, g, from, wtiles, ctiles);
+    if (!rc) rc = launch2(K.unpack, (unsigned)(utiles + 3) / 4, 1, 256, w->stream, g, from, ucols, utiles);
     if (rc) return rc;
     sleep_reset(w);
     w->frame += (int32_t)n;

@@ -8,10 +8,10 @@
 // E and of O is the block of columns 2i and 2i + 1, and with the row below them a
 // word quadruple is 32 blocks, which se_sliced_block advances at once.
 //
-// Packed grid in memory: u16 [half column][row][2K].  A half column is 32 cells
-// wide; the entries of a row are E planes 0..K-1, then O planes.  Column c and
-// row m of it are the world's x = c - xpad and y = m - ypad; everything around
-// the world is WALL.
+// Packed grid in memory: 8 bytes [byte column][row], byte k < 4 plane k of E and
+// byte 4 + k plane k of O.  A byte column is 16 cells wide, so tiles start at any
+// multiple of 16 columns.  Column c and row m of it are the world's x = c - xpad and
+// y = m - ypad; everything around the world is WALL.
 //
 // Hash planes: bits of blocks, 32 blocks of a block row to a word.  The hash input of
 // the block with origin (x, y) in frame f depends on n = 461 x + 2131 y + 2131^2 f
@@ -28,17 +28,14 @@
 // 64w + 2i + 1, at an odd offset the block one column to the left; at an odd y offset
 // block row j is one row further down (rows 2j + 1 and 2j + 2).
 // ---------------------------------------------------------------------------
-typedef unsigned short u16;
-typedef unsigned short se_u16x4 __attribute__((ext_vector_type(4)));
-
 struct se_slgrid {  // == SlicedGrid (se_sliced.hpp)
     u32* in;        // the grid (u32 ids)
     u32* out;
-    u16* pk[2];     // packed grids
+    uint2* pk[2];   // packed grids
     u32* hash;      // hash planes of frames hash_frame0 ...
     int W, H, pitch;
-    int xpad, ypad, hcols, rows;  // packed geometry: columns of 32 cells, rows (a multiple of 64)
-    int brows;                    // block rows (even)
+    int xpad, ypad, bcols, rows;  // packed geometry: byte columns, rows (a multiple of 64)
+    int brows;                    // block rows
     int hash_frame0, hash_shared;
     int hash_pitch, hash_words;   // values of a, words of a plane
     u32 hash_n0[2];               // shared: n0 of the sets of even and of odd n
@@ -56,18 +53,10 @@ __device__ __forceinline__ u32 se_sl_map(u32 q, u32 t0, u32 t1, u32 t2, u32 t3) 
 #endif
 }
 __device__ __forceinline__ u32 se_sl_codes(u32 q) {
-#if SE_SL_REMAP
     return se_sl_map(q, SE_SL_CODE0, SE_SL_CODE1, SE_SL_CODE2, SE_SL_CODE3);
-#else
-    return q;
-#endif
 }
 __device__ __forceinline__ u32 se_sl_ids(u32 q) {
-#if SE_SL_REMAP
     return se_sl_map(q, SE_SL_ID0, SE_SL_ID1, SE_SL_ID2, SE_SL_ID3);
-#else
-    return q;
-#endif
 }
 
 // Swaps the bits of x above `m` (a mask of the low bits of each 2s-bit group)
@@ -120,36 +109,68 @@ __device__ __forceinline__ void se_sl_unslice(const u32* p, u32* d) {
 // (4 rows of 64 cells each), four codes to a word, through LDS to one row a lane
 // (a stride of 17 words keeps both sides free of bank conflicts), and there the
 // bits are transposed into planes.  Bound by HBM: 4 B of ids read per cell, and
-// K/8 B written.  The second packed grid gets the rows and half columns around
+// half a byte written.  The second packed grid gets the rows and columns around
 // the world too, which the step kernel reads and never writes.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ u16* se_sl_at(u16* p, const se_slgrid& g, int hcol, int row) {
-    return p + ((size_t)hcol * g.rows + row) * (2 * SE_SL_K);
+__device__ __forceinline__ uint2* se_sl_at(uint2* p, const se_slgrid& g, int bcol, int row) {
+    return p + ((size_t)bcol * g.rows + row);
 }
 
-__device__ __forceinline__ void se_sl_put(u16* p, const u32* e, const u32* o, int half) {
-    u16 v[2 * SE_SL_K];
+// The byte column of the world's column 64 * wc: packing and unpacking go by 64
+// columns of the world, so that their accesses to the ids are whole cache lines
+// (unpacking 16384^2 by 64 columns of the packed grid, 64 bytes off: 253 us for 198).
+__device__ __forceinline__ int se_sl_bcol(const se_slgrid& g, int wc) { return 4 * wc + (g.xpad >> 4); }
+
+// Planes of a row's 64 cells <-> its four byte columns.
+__device__ __forceinline__ void se_sl_columns(const u32* e, const u32* o, uint2* c) {
+    u32 a[4], b[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        a[k] = k < SE_SL_K ? e[k] : 0u;
+        b[k] = k < SE_SL_K ? o[k] : 0u;
+    }
+    se_sl_bytes4(a[0], a[1], a[2], a[3]);
+    se_sl_bytes4(b[0], b[1], b[2], b[3]);
+#pragma unroll
+    for (int q = 0; q < 4; q++) c[q] = make_uint2(a[q], b[q]);
+}
+__device__ __forceinline__ void se_sl_planes(const uint2* c, u32* e, u32* o) {
+    u32 a[4], b[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        a[q] = c[q].x;
+        b[q] = c[q].y;
+    }
+    se_sl_bytes4(a[0], a[1], a[2], a[3]);
+    se_sl_bytes4(b[0], b[1], b[2], b[3]);
 #pragma unroll
     for (int k = 0; k < SE_SL_K; k++) {
-        v[k] = (u16)(e[k] >> (16 * half));
-        v[SE_SL_K + k] = (u16)(o[k] >> (16 * half));
+        e[k] = a[k];
+        o[k] = b[k];
     }
-    u32* q = reinterpret_cast<u32*>(p);
-#pragma unroll
-    for (int k = 0; k < SE_SL_K; k++) q[k] = (u32)v[2 * k] | ((u32)v[2 * k + 1] << 16);
 }
 
 __device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int m0, u32* lds) {
     const int lane = (int)(threadIdx.x & 63);
-    const int x = 64 * wc - g.xpad + 4 * (lane & 15);
-    constexpr u32 WALL4 = SE_SL_WALL * 0x01010101u;
+    const int x = 16 * se_sl_bcol(g, wc) - g.xpad + 4 * (lane & 15);
+    const int y0 = m0 - g.ypad, xw = 16 * se_sl_bcol(g, wc) - g.xpad;
     uint4 v[16];
+    if (y0 >= 0 && y0 + 64 <= g.H && xw >= 0 && xw + 64 <= g.W) {  // all of the tile inside the world
+        const u32* s = g.in + (size_t)(y0 + (lane >> 4)) * g.pitch + x;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int y = m0 + 4 * i + (lane >> 4) - g.ypad;
-        v[i] = make_uint4(SE_WALLID, SE_WALLID, SE_WALLID, SE_WALLID);
-        if (y >= 0 && y < g.H && x >= 0 && x < g.W)
-            v[i] = *reinterpret_cast<const uint4*>(g.in + (size_t)y * g.pitch + x);
+        for (int i = 0; i < 16; i++) v[i] = se_load_nt(s + (size_t)(4 * i) * g.pitch);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int y = y0 + 4 * i + (lane >> 4);
+            const bool in = y >= 0 && y < g.H && x >= 0 && x < g.W;
+            uint4 t = *reinterpret_cast<const uint4*>(g.in + (in ? (size_t)y * g.pitch + x : 0));
+            t.x = in ? t.x : SE_WALLID;
+            t.y = in && x + 1 < g.W ? t.y : SE_WALLID;
+            t.z = in && x + 2 < g.W ? t.z : SE_WALLID;
+            t.w = in && x + 3 < g.W ? t.w : SE_WALLID;
+            v[i] = t;
+        }
     }
 #pragma unroll
     for (int i = 0; i < 16; i++) {
@@ -159,13 +180,7 @@ __device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int 
             q = se_pack4(se_decode(v[i].x), se_decode(v[i].y), se_decode(v[i].z), se_decode(v[i].w));
         else
             q = se_pack4(v[i].x, v[i].y, v[i].z, v[i].w);
-        q = se_sl_codes(q);
-        const int in = g.W - x;  // cells of the quad inside the world
-        if (in < 4 && in > 0) {
-            const u32 keep = 0xffffffffu >> (8 * (4 - in));
-            q = (q & keep) | (WALL4 & ~keep);
-        }
-        lds[(4 * i + (lane >> 4)) * 17 + (lane & 15)] = q;
+        lds[(4 * i + (lane >> 4)) * 17 + (lane & 15)] = se_sl_codes(q);
     }
     __builtin_amdgcn_wave_barrier();
     u32 q[16], e[SE_SL_K], o[SE_SL_K], de[8], dd[8];
@@ -183,13 +198,15 @@ __device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int 
     se_sl_slice(dd, o);
     const int row = m0 + lane;
     const bool around_y = row < g.ypad || row >= g.ypad + g.H;
+    uint2 cols[4];
+    se_sl_columns(e, o, cols);
 #pragma unroll
-    for (int half = 0; half < 2; half++) {
-        const int hc = 2 * wc + half;
-        if (hc >= g.hcols || row >= g.rows) continue;
-        se_sl_put(se_sl_at(g.pk[0], g, hc, row), e, o, half);
-        const int c = 32 * hc - g.xpad;
-        if (around_y || c < 0 || c + 32 > g.W) se_sl_put(se_sl_at(g.pk[1], g, hc, row), e, o, half);
+    for (int q = 0; q < 4; q++) {
+        const int bc = se_sl_bcol(g, wc) + q;
+        if (bc < 0 || bc >= g.bcols) continue;
+        *se_sl_at(g.pk[0], g, bc, row) = cols[q];
+        const int c = 16 * bc - g.xpad;
+        if (around_y || c < 0 || c + 16 > g.W) *se_sl_at(g.pk[1], g, bc, row) = cols[q];
     }
 }
 
@@ -197,24 +214,12 @@ __device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int 
 __device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, int wc, int m0, u32* lds) {
     const int lane = (int)(threadIdx.x & 63);
     u32 e[SE_SL_K], o[SE_SL_K], de[8], dd[8], q[16];
+    uint2 cols[4];
 #pragma unroll
-    for (int k = 0; k < SE_SL_K; k++) e[k] = o[k] = 0u;
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-        const int hc = 2 * wc + half, row = m0 + lane;
-        if (hc >= g.hcols || row >= g.rows) continue;
-        const u32* p = reinterpret_cast<const u32*>(se_sl_at(g.pk[from], g, hc, row));
-        u32 v[SE_SL_K];
-#pragma unroll
-        for (int k = 0; k < SE_SL_K; k++) v[k] = p[k];
-#pragma unroll
-        for (int k = 0; k < SE_SL_K; k++) {
-            const u32 ev = (v[k / 2] >> (16 * (k & 1))) & 0xffffu;
-            const u32 ov = (v[(SE_SL_K + k) / 2] >> (16 * ((SE_SL_K + k) & 1))) & 0xffffu;
-            e[k] |= ev << (16 * half);
-            o[k] |= ov << (16 * half);
-        }
-    }
+    for (int c = 0; c < 4; c++)
+        cols[c] = se_sl_bcol(g, wc) + c < g.bcols ? *se_sl_at(g.pk[from], g, se_sl_bcol(g, wc) + c, m0 + lane)
+                                                   : make_uint2(0u, 0u);
+    se_sl_planes(cols, e, o);
     se_sl_unslice(e, de);
     se_sl_unslice(o, dd);
 #pragma unroll
@@ -228,7 +233,7 @@ __device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, 
 #pragma unroll
     for (int m = 0; m < 16; m++) lds[lane * 17 + m] = se_sl_ids(q[m]);
     __builtin_amdgcn_wave_barrier();
-    const int x = 64 * wc - g.xpad + 4 * (lane & 15);
+    const int x = 16 * se_sl_bcol(g, wc) - g.xpad + 4 * (lane & 15);
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         const int y = m0 + 4 * i + (lane >> 4) - g.ypad;
@@ -246,11 +251,13 @@ __device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, 
     }
 }
 
+// wtiles columns of 64 cells, from the one left of the world on (se_sl_pack: the
+// margin is packed too), tiles in all
 extern "C" __global__ __launch_bounds__(256) void se_sl_pack(se_slgrid g, int wtiles, int tiles) {
     __shared__ u32 lds[4][64 * 17];
     const int wave = (int)(threadIdx.x >> 6), t = (int)blockIdx.x * 4 + wave;
     if (t >= tiles) return;
-    se_sl_pack_tile(g, t % wtiles, (t / wtiles) * 64, lds[wave]);
+    se_sl_pack_tile(g, t % wtiles - 1, (t / wtiles) * 64, lds[wave]);
 }
 
 extern "C" __global__ __launch_bounds__(256) void se_sl_unpack(se_slgrid g, int from, int wtiles, int tiles) {
@@ -326,23 +333,21 @@ extern "C" __global__ __launch_bounds__(256) void se_sl_hash(se_slgrid g) {
 //     columns) and the blocks are (O, E) instead of (E, O).
 // Blocks are never split between lanes otherwise, so there are no barriers and no
 // LDS.  What the shifts bring in at the tile's sides is wrong inside the world and
-// right at its border (WALL), so the valid region shrinks by one cell per
-// sub-step on the sides that cut into the world: 32 columns and `halo` rows are
-// given up on each side of a tile, none of a world that fits one tile.
+// right at its border (WALL, code 0), so the valid region shrinks by one cell per
+// sub-step on the sides that cut into the world: 16 or 32 columns and `halo` rows
+// are given up on each side of a tile, none of a world that fits one tile.
 // ---------------------------------------------------------------------------
 template <int NW, int R>
 struct se_sltile {
     u32 e[R][NW][SE_SL_K], o[R][NW][SE_SL_K];
 };
 
-__device__ __forceinline__ constexpr u32 se_sl_wall(int k) { return (SE_SL_WALL >> k) & 1u ? 0xffffffffu : 0u; }
-
-// lane i gets lane i + 1 (wave_shl), the last lane `fill`; and the other way round
-__device__ __forceinline__ u32 se_sl_from_below(u32 v, u32 fill) {
-    return (u32)__builtin_amdgcn_update_dpp((int)fill, (int)v, 0x130, 0xf, 0xf, false);
+// lane i gets lane i + 1 (wave_shl), the last lane 0 (WALL); and the other way round
+__device__ __forceinline__ u32 se_sl_from_below(u32 v) {
+    return (u32)__builtin_amdgcn_mov_dpp((int)v, 0x130, 0xf, 0xf, true);
 }
-__device__ __forceinline__ u32 se_sl_from_above(u32 v, u32 fill) {
-    return (u32)__builtin_amdgcn_update_dpp((int)fill, (int)v, 0x138, 0xf, 0xf, false);
+__device__ __forceinline__ u32 se_sl_from_above(u32 v) {
+    return (u32)__builtin_amdgcn_mov_dpp((int)v, 0x138, 0xf, 0xf, true);
 }
 
 template <int NW, int R>
@@ -351,7 +356,7 @@ __device__ __forceinline__ void se_sl_rows_up(se_sltile<NW, R>& t) {
     for (int w = 0; w < NW; w++)
 #pragma unroll
         for (int k = 0; k < SE_SL_K; k++) {
-            const u32 e = se_sl_from_below(t.e[0][w][k], se_sl_wall(k)), o = se_sl_from_below(t.o[0][w][k], se_sl_wall(k));
+            const u32 e = se_sl_from_below(t.e[0][w][k]), o = se_sl_from_below(t.o[0][w][k]);
 #pragma unroll
             for (int r = 0; r + 1 < R; r++) {
                 t.e[r][w][k] = t.e[r + 1][w][k];
@@ -368,8 +373,7 @@ __device__ __forceinline__ void se_sl_rows_down(se_sltile<NW, R>& t) {
     for (int w = 0; w < NW; w++)
 #pragma unroll
         for (int k = 0; k < SE_SL_K; k++) {
-            const u32 e = se_sl_from_above(t.e[R - 1][w][k], se_sl_wall(k)),
-                      o = se_sl_from_above(t.o[R - 1][w][k], se_sl_wall(k));
+            const u32 e = se_sl_from_above(t.e[R - 1][w][k]), o = se_sl_from_above(t.o[R - 1][w][k]);
 #pragma unroll
             for (int r = R - 1; r > 0; r--) {
                 t.e[r][w][k] = t.e[r - 1][w][k];
@@ -458,21 +462,21 @@ __device__ __forceinline__ void se_sl_hash_of(const se_slwords<NW, R>& r, u32 (&
 #if !SE_SL_KEEP
 // Puts back the WALL outside the world (rules may change it); ysh: rows moved up.
 template <int NW, int R>
-__device__ __forceinline__ void se_sl_keep_wall(se_sltile<NW, R>& t, const se_slgrid& g, int wc0, int y0) {
+__device__ __forceinline__ void se_sl_keep_wall(se_sltile<NW, R>& t, const se_slgrid& g, int c0, int y0) {
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const u32 rm = y0 + r >= 0 && y0 + r < g.H ? 0xffffffffu : 0u;
 #pragma unroll
         for (int w = 0; w < NW; w++) {
-            const int x0 = 64 * (wc0 + w) - g.xpad;  // column of bit 0 of E
+            const int x0 = c0 + 64 * w - g.xpad;  // column of bit 0 of E
             const int lo = x0 < 0 ? (-x0 + 1) / 2 : 0, lo1 = x0 < 0 ? -x0 / 2 : 0;
             const int hi = min(32, max(0, (g.W - x0 + 1) / 2)), hi1 = min(32, max(0, (g.W - x0) / 2));
             const u32 me = (u32)((1ull << hi) - 1ull) & ~(u32)((1ull << min(lo, 32)) - 1ull) & rm;
             const u32 mo = (u32)((1ull << hi1) - 1ull) & ~(u32)((1ull << min(lo1, 32)) - 1ull) & rm;
 #pragma unroll
             for (int k = 0; k < SE_SL_K; k++) {
-                t.e[r][w][k] = (t.e[r][w][k] & me) | (se_sl_wall(k) & ~me);
-                t.o[r][w][k] = (t.o[r][w][k] & mo) | (se_sl_wall(k) & ~mo);
+                t.e[r][w][k] &= me;
+                t.o[r][w][k] &= mo;
             }
         }
     }
@@ -491,7 +495,7 @@ __device__ __forceinline__ void se_sl_substep(se_sltile<NW, R>& t, const se_slwo
             for (int k = 0; k < SE_SL_K; k++)
 #pragma unroll
                 for (int w = NW - 1; w >= 0; w--)
-                    t.o[r][w][k] = __builtin_amdgcn_alignbit(t.o[r][w][k], w ? t.o[r][w - 1][k] : se_sl_wall(k), 31);
+                    t.o[r][w][k] = __builtin_amdgcn_alignbit(t.o[r][w][k], w ? t.o[r][w - 1][k] : 0u, 31);
     }
 #pragma unroll
     for (int w = 0; w < NW; w++)
@@ -507,7 +511,7 @@ __device__ __forceinline__ void se_sl_substep(se_sltile<NW, R>& t, const se_slwo
             for (int k = 0; k < SE_SL_K; k++)
 #pragma unroll
                 for (int w = 0; w < NW; w++)
-                    t.o[r][w][k] = __builtin_amdgcn_alignbit(w + 1 < NW ? t.o[r][w + 1][k] : se_sl_wall(k),
+                    t.o[r][w][k] = __builtin_amdgcn_alignbit(w + 1 < NW ? t.o[r][w + 1][k] : 0u,
                                                              t.o[r][w][k], 1);
     }
 }
@@ -525,11 +529,11 @@ __device__ __forceinline__ void se_sl_advance(se_sltile<NW, R>& t, const se_slgr
     u32 f = (u32)frame0;
     const u32 end = f + (u32)nsub, first = (f + 3u) & ~3u;
 #if !SE_SL_KEEP
-    const int wc0 = blk0 / 32;
-    const bool edge = 64 * wc0 < g.xpad || 64 * (wc0 + NW) > g.xpad + g.W || row0 < g.ypad ||
+    const int c0 = 2 * blk0;
+    const bool edge = c0 < g.xpad || c0 + 64 * NW > g.xpad + g.W || row0 < g.ypad ||
                       row0 + 64 * R > g.ypad + g.H;
     const int y0 = row0 + R * lane - g.ypad;
-#define SE_SL_FIX(up) if (edge) se_sl_keep_wall<NW, R>(t, g, wc0, y0 + (up))
+#define SE_SL_FIX(up) if (edge) se_sl_keep_wall<NW, R>(t, g, c0, y0 + (up))
 #else
 #define SE_SL_FIX(up)
 #endif
@@ -588,78 +592,71 @@ __device__ __forceinline__ void se_sl_advance(se_sltile<NW, R>& t, const se_slgr
 #undef SE_SL_FIX
 }
 
-// Rows of two neighbouring half columns <-> words (R rows x 2K planes each).
 template <int NW, int R>
-__device__ __forceinline__ void se_sl_load(se_sltile<NW, R>& t, u16* pk, const se_slgrid& g, int hc0, int row) {
-    constexpr int D = R * SE_SL_K;  // u32 of a lane's rows in one half column
+__device__ __forceinline__ void se_sl_load(se_sltile<NW, R>& t, const se_slgrid& g, int from, int bc0, int row) {
+    uint2 c[NW][4][R];
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint4* s = reinterpret_cast<const uint4*>(se_sl_at(g.pk[from], g, bc0 + 4 * w + q, row));
+#pragma unroll
+            for (int r = 0; r < R; r += 2) {  // row is even: two rows are 16 aligned bytes
+                const uint4 v = s[r / 2];
+                c[w][q][r] = make_uint2(v.x, v.y);
+                c[w][q][r + 1] = make_uint2(v.z, v.w);
+            }
+        }
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint2 col[4] = {c[w][0][r], c[w][1][r], c[w][2][r], c[w][3][r]};
+            se_sl_planes(col, t.e[r][w], t.o[r][w]);
+        }
+}
+
+// byte columns first .. last of the tile
+template <int NW, int R>
+__device__ __forceinline__ void se_sl_store(const se_sltile<NW, R>& t, const se_slgrid& g, int to, int bc0, int row,
+                                            int first, int last) {
 #pragma unroll
     for (int w = 0; w < NW; w++) {
-        const u32* a = reinterpret_cast<const u32*>(se_sl_at(pk, g, hc0 + 2 * w, row));
-        const u32* b = reinterpret_cast<const u32*>(se_sl_at(pk, g, hc0 + 2 * w + 1, row));
-        u32 va[D], vb[D];
+        uint2 col[R][4];
 #pragma unroll
-        for (int i = 0; i < D; i += 2) {
-            *reinterpret_cast<uint2*>(va + i) = *reinterpret_cast<const uint2*>(a + i);
-            *reinterpret_cast<uint2*>(vb + i) = *reinterpret_cast<const uint2*>(b + i);
-        }
+        for (int r = 0; r < R; r++) se_sl_columns(t.e[r][w], t.o[r][w], col[r]);
 #pragma unroll
-        for (int i = 0; i < 2 * D; i++) {
-            const int r = i / (2 * SE_SL_K), k = i % (2 * SE_SL_K);
-            const u32 v = __builtin_amdgcn_perm(vb[i / 2], va[i / 2], i & 1 ? 0x07060302u : 0x05040100u);
-            if (k < SE_SL_K) t.e[r][w][k] = v;
-            else t.o[r][w][k - SE_SL_K] = v;
+        for (int q = 0; q < 4; q++) {
+            if (4 * w + q < first || 4 * w + q > last) continue;
+            uint4* d = reinterpret_cast<uint4*>(se_sl_at(g.pk[to], g, bc0 + 4 * w + q, row));
+#pragma unroll
+            for (int r = 0; r < R; r += 2)
+                d[r / 2] = make_uint4(col[r][q].x, col[r][q].y, col[r + 1][q].x, col[r + 1][q].y);
         }
     }
 }
 
-template <int NW, int R>
-__device__ __forceinline__ void se_sl_store(const se_sltile<NW, R>& t, u16* pk, const se_slgrid& g, int hc0, int row,
-                                            int first, int last) {
-    constexpr int D = R * SE_SL_K;
-#pragma unroll
-    for (int hc = 0; hc < 2 * NW; hc++) {
-        if (hc < first || hc > last) continue;
-        u32* a = reinterpret_cast<u32*>(se_sl_at(pk, g, hc0 + hc, row));
-        u32 v[D];
-#pragma unroll
-        for (int i = 0; i < D; i++) {
-            u32 lo, hi;
-            {
-                const int r = 2 * i / (2 * SE_SL_K), k = 2 * i % (2 * SE_SL_K);
-                lo = k < SE_SL_K ? t.e[r][hc / 2][k] : t.o[r][hc / 2][k - SE_SL_K];
-            }
-            {
-                const int r = (2 * i + 1) / (2 * SE_SL_K), k = (2 * i + 1) % (2 * SE_SL_K);
-                hi = k < SE_SL_K ? t.e[r][hc / 2][k] : t.o[r][hc / 2][k - SE_SL_K];
-            }
-            v[i] = __builtin_amdgcn_perm(hi, lo, hc & 1 ? 0x07060302u : 0x05040100u);
-        }
-#pragma unroll
-        for (int i = 0; i < D; i += 2) *reinterpret_cast<uint2*>(a + i) = *reinterpret_cast<uint2*>(v + i);
-    }
-}
-
-// `from`: the packed grid read, the other is written.  halo 0: the world fits the
-// one tile, all of which is stored.
+// `from`: the packed grid read, the other is written.  side: byte columns given up
+// on each side (1 or 2, for up to 16 or 32 sub-steps), halo: rows; both 0: the
+// world fits the one tile, all of which is stored.
 template <int NW, int R, int AHEAD>
 __device__ __forceinline__ void se_sl_tile(const se_slgrid& g, int from, int tx, int ty, int frame0, int nsub,
-                                           int halo) {
+                                           int side, int halo) {
     const int lane = (int)(threadIdx.x & 63);
-    const int hc0 = tx * (2 * NW - 2), row0 = ty * (64 * R - 2 * halo);
+    const int bc0 = tx * (4 * NW - 2 * side), row0 = ty * (64 * R - 2 * halo);
     const int row = row0 + R * lane;
     se_sltile<NW, R> t;
-    se_sl_load<NW, R>(t, g.pk[from], g, hc0, row);
-    se_sl_advance<NW, R, AHEAD>(t, g, 16 * hc0, row0, lane, frame0, nsub);
+    se_sl_load<NW, R>(t, g, from, bc0, row);
+    se_sl_advance<NW, R, AHEAD>(t, g, 8 * bc0, row0, lane, frame0, nsub);
     if (R * lane < halo || R * lane >= 64 * R - halo) return;
-    if (halo == 0) se_sl_store<NW, R>(t, g.pk[from ^ 1], g, hc0, row, 0, 2 * NW - 1);
-    else se_sl_store<NW, R>(t, g.pk[from ^ 1], g, hc0, row, 1, 2 * NW - 2);
+    se_sl_store<NW, R>(t, g, from ^ 1, bc0, row, side, 4 * NW - 1 - side);
 }
 
-#define SE_SL_STEP(NW, R, AHEAD)                                                                                     \
-    extern "C" __global__ __launch_bounds__(64) void se_sl_step_##NW##x##R(se_slgrid g, int from, int tiles_x, \
-                                                                           int frame0, int nsub, int halo) {   \
+#define SE_SL_STEP(NW, R, AHEAD)                                                                              \
+    extern "C" __global__ __launch_bounds__(64, 2) void se_sl_step_##NW##x##R(                                    \
+        se_slgrid g, int from, int tiles_x, int frame0, int nsub, int side, int halo) {                        \
         const int tile = se_xcd_tile((int)blockIdx.x, (int)gridDim.x);                                         \
-        se_sl_tile<NW, R, AHEAD>(g, from, tile % tiles_x, tile / tiles_x, frame0, nsub, halo);                        \
+        se_sl_tile<NW, R, AHEAD>(g, from, tile % tiles_x, tile / tiles_x, frame0, nsub, side, halo);           \
     }
 SE_SL_STEP(2, 2, 4)
 SE_SL_STEP(4, 2, 2)

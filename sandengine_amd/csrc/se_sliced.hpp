@@ -11,10 +11,10 @@ namespace se_rt {
 struct SlicedGrid {
     uint32_t* in = nullptr;
     uint32_t* out = nullptr;
-    uint16_t* pk[2] = {nullptr, nullptr};
+    void* pk[2] = {nullptr, nullptr};
     uint32_t* hash = nullptr;
     int W = 0, H = 0, pitch = 0;
-    int xpad = 0, ypad = 0, hcols = 0, rows = 0;
+    int xpad = 0, ypad = 0, bcols = 0, rows = 0;
     int brows = 0;
     int hash_frame0 = 0, hash_shared = 0;
     int hash_pitch = 0, hash_words = 0;
@@ -26,7 +26,7 @@ static_assert(sizeof(SlicedGrid) == 96, "se_slgrid layout");
 struct SlicedShape {
     int kernel = 0;            // index into SlicedKernels::step
     int nw = 0, r = 0;         // words and rows of a lane
-    int halo = 0;              // rows given up on each side; 0: the world fits one tile
+    int side = 0, halo = 0;    // byte columns and rows given up on each side; 0: the world fits one tile
     int tiles_x = 0, tiles_y = 0;
     uint32_t max_sub = 0;      // sub-steps of one launch (any number when the world fits one tile)
 };
@@ -35,7 +35,7 @@ struct SlicedShape {
 SlicedShape sliced_shape(uint32_t W, uint32_t H, uint32_t sub);
 // Fills the geometry fields of g for that shape.
 void sliced_geometry(const SlicedShape& s, uint32_t W, uint32_t H, SlicedGrid& g);
-size_t sliced_packed_bytes(const SlicedGrid& g, int planes);  // of one packed grid
+size_t sliced_packed_bytes(const SlicedGrid& g);  // of one packed grid
 // Sets up the hash planes of frames [frame0, frame0 + nf) in g (all but the pointer):
 // the form and its sizes; returns their bytes, with room for the words that the step
 // kernel loads ahead.
