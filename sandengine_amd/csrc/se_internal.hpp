@@ -67,7 +67,8 @@ struct SlicedKernels {
     bool ok = false;
     int planes = 0, classes = 0;  // bit planes of a cell, hash planes of a frame
     hipFunction_t pack = nullptr, unpack = nullptr, hash = nullptr;
-    hipFunction_t step[2] = {};   // words x rows of a lane: 2x2, 4x2
+    hipFunction_t bpack = nullptr, bunpack = nullptr, bhash = nullptr;  // the worlds of a batch
+    hipFunction_t step[4] = {};  // 2x2 and 4x2 tiles by one wavefront (up to three planes), 2x2 by two, 4x2 by four
 };
 
 }  // namespace se_rt

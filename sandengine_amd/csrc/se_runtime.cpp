@@ -418,20 +418,27 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         HIPCHECK(hipModuleGetFunction(&K.pack, m->mod, "se_sl_pack"));
         HIPCHECK(hipModuleGetFunction(&K.unpack, m->mod, "se_sl_unpack"));
         HIPCHECK(hipModuleGetFunction(&K.hash, m->mod, "se_sl_hash"));
-        HIPCHECK(hipModuleGetFunction(&K.step[0], m->mod, "se_sl_step_2x2"));
-        HIPCHECK(hipModuleGetFunction(&K.step[1], m->mod, "se_sl_step_4x2"));
+        HIPCHECK(hipModuleGetFunction(&K.step[2], m->mod, "se_sl_step_2x2s"));
+        HIPCHECK(hipModuleGetFunction(&K.step[3], m->mod, "se_sl_step_4x2s"));
+        if (info.sliced.planes <= 3) {
+            HIPCHECK(hipModuleGetFunction(&K.step[0], m->mod, "se_sl_step_2x2"));
+            HIPCHECK(hipModuleGetFunction(&K.step[1], m->mod, "se_sl_step_4x2"));
+        }
+        HIPCHECK(hipModuleGetFunction(&K.bpack, m->mod, "se_sl_bpack"));
+        HIPCHECK(hipModuleGetFunction(&K.bunpack, m->mod, "se_sl_bunpack"));
+        HIPCHECK(hipModuleGetFunction(&K.bhash, m->mod, "se_sl_bhash"));
         K.planes = info.sliced.planes;
         K.classes = (int)info.sliced.classes.size();
         K.ok = true;
         // listed after the LDS instantiations (never the default among them)
-        m->lds.push_back({{128, 128, 32, 64, true}, K.step[0]});
+        m->lds.push_back({{128, 128, 32, 128, true}, K.step[2]});
         m->batch.push_back(nullptr);
         m->lds_bytes.push_back(0);
         int per_cu = 0, cus = 0;
-        HIPCHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, K.step[0], 64, 0));
+        HIPCHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, K.step[2], 128, 0));
         HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
         m->lds_grid.push_back(std::max(8, (std::max(per_cu, 1) * cus) & ~7));
-        m->lds_waves.push_back(std::max(per_cu, 1));
+        m->lds_waves.push_back(2 * std::max(per_cu, 1));
     }
     std::lock_guard<std::mutex> lk(ctx->mu);
     ctx->cache[key] = {src, m};
@@ -605,7 +612,7 @@ int blocked_steps(se_world* w, uint32_t nsteps, uint32_t sub) {
     }
     auto* v = pick_lds(w, sub);
     if (!v) return fail(SE_ERR_ARG, "no LDS variant supports " + std::to_string(sub) + " sub-steps");
-    if (v->first.sliced || (w->lds_variant < 0 && se_rt::sliced_pays(w, nsteps))) {
+    if (v->first.sliced || (w->lds_variant < 0 && se_rt::sliced_pays(w->mod.get(), nsteps))) {
         // the sliced kernels take neither the clearing frame nor modifications: the
         // step that carries them is a plain one
         if (nsteps && (w->frame + 1 == 1 || !w->pending.empty())) {

@@ -18,9 +18,16 @@ namespace {
 constexpr size_t kHashBudget = 128u << 20;  // hash planes made ahead, unless one launch needs more
 
 struct Tile {
-    int nw, r;
+    int nw, r, waves;
 };
-constexpr Tile kTiles[2] = {{2, 2}, {4, 2}};  // as instantiated in se_sliced.hip
+constexpr Tile kTiles[4] = {{2, 2, 1}, {4, 2, 1}, {2, 2, 2}, {4, 2, 4}};  // as instantiated in se_sliced.hip
+
+void set_tile(se_rt::SlicedShape& s, int kernel) {
+    s.kernel = kernel;
+    s.nw = kTiles[kernel].nw;
+    s.r = kTiles[kernel].r;
+    s.threads = 64u * kTiles[kernel].waves;
+}
 
 template <typename... A>
 int launch2(hipFunction_t f, unsigned gx, unsigned gy, unsigned block, hipStream_t s, A... args) {
@@ -32,37 +39,53 @@ int launch2(hipFunction_t f, unsigned gx, unsigned gy, unsigned block, hipStream
 
 }  // namespace
 
-se_rt::SlicedShape se_rt::sliced_shape(uint32_t W, uint32_t H, uint32_t sub) {
+// A world with its WALL border inside one tile needs no halo: one column and one row
+// more than the world has to the right and below (the wave shifts bring WALL in from
+// the other sides).
+se_rt::SlicedShape se_rt::sliced_one_tile(uint32_t W, uint32_t H, bool wide) {
     SlicedShape s;
-    // A world with its WALL border inside one tile needs no halo: one column and
-    // one row more than the world has to the right and below (the wave shifts
-    // bring WALL in from the other sides).
-    for (int i = 0; i < 2; i++) {
+    for (int i = 2; i < (wide ? 4 : 3) && !s.nw; i++) {
         if (W + 4 > 64u * kTiles[i].nw - 1 || H + 2 > 64u * kTiles[i].r) continue;
-        s.kernel = i;
-        s.nw = kTiles[i].nw;
-        s.r = kTiles[i].r;
+        set_tile(s, i);
         s.tiles_x = s.tiles_y = 1;
-        s.max_sub = sub ? sub : 1u << 20;
-        return s;
+        s.max_sub = 1u << 20;
     }
-    // The tile and the depth of a launch, by how many 2x2 tiles (64 useful columns and
-    // rows at 32 sub-steps) the world makes.  Up to one a SIMD the launches are a
-    // serial chain of sub-steps: the smallest tile and the deepest launch
-    // (1000x700: 132 us for 200 steps, 214 with 4x2, 155 with 16 sub-steps).  Beyond
-    // that the rows and columns given up count (16 columns a side up to 16
-    // sub-steps, 32 beyond), and from 8 a SIMD on the wider tile pays (4096^2, 200
-    // steps: 456 us with 2x2 and 16, 494 with 4x2, 526 with 32; 16384^2, 100 steps:
-    // 1.45 ms with 4x2 and 12, 1.55 with 16, 1.56 with 2x2; twelve materials at
-    // 8192^2, 64 steps: 761, 800 and 770 us).
-    const size_t few = (size_t)((W + 63) / 64) * ((H + 63) / 64);
-    const int i = few > 8192 ? 1 : 0;
-    const uint32_t deep = few > 8192 ? 12 : few > 1024 ? 16 : 32;
+    return s;
+}
 
-    s.kernel = i;
-    s.nw = kTiles[i].nw;
-    s.r = kTiles[i].r;
-    s.max_sub = sub ? std::min(sub, deep) : deep;
+// The tile and the depth of a launch, by how many squares of 64 x 64 cells the worlds
+// make.  While those leave SIMDs idle a launch is a serial chain of sub-steps: split
+// tiles, the small one first, and the deepest launch.  Beyond that the rows and
+// columns given up count (16 columns a side up to 16 sub-steps, 32 beyond), and
+// where one wavefront a tile has the registers for it, the barriers.  us a call
+// (2x2s 32 deep / 4x2s 32 / 2x2 16 / 4x2s 16, and from the third on 4x2 12):
+//   1000x700   200 steps  113 / 120 / 160 / 138
+//   2000x1900  200 steps  184 / 186 / 209 / 183 / 299
+//   4096^2     200 steps  544 / 476 / 445 / 455 / 511
+//   16384^2    100 steps     -      / 1505 / 1477 / 1367
+// and with four planes (2x2s 32 / 4x2s 32 / 2x2s 16 / 4x2s 16)
+//   800^2      150 steps  152 / 161 / 168 / 176
+//   1537x1111  150 steps  221 / 191 / 199 / 203
+//   4096^2      64 steps  433 / 366 / 338 / 341
+//   8192^2      64 steps    -  /  -  / 703 / 646
+void se_rt::sliced_choice(size_t few, const SlicedKernels& K, int* kernel, uint32_t* deep) {
+    const bool one_wave = K.step[0] != nullptr;
+    if (few <= 2048) {
+        *kernel = few <= 256 ? 2 : 3;
+        *deep = 32;
+    } else if (few <= 8192) {
+        *kernel = one_wave ? 0 : 2;
+        *deep = 16;
+    } else {
+        *kernel = one_wave ? 1 : 3;
+        *deep = one_wave ? 12 : 16;
+    }
+}
+
+se_rt::SlicedShape se_rt::sliced_tiles(uint32_t W, uint32_t H, int kernel, uint32_t max_sub) {
+    SlicedShape s;
+    set_tile(s, kernel);
+    s.max_sub = std::min(max_sub, 32u);
     s.halo = (int)(s.max_sub + 3) & ~3;
     s.side = s.max_sub > 16 ? 2 : 1;
     const uint32_t ux = 64u * s.nw - 32u * s.side, uy = 64u * s.r - 2u * s.halo;  // useful columns and rows of a tile
@@ -70,6 +93,11 @@ se_rt::SlicedShape se_rt::sliced_shape(uint32_t W, uint32_t H, uint32_t sub) {
     s.tiles_y = (int)((H + uy - 1) / uy);
     return s;
 }
+
+// Packing covers the margins (one column of 64 more on the left); unpacking the
+// world's columns.
+int se_rt::sliced_pack_tiles(const SlicedGrid& g) { return (1 + (g.bcols - g.xpad / 16 + 3) / 4) * (g.rows / 64); }
+int se_rt::sliced_unpack_columns(const SlicedGrid& g) { return (g.W + (g.xpad & 15) + 63) / 64; }
 
 void se_rt::sliced_geometry(const SlicedShape& s, uint32_t W, uint32_t H, SlicedGrid& g) {
     g.W = (int)W;
@@ -109,8 +137,9 @@ size_t se_rt::sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int
     for (int c = 0; c < 2; c++) {
         const int64_t m = (hi[c] - lo[c]) / 2 + 2131ll * g.brows + 461ll * 32 * (wcols + 1);
         words = std::max(words, (m / 461 + 2144) / 32 + 2);
-        g.hash_n0[c] = (uint32_t)lo[c];
     }
+    g.hash_n0 = (uint32_t)lo[0];
+    g.hash_n1 = (uint32_t)lo[1];
     // The shared form where it hashes less: its sets hold every n between the first
     // and the last, 4.5 M more with each frame, used or not.  16384^2 (67 M blocks a
     // frame) takes 1.6 us a frame and 21 direct, 8192^2 with twelve materials (17 M) 4
@@ -121,10 +150,10 @@ size_t se_rt::sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int
     g.hash_words = (int)(g.hash_shared ? words * 464 : (int64_t)wcols * g.brows);
     // The step kernel loads up to four frames past the last one and a word past a
     // row's last: 4 * 4541161 / 2 / 461 bits further on, or four more frames.
-    const size_t sets = g.hash_shared ? 2 : nf;
+    g.hash_sets = g.hash_shared ? 2 : (int)nf;
     const size_t past = g.hash_shared ? (size_t)(4 * 4541161 / 2 / 461 / 32 + 70) * 464
                                       : 4 * (size_t)g.hash_words + g.brows;
-    return (sets * g.hash_words + past) * classes * sizeof(uint32_t);
+    return ((size_t)g.hash_sets * g.hash_words + past) * classes * sizeof(uint32_t);
 }
 
 // Packing, hashing and unpacking cost three launches more than the LDS kernels
@@ -134,21 +163,30 @@ size_t se_rt::sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int
 // against sliced, us: four materials 256^2 8 steps 22 and 19, 12 steps 37 and 20;
 // 4096^2 46 and 55, 83 and 64; 16384^2 427 and 567, 831 and 607; twelve at 8192^2
 // 226 and 223, 368 and 261; feature rules 4096^2 2 steps 52 and 53, 4 steps 88 and 66).
-bool se_rt::sliced_pays(const se_world* w, uint32_t n) {
-    return w->mod->sliced.ok && n >= (w->mod->table_form == 0 ? 4u : 9u);
+bool se_rt::sliced_pays(const se_module* m, uint32_t n) {
+    return m->sliced.ok && n >= (m->table_form == 0 ? 4u : 9u);
 }
 
 int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     *done = false;
     const SlicedKernels& K = w->mod->sliced;
-    const SlicedShape shape = sliced_shape(w->W, w->H, sub);
-    SlicedGrid g;
+    SlicedShape shape = sliced_one_tile(w->W, w->H, true);
+    if (!shape.nw) {
+        int kernel;
+        uint32_t deep;
+        sliced_choice(sliced_squares(w->W, w->H), K, &kernel, &deep);
+        shape = sliced_tiles(w->W, w->H, kernel, sub ? std::min(sub, deep) : deep);
+    } else if (sub) {
+        shape.max_sub = sub;
+    }
+    SlicedWorld one;
+    SlicedGrid& g = one.g;
     sliced_geometry(shape, w->W, w->H, g);
     g.pitch = (int)w->pitch;
     const size_t packed = sliced_packed_bytes(g);
     const uint32_t per_launch = std::min(shape.max_sub, n);
     // frames hashed at a time: as many whole launches as the budget holds
-    uint32_t ahead = n;
+    uint32_t ahead = std::min(n, kSlicedMostFrames);
     size_t hash = sliced_hash_layout(g, w->frame + 1, ahead, K.classes);
     while (hash > kHashBudget && ahead > (shape.halo ? per_launch : 1u)) {
         ahead = ahead / 2;
@@ -174,22 +212,26 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
         ctx->sliced_bytes = bytes;
     }
     *done = true;
+    one.frame0 = w->frame + 1;
+    one.steps = (int)n;
+    one.tiles_x = shape.tiles_x;
+    one.side = shape.side;
+    one.halo = shape.halo;
     g.in = w->buf[w->cur];
     g.out = w->buf[w->cur ^ 1];
-    g.pk[0] = ctx->sliced_mem;
-    g.pk[1] = (char*)ctx->sliced_mem + packed;
+    g.pk0 = ctx->sliced_mem;
+    g.pk1 = (char*)ctx->sliced_mem + packed;
     g.hash = (uint32_t*)((char*)ctx->sliced_mem + 2 * packed);
 
-    // 64 columns x 64 rows a wavefront; packing also covers the margins
-    const int pcols = 1 + (g.bcols - g.xpad / 16 + 3) / 4, ptiles = pcols * (g.rows / 64);
-    const int ucols = (int)(w->W + (g.xpad & 15) + 63) / 64, utiles = ucols * (g.rows / 64);
+    const int ptiles = sliced_pack_tiles(g), pcols = ptiles / (g.rows / 64);
+    const int ucols = sliced_unpack_columns(g), utiles = ucols * (g.rows / 64);
     int rc = launch2(K.pack, (unsigned)(ptiles + 3) / 4, 1, 256, w->stream, g, pcols, ptiles);
     int from = 0;
     for (uint32_t at = 0; at < n && !rc;) {
         const uint32_t nf = std::min(ahead, n - at);
         const size_t need = sliced_hash_layout(g, w->frame + 1 + (int)at, nf, K.classes);
         if (2 * packed + need > ctx->sliced_bytes) return fail(SE_ERR_STATE, "internal: hash planes exceed their scratch");
-        rc = launch2(K.hash, (unsigned)(g.hash_words + 255) / 256, g.hash_shared ? 2u : nf, 256, w->stream, g);
+        rc = launch2(K.hash, (unsigned)(g.hash_words + 255) / 256, (unsigned)g.hash_sets, 256, w->stream, g);
         for (uint32_t d = 0; d < nf && !rc;) {
             // a launch after the first starts at the head of a cycle where that costs
             // no further launch
@@ -198,8 +240,9 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
             if (m < nf - d && lead < m && (nf - d - (m - lead) + shape.max_sub - 1) / shape.max_sub ==
                                               (nf - d - m + shape.max_sub - 1) / shape.max_sub)
                 m -= lead;
-            rc = launch2(K.step[shape.kernel], (unsigned)(shape.tiles_x * shape.tiles_y), 1, 64, w->stream, g, from,
-                         shape.tiles_x, g.hash_frame0 + (int)d, (int)m, shape.side, shape.halo);
+            rc = launch2(K.step[shape.kernel], (unsigned)(shape.tiles_x * shape.tiles_y), 1, shape.threads, w->stream, one,
+                         (const SlicedWorld*)nullptr, (const int*)nullptr, 0, (const SlicedGrid*)nullptr, from,
+                         (int)(at + d), (int)m);
             from ^= 1;
             d += m;
         }

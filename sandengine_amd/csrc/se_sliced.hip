@@ -29,17 +29,23 @@
 // block row j is one row further down (rows 2j + 1 and 2j + 2).
 // ---------------------------------------------------------------------------
 struct se_slgrid {  // == SlicedGrid (se_sliced.hpp)
-    u32* in;        // the grid (u32 ids)
-    u32* out;
-    uint2* pk[2];   // packed grids
-    u32* hash;      // hash planes of frames hash_frame0 ...
+    // addresses (as numbers: a pointer read from a record in memory would be generic,
+    // and its accesses wait on the LDS counter too)
+    u64 in, out;    // the grid (u32 ids)
+    u64 pk0, pk1;   // packed grids
+    u64 hash;       // hash planes of frames hash_frame0 ...
     int W, H, pitch;
     int xpad, ypad, bcols, rows;  // packed geometry: byte columns, rows (a multiple of 64)
     int brows;                    // block rows
-    int hash_frame0, hash_shared;
+    int hash_frame0, hash_shared, hash_sets;
     int hash_pitch, hash_words;   // values of a, words of a plane
-    u32 hash_n0[2];               // shared: n0 of the sets of even and of odd n
+    u32 hash_n0, hash_n1;         // shared: n0 of the sets of even and of odd n
 };
+
+template <typename T>
+__device__ __forceinline__ T* se_sl_ptr(u64 a) {
+    return (T*)(__attribute__((address_space(1))) T*)a;
+}
 
 // Codes of four ids < SE_NMAT packed in bytes, and ids of four codes.
 __device__ __forceinline__ u32 se_sl_map(u32 q, u32 t0, u32 t1, u32 t2, u32 t3) {
@@ -112,8 +118,8 @@ __device__ __forceinline__ void se_sl_unslice(const u32* p, u32* d) {
 // half a byte written.  The second packed grid gets the rows and columns around
 // the world too, which the step kernel reads and never writes.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint2* se_sl_at(uint2* p, const se_slgrid& g, int bcol, int row) {
-    return p + ((size_t)bcol * g.rows + row);
+__device__ __forceinline__ uint2* se_sl_at(const se_slgrid& g, int which, int bcol, int row) {
+    return se_sl_ptr<uint2>(which ? g.pk1 : g.pk0) + ((size_t)bcol * g.rows + row);
 }
 
 // The byte column of the world's column 64 * wc: packing and unpacking go by 64
@@ -156,7 +162,7 @@ __device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int 
     const int y0 = m0 - g.ypad, xw = 16 * se_sl_bcol(g, wc) - g.xpad;
     uint4 v[16];
     if (y0 >= 0 && y0 + 64 <= g.H && xw >= 0 && xw + 64 <= g.W) {  // all of the tile inside the world
-        const u32* s = g.in + (size_t)(y0 + (lane >> 4)) * g.pitch + x;
+        const u32* s = se_sl_ptr<const u32>(g.in) + (size_t)(y0 + (lane >> 4)) * g.pitch + x;
 #pragma unroll
         for (int i = 0; i < 16; i++) v[i] = se_load_nt(s + (size_t)(4 * i) * g.pitch);
     } else {
@@ -164,7 +170,7 @@ __device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int 
         for (int i = 0; i < 16; i++) {
             const int y = y0 + 4 * i + (lane >> 4);
             const bool in = y >= 0 && y < g.H && x >= 0 && x < g.W;
-            uint4 t = *reinterpret_cast<const uint4*>(g.in + (in ? (size_t)y * g.pitch + x : 0));
+            uint4 t = *reinterpret_cast<const uint4*>(se_sl_ptr<const u32>(g.in) + (in ? (size_t)y * g.pitch + x : 0));
             t.x = in ? t.x : SE_WALLID;
             t.y = in && x + 1 < g.W ? t.y : SE_WALLID;
             t.z = in && x + 2 < g.W ? t.z : SE_WALLID;
@@ -204,9 +210,9 @@ __device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int 
     for (int q = 0; q < 4; q++) {
         const int bc = se_sl_bcol(g, wc) + q;
         if (bc < 0 || bc >= g.bcols) continue;
-        *se_sl_at(g.pk[0], g, bc, row) = cols[q];
+        *se_sl_at(g, 0, bc, row) = cols[q];
         const int c = 16 * bc - g.xpad;
-        if (around_y || c < 0 || c + 16 > g.W) *se_sl_at(g.pk[1], g, bc, row) = cols[q];
+        if (around_y || c < 0 || c + 16 > g.W) *se_sl_at(g, 1, bc, row) = cols[q];
     }
 }
 
@@ -217,7 +223,7 @@ __device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, 
     uint2 cols[4];
 #pragma unroll
     for (int c = 0; c < 4; c++)
-        cols[c] = se_sl_bcol(g, wc) + c < g.bcols ? *se_sl_at(g.pk[from], g, se_sl_bcol(g, wc) + c, m0 + lane)
+        cols[c] = se_sl_bcol(g, wc) + c < g.bcols ? *se_sl_at(g, from, se_sl_bcol(g, wc) + c, m0 + lane)
                                                    : make_uint2(0u, 0u);
     se_sl_planes(cols, e, o);
     se_sl_unslice(e, de);
@@ -239,7 +245,7 @@ __device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, 
         const int y = m0 + 4 * i + (lane >> 4) - g.ypad;
         const u32 p = lds[(4 * i + (lane >> 4)) * 17 + (lane & 15)];
         if (y < 0 || y >= g.H || x < 0 || x >= g.W) continue;
-        u32* dst = g.out + (size_t)y * g.pitch + x;
+        u32* dst = se_sl_ptr<u32>(g.out) + (size_t)y * g.pitch + x;
         const uint4 v = make_uint4(p & 0xffu, (p >> 8) & 0xffu, (p >> 16) & 0xffu, p >> 24);
         if (x + 3 < g.W) {
             se_store_quad<true>(dst, v);
@@ -285,14 +291,12 @@ __device__ __forceinline__ void se_sl_push(u32& acc, u32 h, u32 t) {
     __asm__("v_cmp_ge_u32 vcc, %2, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(acc) : "v"(h), "s"(t) : "vcc");
 }
 
-// grid: x over the words of a plane, y over the sets
-extern "C" __global__ __launch_bounds__(256) void se_sl_hash(se_slgrid g) {
-    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x, set = (int)blockIdx.y;
-    if (i >= g.hash_words) return;
+// word i of a set
+__device__ __forceinline__ void se_sl_hash_word(const se_slgrid& g, int i, int set) {
     const int u = i / g.hash_pitch, a = i - u * g.hash_pitch;
     u32 n;  // of the block at bit 31
     if (g.hash_shared) {
-        n = g.hash_n0[set] + 2u * (2131u * (u32)a + 461u * (u32)(32 * u + 31 - SE_SL_B0));
+        n = (set ? g.hash_n1 : g.hash_n0) + 2u * (2131u * (u32)a + 461u * (u32)(32 * u + 31 - SE_SL_B0));
     } else {
         const u32 f = (u32)(g.hash_frame0 + set);
         int ox, oy;
@@ -317,13 +321,19 @@ extern "C" __global__ __launch_bounds__(256) void se_sl_hash(se_slgrid g) {
 #pragma unroll
         for (int p = 0; p < SE_SL_P; p++) se_sl_push(acc[p], h[se_sliced_class_lane(p)], se_sliced_class_max(p));
     }
-    u32* out = g.hash + ((size_t)set * g.hash_words + i) * SE_SL_P;
+    u32* out = se_sl_ptr<u32>(g.hash) + ((size_t)set * g.hash_words + i) * SE_SL_P;
 #pragma unroll
     for (int p = 0; p < SE_SL_P; p++) out[p] = acc[p];
 }
 
+// grid: x over the words of a plane, y over the sets
+extern "C" __global__ __launch_bounds__(256) void se_sl_hash(se_slgrid g) {
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (i < g.hash_words) se_sl_hash_word(g, i, (int)blockIdx.y);
+}
+
 // ---------------------------------------------------------------------------
-// Step kernel: one wavefront advances a tile of NW words (64 * NW columns) by
+// Step kernel: S wavefronts advance a tile of S * NW words (64 columns each) by
 // 64 * R rows through `nsub` sub-steps entirely in registers.  Lane l holds rows
 // R*l .. R*l + R - 1 of every word column.
 //   * y offset 1: every lane gives its first row to the lane above it (a wave
@@ -331,8 +341,8 @@ extern "C" __global__ __launch_bounds__(256) void se_sl_hash(se_slgrid g) {
 //     tile's outermost rows take WALL.
 //   * x offset 1: the O words move up by one block (alignbit over the word
 //     columns) and the blocks are (O, E) instead of (E, O).
-// Blocks are never split between lanes otherwise, so there are no barriers and no
-// LDS.  What the shifts bring in at the tile's sides is wrong inside the world and
+// Blocks are never split between lanes otherwise, so one wavefront needs no barriers
+// and no LDS; two that share a tile exchange a word column at odd x offsets.  What the shifts bring in at the tile's sides is wrong inside the world and
 // right at its border (WALL, code 0), so the valid region shrinks by one cell per
 // sub-step on the sides that cut into the world: 16 or 32 columns and `halo` rows
 // are given up on each side of a tile, none of a world that fits one tile.
@@ -402,7 +412,8 @@ __device__ __forceinline__ se_slplace<R> se_sl_place(const se_slgrid& g, u32 f, 
     int ox, oy;
     se_offset(f, ox, oy);
     const u32 parity = (u32)(ox + oy + (int)f) & 1u;
-    const u32 m = (461u * (u32)(-ox - g.xpad) + 2131u * (u32)(oy - g.ypad) + 4541161u * f - g.hash_n0[parity]) >> 1;
+    const u32 m = (461u * (u32)(-ox - g.xpad) + 2131u * (u32)(oy - g.ypad) + 4541161u * f -
+                   (parity ? g.hash_n1 : g.hash_n0)) >> 1;
     const u32 a0 = m % 461u * 204u % 461u;  // 204 * 2131 = 1 mod 461
     const u32 b0 = (m + 461u * SE_SL_B0 - 2131u * a0) / 461u;
     const bool sh = g.hash_shared != 0;
@@ -427,7 +438,7 @@ __device__ __forceinline__ void se_sl_hash_load(const se_slgrid& g, const se_slp
         h.shift[i] = q.b[i];  // alignbit takes it modulo 32
 #pragma unroll
         for (int w = 0; w <= NW; w++) {
-            const u32* s = g.hash + (size_t)w * (size_t)(g.hash_pitch * SE_SL_P);
+            const u32* s = se_sl_ptr<const u32>(g.hash) + (size_t)w * (size_t)(g.hash_pitch * SE_SL_P);
 #pragma unroll
             for (int p = 0; p < SE_SL_P; p++) h.v[i][w][p] = s[at + (u32)p];
         }
@@ -483,20 +494,82 @@ __device__ __forceinline__ void se_sl_keep_wall(se_sltile<NW, R>& t, const se_sl
 }
 #endif
 
+// The wavefronts of a tile (S of them side by side, NW word columns each) pass the
+// O words at their common side through LDS: lds[side][row][plane][lane], for the
+// shift up and for the shift down in turn, one barrier each.  A set is written
+// again only after the barrier that follows its reads.
+template <int R, int S>
+struct se_slshare {
+    u32 up[S - 1][R][SE_SL_K][64], down[S - 1][R][SE_SL_K][64];
+};
+template <int R>
+struct se_slshare<R, 1> {};
+
+template <int NW, int R, int S>
+__device__ __forceinline__ void se_sl_shift_up(se_sltile<NW, R>& t, se_slshare<R, S>& sh, int wv, int lane) {
+    u32 in[R][SE_SL_K];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int k = 0; k < SE_SL_K; k++) in[r][k] = 0u;
+    if constexpr (S > 1) {
+        if (wv < S - 1)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int k = 0; k < SE_SL_K; k++) sh.up[wv][r][k][lane] = t.o[r][NW - 1][k];
+        __syncthreads();
+        if (wv > 0)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int k = 0; k < SE_SL_K; k++) in[r][k] = sh.up[wv - 1][r][k][lane];
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int k = 0; k < SE_SL_K; k++)
+#pragma unroll
+            for (int w = NW - 1; w >= 0; w--)
+                t.o[r][w][k] = __builtin_amdgcn_alignbit(t.o[r][w][k], w ? t.o[r][w - 1][k] : in[r][k], 31);
+}
+
+template <int NW, int R, int S>
+__device__ __forceinline__ void se_sl_shift_down(se_sltile<NW, R>& t, se_slshare<R, S>& sh, int wv, int lane) {
+    u32 in[R][SE_SL_K];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int k = 0; k < SE_SL_K; k++) in[r][k] = 0u;
+    if constexpr (S > 1) {
+        if (wv > 0)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int k = 0; k < SE_SL_K; k++) sh.down[wv - 1][r][k][lane] = t.o[r][0][k];
+        __syncthreads();
+        if (wv < S - 1)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int k = 0; k < SE_SL_K; k++) in[r][k] = sh.down[wv][r][k][lane];
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int k = 0; k < SE_SL_K; k++)
+#pragma unroll
+            for (int w = 0; w < NW; w++)
+                t.o[r][w][k] = __builtin_amdgcn_alignbit(w + 1 < NW ? t.o[r][w + 1][k] : in[r][k], t.o[r][w][k], 1);
+}
+
 // One sub-step at x offset OX with the rows already paired (y offset applied).
-template <int NW, int R, bool OX>
-__device__ __forceinline__ void se_sl_substep(se_sltile<NW, R>& t, const se_slwords<NW, R>& raw) {
+template <int NW, int R, int S, bool OX>
+__device__ __forceinline__ void se_sl_substep(se_sltile<NW, R>& t, const se_slwords<NW, R>& raw, se_slshare<R, S>& sh,
+                                              int wv, int lane) {
     u32 h[R / 2][NW][SE_SL_P];
     se_sl_hash_of<NW, R>(raw, h);
-    if (OX) {
-#pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int k = 0; k < SE_SL_K; k++)
-#pragma unroll
-                for (int w = NW - 1; w >= 0; w--)
-                    t.o[r][w][k] = __builtin_amdgcn_alignbit(t.o[r][w][k], w ? t.o[r][w - 1][k] : 0u, 31);
-    }
+    if (OX) se_sl_shift_up<NW, R, S>(t, sh, wv, lane);
 #pragma unroll
     for (int w = 0; w < NW; w++)
 #pragma unroll
@@ -504,16 +577,7 @@ __device__ __forceinline__ void se_sl_substep(se_sltile<NW, R>& t, const se_slwo
             if (OX) se_sliced_block(t.o[2 * b][w], t.e[2 * b][w], t.o[2 * b + 1][w], t.e[2 * b + 1][w], h[b][w]);
             else se_sliced_block(t.e[2 * b][w], t.o[2 * b][w], t.e[2 * b + 1][w], t.o[2 * b + 1][w], h[b][w]);
         }
-    if (OX) {
-#pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int k = 0; k < SE_SL_K; k++)
-#pragma unroll
-                for (int w = 0; w < NW; w++)
-                    t.o[r][w][k] = __builtin_amdgcn_alignbit(w + 1 < NW ? t.o[r][w + 1][k] : 0u,
-                                                             t.o[r][w][k], 1);
-    }
+    if (OX) se_sl_shift_down<NW, R, S>(t, sh, wv, lane);
 }
 
 // Whole cycles of four frames run in a loop of their own: every offset is a
@@ -521,9 +585,9 @@ __device__ __forceinline__ void se_sl_substep(se_sltile<NW, R>& t, const se_slwo
 // names.  Up to three frames before and after them take the general step.  The
 // hash words are loaded AHEAD frames before their use: a 2x2 tile's sub-step takes
 // 0.3 us, and the words come from beyond the L2.
-template <int NW, int R, int AHEAD>
+template <int NW, int R, int S, int AHEAD>
 __device__ __forceinline__ void se_sl_advance(se_sltile<NW, R>& t, const se_slgrid& g, int blk0, int row0, int lane,
-                                              int frame0, int nsub) {
+                                              int frame0, int nsub, se_slshare<R, S>& sh, int wv) {
     static_assert(AHEAD == 2 || AHEAD == 4, "sets of words by phase");
     const int j0 = row0 / 2 + (R / 2) * lane;
     u32 f = (u32)frame0;
@@ -541,8 +605,8 @@ __device__ __forceinline__ void se_sl_advance(se_sltile<NW, R>& t, const se_slgr
         int ox, oy;
         se_offset(fr, ox, oy);
         if (oy) se_sl_rows_up(t);
-        if (ox) se_sl_substep<NW, R, true>(t, h);
-        else se_sl_substep<NW, R, false>(t, h);
+        if (ox) se_sl_substep<NW, R, S, true>(t, h, sh, wv, lane);
+        else se_sl_substep<NW, R, S, false>(t, h, sh, wv, lane);
         SE_SL_FIX(oy);
         if (oy) se_sl_rows_down(t);
     };
@@ -563,21 +627,21 @@ __device__ __forceinline__ void se_sl_advance(se_sltile<NW, R>& t, const se_slgr
         // (the last cycle's loads run on into the frames after the last: the planes
         // have room for them)
         do {
-            se_sl_substep<NW, R, false>(t, h[0]);          // offsets (0, 0)
+            se_sl_substep<NW, R, S, false>(t, h[0], sh, wv, lane);          // offsets (0, 0)
             SE_SL_FIX(0);
             se_sl_hash_load<NW, R>(g, q[AHEAD & 3], h[0]);
             se_sl_next_cycle<R>(g, q[AHEAD & 3]);
             se_sl_rows_up(t);
-            se_sl_substep<NW, R, true>(t, h[1]);           // (1, 1)
+            se_sl_substep<NW, R, S, true>(t, h[1], sh, wv, lane);           // (1, 1)
             SE_SL_FIX(1);
             se_sl_hash_load<NW, R>(g, q[(AHEAD + 1) & 3], h[1]);
             se_sl_next_cycle<R>(g, q[(AHEAD + 1) & 3]);
-            se_sl_substep<NW, R, false>(t, h[2 % AHEAD]);  // (0, 1)
+            se_sl_substep<NW, R, S, false>(t, h[2 % AHEAD], sh, wv, lane);  // (0, 1)
             SE_SL_FIX(1);
             se_sl_hash_load<NW, R>(g, q[(AHEAD + 2) & 3], h[2 % AHEAD]);
             se_sl_next_cycle<R>(g, q[(AHEAD + 2) & 3]);
             se_sl_rows_down(t);
-            se_sl_substep<NW, R, true>(t, h[3 % AHEAD]);   // (1, 0)
+            se_sl_substep<NW, R, S, true>(t, h[3 % AHEAD], sh, wv, lane);   // (1, 0)
             SE_SL_FIX(0);
             se_sl_hash_load<NW, R>(g, q[(AHEAD + 3) & 3], h[3 % AHEAD]);
             se_sl_next_cycle<R>(g, q[(AHEAD + 3) & 3]);
@@ -599,7 +663,7 @@ __device__ __forceinline__ void se_sl_load(se_sltile<NW, R>& t, const se_slgrid&
     for (int w = 0; w < NW; w++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const uint4* s = reinterpret_cast<const uint4*>(se_sl_at(g.pk[from], g, bc0 + 4 * w + q, row));
+            const uint4* s = reinterpret_cast<const uint4*>(se_sl_at(g, from, bc0 + 4 * w + q, row));
 #pragma unroll
             for (int r = 0; r < R; r += 2) {  // row is even: two rows are 16 aligned bytes
                 const uint4 v = s[r / 2];
@@ -616,7 +680,7 @@ __device__ __forceinline__ void se_sl_load(se_sltile<NW, R>& t, const se_slgrid&
         }
 }
 
-// byte columns first .. last of the tile
+// byte columns first .. last of the NW word columns
 template <int NW, int R>
 __device__ __forceinline__ void se_sl_store(const se_sltile<NW, R>& t, const se_slgrid& g, int to, int bc0, int row,
                                             int first, int last) {
@@ -628,7 +692,7 @@ __device__ __forceinline__ void se_sl_store(const se_sltile<NW, R>& t, const se_
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             if (4 * w + q < first || 4 * w + q > last) continue;
-            uint4* d = reinterpret_cast<uint4*>(se_sl_at(g.pk[to], g, bc0 + 4 * w + q, row));
+            uint4* d = reinterpret_cast<uint4*>(se_sl_at(g, to, bc0 + 4 * w + q, row));
 #pragma unroll
             for (int r = 0; r < R; r += 2)
                 d[r / 2] = make_uint4(col[r][q].x, col[r][q].y, col[r + 1][q].x, col[r + 1][q].y);
@@ -639,24 +703,96 @@ __device__ __forceinline__ void se_sl_store(const se_sltile<NW, R>& t, const se_
 // `from`: the packed grid read, the other is written.  side: byte columns given up
 // on each side (1 or 2, for up to 16 or 32 sub-steps), halo: rows; both 0: the
 // world fits the one tile, all of which is stored.
-template <int NW, int R, int AHEAD>
+template <int NW, int R, int S, int AHEAD>
 __device__ __forceinline__ void se_sl_tile(const se_slgrid& g, int from, int tx, int ty, int frame0, int nsub,
-                                           int side, int halo) {
-    const int lane = (int)(threadIdx.x & 63);
-    const int bc0 = tx * (4 * NW - 2 * side), row0 = ty * (64 * R - 2 * halo);
+                                           int side, int halo, se_slshare<R, S>& sh) {
+    const int lane = (int)(threadIdx.x & 63), wv = S > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+    const int bc0 = tx * (4 * NW * S - 2 * side) + 4 * NW * wv, row0 = ty * (64 * R - 2 * halo);
     const int row = row0 + R * lane;
     se_sltile<NW, R> t;
     se_sl_load<NW, R>(t, g, from, bc0, row);
-    se_sl_advance<NW, R, AHEAD>(t, g, 8 * bc0, row0, lane, frame0, nsub);
+    se_sl_advance<NW, R, S, AHEAD>(t, g, 8 * bc0, row0, lane, frame0, nsub, sh, wv);
     if (R * lane < halo || R * lane >= 64 * R - halo) return;
-    se_sl_store<NW, R>(t, g, from ^ 1, bc0, row, side, 4 * NW - 1 - side);
+    se_sl_store<NW, R>(t, g, from ^ 1, bc0, row, side - 4 * NW * wv, 4 * NW * S - 1 - side - 4 * NW * wv);
 }
 
-#define SE_SL_STEP(NW, R, AHEAD)                                                                              \
-    extern "C" __global__ __launch_bounds__(64, 2) void se_sl_step_##NW##x##R(                                    \
-        se_slgrid g, int from, int tiles_x, int frame0, int nsub, int side, int halo) {                        \
-        const int tile = se_xcd_tile((int)blockIdx.x, (int)gridDim.x);                                         \
-        se_sl_tile<NW, R, AHEAD>(g, from, tile % tiles_x, tile / tiles_x, frame0, nsub, side, halo);           \
+// A world and how it is cut into tiles.  In a batch (device memory, filled by the
+// host) the hash fields are those of its group: worlds that start at the same frame
+// read the same planes.
+struct se_slworld {  // == SlicedWorld (se_sliced.hpp)
+    se_slgrid g;
+    int frame0, steps, tiles_x, side, halo, group;
+    int result, pad;  // packed grid that holds the world after its last launch
+};
+
+// Steps [done, done + k) of `one` (n = 0), or of worlds [0, n) (longest first, their
+// tiles counted by prefix); one workgroup per tile.
+#define SE_SL_STEP(NW, R, S, AHEAD, WAVES, NAME)                                                                              \
+    extern "C" __global__ __launch_bounds__(64 * S, WAVES) void se_sl_step_##NAME(                                 \
+        se_slworld one, const se_slworld* __restrict__ worlds, const int* __restrict__ prefix, int n,          \
+        const se_slgrid* __restrict__ groups, int from, int done, int k) {                                     \
+        __shared__ se_slshare<R, S> sh;                                                                        \
+        se_slworld v = one;                                                                                    \
+        int tile;                                                                                              \
+        if (n == 0) {                                                                                          \
+            tile = se_xcd_tile((int)blockIdx.x, (int)gridDim.x);                                               \
+        } else {                                                                                               \
+            const int w = se_owner(prefix, n, (int)blockIdx.x);                                                \
+            tile = (int)blockIdx.x - prefix[w];                                                                \
+            v = worlds[w];                                                                                     \
+            const se_slgrid& G = groups[v.group];                                                              \
+            v.g.hash = G.hash;                                                                                 \
+            v.g.hash_frame0 = G.hash_frame0;                                                                   \
+            v.g.hash_shared = G.hash_shared;                                                                   \
+            v.g.hash_pitch = G.hash_pitch;                                                                     \
+            v.g.hash_words = G.hash_words;                                                                     \
+            v.g.hash_n0 = G.hash_n0;                                                                           \
+            v.g.hash_n1 = G.hash_n1;                                                                           \
+        }                                                                                                      \
+        se_sl_tile<NW, R, S, AHEAD>(v.g, from, tile % v.tiles_x, tile / v.tiles_x, v.frame0 + done,               \
+                                 min(k, v.steps - done), v.side, v.halo, sh);                                      \
     }
-SE_SL_STEP(2, 2, 4)
-SE_SL_STEP(4, 2, 2)
+// By two and by four wavefronts: half the instructions in a sub-step's chain, which
+// is what a world of few tiles waits for (us a call, one wavefront for 2x2: 100x90 500
+// steps 229 / 162, 1000x700 200 steps 141 / 113, twelve materials 800x800 150 steps
+// 201 / 152); the wider tile gives up a smaller share of its columns.
+SE_SL_STEP(1, 2, 2, 4, 1, 2x2s)
+SE_SL_STEP(1, 2, 4, 4, 1, 4x2s)
+// By one: no barriers, for worlds that fill the SIMDs many times over (16384^2, 100
+// steps: 1.37 ms with 4x2, 1.39 with 4x2s; 4096^2, 200 steps: 445 and 455 us).  With
+// four planes one wavefront's registers leave two or three a SIMD and the
+// split tiles are faster (8192^2, twelve materials, 64 steps: 646 us with 4x2s, 758).
+#if SE_SL_K <= 3
+SE_SL_STEP(2, 2, 1, 4, 3, 2x2)
+SE_SL_STEP(4, 2, 1, 2, 3, 4x2)
+#endif
+
+// Batch forms of the other kernels: prefix sums count 64 x 64 tiles (pack, unpack);
+// grid z over the groups (hash).
+extern "C" __global__ __launch_bounds__(256) void se_sl_bpack(const se_slworld* __restrict__ worlds,
+                                                              const int* __restrict__ prefix, int n) {
+    __shared__ u32 lds[4][64 * 17];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), t = (int)blockIdx.x * 4 + wave;
+    if (t >= prefix[n]) return;
+    const int w = se_owner(prefix, n, t), i = t - prefix[w];
+    const se_slgrid g = worlds[w].g;
+    const int cols = 1 + (g.bcols - (g.xpad >> 4) + 3) / 4;
+    se_sl_pack_tile(g, i % cols - 1, (i / cols) * 64, lds[wave]);
+}
+
+extern "C" __global__ __launch_bounds__(256) void se_sl_bunpack(const se_slworld* __restrict__ worlds,
+                                                                const int* __restrict__ prefix, int n) {
+    __shared__ u32 lds[4][64 * 17];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), t = (int)blockIdx.x * 4 + wave;
+    if (t >= prefix[n]) return;
+    const int w = se_owner(prefix, n, t), i = t - prefix[w];
+    const se_slgrid g = worlds[w].g;
+    const int cols = 1 + (g.bcols - (g.xpad >> 4) + 3) / 4;  // as packing: the first column holds no cells
+    if (i % cols > 0) se_sl_unpack_tile(g, worlds[w].result, i % cols - 1, (i / cols) * 64, lds[wave]);
+}
+
+extern "C" __global__ __launch_bounds__(256) void se_sl_bhash(const se_slgrid* __restrict__ groups) {
+    const se_slgrid g = groups[blockIdx.z];
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (i < g.hash_words && (int)blockIdx.y < g.hash_sets) se_sl_hash_word(g, i, (int)blockIdx.y);
+}

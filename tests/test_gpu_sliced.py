@@ -95,3 +95,19 @@ def test_sliced_equals_oracle(name):
     w.step_blocked(steps)
     np.testing.assert_array_equal(w.download(), O.run(blob, g, 7, steps))
     w.close()
+
+
+def test_sliced_long_run_of_a_small_world():
+    """More steps in one call than one launch hashes ahead."""
+    print("\n[gpu] sliced 40000 steps of a 20x14 world", flush=True)
+    r = rs("four_materials")
+    a, b = S.World(_ctx, r, 20, 14), S.World(_ctx, r, 20, 14)
+    for w in (a, b):
+        w.upload(grid("four_materials", 20, 14, 3))
+        w.frame = 1
+    a.step(40000)
+    b.step_blocked(40000)
+    assert a.frame == b.frame
+    np.testing.assert_array_equal(a.download(), b.download())
+    a.close()
+    b.close()
