@@ -8,6 +8,8 @@
 //     r covers every world with more than r*k steps; worlds are ordered by step
 //     count (longest first) so the active set of a round is a prefix, and one
 //     persistent launch per round strides over all of their tiles.
+// Rule sets with a sliced form run these two lists with the sliced kernels instead
+// (SlicedPlan below).
 // The single-tile launch and the rounds of every group go to their own streams
 // and overlap on the device; the whole submission can be captured in one
 // hipGraph.  The reference has no batched mode: each Simulation is one world
@@ -16,6 +18,7 @@
 #include <cstdio>
 
 #include "se_internal.hpp"
+#include "se_sliced.hpp"
 
 using se_rt::DeviceGuard;
 using se_rt::fail;
@@ -78,7 +81,12 @@ struct se_batch {
     };
     std::map<se_module*, Tuned> tuned;
     hipStream_t streams[8] = {};
+    // records, packed grids and hash planes of the sliced plans, kept from run to run
+    // and freed by se_batch_clear (a run ends with the device idle)
+    void* arena = nullptr;
+    size_t arena_bytes = 0;
     ~se_batch() {
+        (void)hipFree(arena);
         for (auto s : streams)
             if (s) (void)hipStreamDestroy(s);
     }
@@ -207,6 +215,214 @@ void finish_plan(Plan& P) {
     }
 }
 
+// ---------------------------------------------------------------- sliced plans
+// The worlds of a rule set whose list is `single` (each fits one 2x2 tile with its
+// border) or not, longest first: packed once, advanced in launches of up to k steps
+// over the worlds that have steps left, unpacked once.  Worlds that start at the
+// same frame -- all of them in the usual batch -- form a group that shares hash
+// planes, made for the group's largest extents.  They are made a chunk of frames at a
+// time on a stream of their own, while the steps of the chunk before run (which
+// leave most of the device idle when the worlds are few): two sets of planes a plan,
+// and events both ways.  A chunk's end costs some 10 us of waiting on events, and
+// nothing runs beside the first chunk's planes: chunks start at 64 frames and double.
+// Worlds inside one tile have small planes, made for the whole run where they fit.
+// Bound by vector instructions, about half of them the planes' (no two frames of small
+// worlds share a plane), at the occupancy that a few hundred tiles give.  48 worlds of
+// 64 to 1024 cells a side, two rule sets, 100 to 1000 steps each: 5.6 to 6.3 ms a run with the LDS
+// kernels, 1.9 ms so; 2.0 to 2.1 with the one-tile worlds last, or queued behind planes.
+constexpr size_t kBatchHashBudget = 256u << 20, kBatchHashMost = 1024u << 20;
+constexpr uint32_t kBatchChunk = 64, kBatchChunkMost = 256;  // frames
+
+struct SlicedPlan {
+    se_module* mod = nullptr;
+    std::vector<std::pair<se_world*, uint32_t>> list;
+    se_rt::SlicedShape shape;  // kernel, side, halo and depth of every world's tiles
+    std::vector<se_rt::SlicedWorld> recs;
+    std::vector<int> tiles, packs;                // prefix sums over the list
+    std::vector<se_rt::SlicedGrid> groups;        // [chunk][group]: hash fields
+    std::vector<int> words;                       // [chunk]: prefix sums over its groups, in 256 hash words
+    size_t n_groups = 0, hash_bytes = 0, packed_bytes = 0, meta_bytes = 0;
+    struct Launch {
+        uint32_t done, k;
+        int n, from;
+    };
+    std::vector<std::vector<Launch>> chunks;
+    char* base = nullptr;  // device: records, prefix sums, groups, packed grids, hash planes
+
+    size_t off_tiles() const { return (recs.size() * sizeof(se_rt::SlicedWorld) + 255) & ~(size_t)255; }
+    size_t off_packs() const { return off_tiles() + ((tiles.size() * sizeof(int) + 255) & ~(size_t)255); }
+    size_t off_groups() const { return off_packs() + ((packs.size() * sizeof(int) + 255) & ~(size_t)255); }
+    size_t off_words() const { return off_groups() + ((groups.size() * sizeof(se_rt::SlicedGrid) + 255) & ~(size_t)255); }
+};
+
+// Everything but the addresses.  squares: of the whole batch (sliced_choice).  False when the hash planes would take too much
+// memory (many worlds at different frames).
+bool make_sliced(SlicedPlan& P, bool single, uint32_t k, size_t squares) {
+    const se_rt::SlicedKernels& K = P.mod->sliced;
+    std::stable_sort(P.list.begin(), P.list.end(),
+                     [](const std::pair<se_world*, uint32_t>& a, const std::pair<se_world*, uint32_t>& b) {
+                         return a.second > b.second;
+                     });
+    int kernel = 0;
+    uint32_t deep = 1u << 20;
+    if (!single) {
+        se_rt::sliced_choice(squares, K, &kernel, &deep);
+        if (k) deep = std::min(k, 32u);
+    }
+    std::map<int32_t, size_t> at;  // first frame -> group
+    std::vector<se_rt::SlicedGrid> extent;  // per group: pads, largest extents
+    std::vector<uint32_t> steps;
+    std::vector<int> frame;
+    P.tiles.assign(1, 0);
+    P.packs.assign(1, 0);
+    for (auto& it : P.list) {
+        se_world* w = it.first;
+        const se_rt::SlicedShape s = single ? se_rt::sliced_one_tile(w->W, w->H, false)
+                                            : se_rt::sliced_tiles(w->W, w->H, kernel, deep);
+        P.shape = s;
+        se_rt::SlicedWorld r;
+        se_rt::sliced_geometry(s, w->W, w->H, r.g);
+        r.g.in = w->buf[w->cur];
+        r.g.out = w->buf[w->cur ^ 1];
+        r.g.pitch = (int)w->pitch;
+        r.frame0 = w->frame + 1;
+        r.steps = (int)it.second;
+        r.tiles_x = s.tiles_x;
+        r.side = s.side;
+        r.halo = s.halo;
+        auto found = at.find(r.frame0);
+        if (found == at.end()) {
+            found = at.emplace(r.frame0, extent.size()).first;
+            extent.push_back(r.g);
+            steps.push_back(0);
+            frame.push_back(r.frame0);
+        }
+        r.group = (int)found->second;
+        se_rt::SlicedGrid& e = extent[found->second];
+        e.bcols = std::max(e.bcols, r.g.bcols);
+        e.brows = std::max(e.brows, r.g.brows);
+        steps[found->second] = std::max(steps[found->second], it.second);
+        P.tiles.push_back(P.tiles.back() + s.tiles_x * s.tiles_y);
+        P.packs.push_back(P.packs.back() + se_rt::sliced_pack_tiles(r.g));
+        P.packed_bytes += 2 * se_rt::sliced_packed_bytes(r.g);
+        P.recs.push_back(r);
+    }
+    // the first launch ends at the head of a cycle where all worlds start in one phase
+    bool in_phase = true;
+    for (auto& r : P.recs) in_phase = in_phase && ((r.frame0 ^ P.recs[0].frame0) & 3) == 0;
+    const uint32_t most = P.list[0].second;
+    uint32_t first = std::min(deep, most);
+    const uint32_t lead = (uint32_t)(P.recs[0].frame0 + (int)first) & 3u;
+    if (in_phase && !single && first < most && lead < first) first -= lead;
+    // Frames hashed at a time (a chunk): all of them within the budget, else fewer, at
+    // least one launch's.  Each group's planes lie where its largest chunk has room.
+    P.n_groups = extent.size();
+    const uint32_t least = std::min(single ? 32u : deep, most);
+    for (uint32_t ahead = single ? se_rt::kSlicedMostFrames : std::max(1u, kBatchChunkMost / deep) * deep;;) {
+        uint32_t length = std::min(ahead, single ? ahead : std::max(1u, kBatchChunk / deep) * deep);
+        P.groups.clear();
+        P.words.clear();
+        P.chunks.clear();
+        std::vector<size_t> need(P.n_groups, 0), offset(P.n_groups, 0);
+        int from = 0;
+        for (uint32_t done = 0; done < most;) {
+            const uint32_t stop = std::min(most, done + length);
+            length = std::min(ahead, 2 * length);
+            P.words.push_back(0);
+            for (size_t i = 0; i < P.n_groups; i++) {
+                se_rt::SlicedGrid g = extent[i];
+                if (done < steps[i])
+                    need[i] = std::max(need[i], se_rt::sliced_hash_layout(g, frame[i] + (int)done,
+                                                                          std::min(stop, steps[i]) - done, K.classes));
+                P.groups.push_back(g);
+                P.words.push_back(P.words.back() + (int)(((size_t)g.hash_words * g.hash_sets + 255) / 256));
+            }
+            P.chunks.emplace_back();
+            while (done < stop) {
+                const uint32_t m = std::min(done == 0 ? first : deep, stop - done);
+                int n = 0;
+                while (n < (int)P.recs.size() && P.recs[n].steps > (int)done) P.recs[n++].result ^= 1;
+                P.chunks.back().push_back({done, m, n, from});
+                from ^= 1;
+                done += m;
+            }
+        }
+        size_t set = 0;
+        for (size_t i = 0; i < P.n_groups; i++) {
+            offset[i] = set;
+            set += (need[i] + 255) & ~(size_t)255;
+        }
+        P.hash_bytes = P.chunks.size() > 1 ? 2 * set : set;
+        for (size_t j = 0; j < P.groups.size(); j++)  // offsets until the arena is known
+            P.groups[j].hash = (uint32_t*)(offset[j % P.n_groups] + (j / P.n_groups & 1) * set);
+        if (P.hash_bytes <= (single ? kBatchHashBudget / 4 : kBatchHashBudget) || ahead <= least) break;
+        ahead = std::max(least, ahead / 2);
+        if (!single) ahead = std::max(1u, ahead / deep) * deep;
+        for (auto& r : P.recs) r.result = 0;
+    }
+    P.meta_bytes = P.off_words() + ((P.words.size() * sizeof(int) + 255) & ~(size_t)255);
+    return P.hash_bytes <= kBatchHashMost;
+}
+
+// Device addresses from `base` on, and the records there.
+int place_sliced(SlicedPlan& P, char* base) {
+    P.base = base;
+    char* p = base + P.meta_bytes;
+    for (auto& r : P.recs) {
+        const size_t bytes = se_rt::sliced_packed_bytes(r.g);
+        r.g.pk0 = p;
+        r.g.pk1 = p + bytes;
+        p += 2 * bytes;
+    }
+    for (auto& g : P.groups) g.hash = (uint32_t*)(p + (size_t)g.hash);
+    std::vector<char> meta(P.meta_bytes);
+    std::memcpy(meta.data(), P.recs.data(), P.recs.size() * sizeof(P.recs[0]));
+    std::memcpy(meta.data() + P.off_tiles(), P.tiles.data(), P.tiles.size() * sizeof(int));
+    std::memcpy(meta.data() + P.off_packs(), P.packs.data(), P.packs.size() * sizeof(int));
+    std::memcpy(meta.data() + P.off_groups(), P.groups.data(), P.groups.size() * sizeof(P.groups[0]));
+    std::memcpy(meta.data() + P.off_words(), P.words.data(), P.words.size() * sizeof(int));
+    HIPCHECK(hipMemcpy(base, meta.data(), meta.size(), hipMemcpyHostToDevice));
+    return SE_OK;
+}
+
+int sliced_pack(SlicedPlan& P, hipStream_t s) {
+    return launch_ex(P.mod->sliced.bpack, (unsigned)(P.packs.back() + 3) / 4, 256, 0u, s, (const void*)P.base,
+                     (const int*)(P.base + P.off_packs()), (int)P.recs.size());
+}
+int sliced_unpack(SlicedPlan& P, hipStream_t s) {
+    return launch_ex(P.mod->sliced.bunpack, (unsigned)(P.packs.back() + 3) / 4, 256, 0u, s, (const void*)P.base,
+                     (const int*)(P.base + P.off_packs()), (int)P.recs.size());
+}
+
+// Chunk c: its planes on hs, then its steps on s.  events: two per chunk, planes made
+// and steps done.
+int sliced_chunk(SlicedPlan& P, size_t c, hipStream_t s, hipStream_t hs, const std::vector<hipEvent_t>& events) {
+    const se_rt::SlicedGrid* g = (const se_rt::SlicedGrid*)(P.base + P.off_groups()) + c * P.n_groups;
+    const size_t row = c * (P.n_groups + 1);
+    if (c >= 2) HIPCHECK(hipStreamWaitEvent(hs, events[2 * (c - 2) + 1], 0));  // the set's planes have been read
+    int rc = launch_ex(P.mod->sliced.bhash, (unsigned)P.words[row + P.n_groups], 256, 0u, hs, (const void*)g,
+                       (const int*)(P.base + P.off_words()) + row, (int)P.n_groups);
+    if (rc) return rc;
+    HIPCHECK(hipEventRecord(events[2 * c], hs));
+    HIPCHECK(hipStreamWaitEvent(s, events[2 * c], 0));
+    for (auto& l : P.chunks[c]) {
+        rc = launch_ex(P.mod->sliced.step[P.shape.kernel], (unsigned)P.tiles[l.n], P.shape.threads, 0u, s,
+                       se_rt::SlicedWorld(), (const void*)P.base, (const int*)(P.base + P.off_tiles()), l.n,
+                       (const void*)g, l.from, (int)l.done, (int)l.k);
+        if (rc) return rc;
+    }
+    HIPCHECK(hipEventRecord(events[2 * c + 1], s));
+    return SE_OK;
+}
+
+void finish_sliced(SlicedPlan& P) {
+    for (auto& it : P.list) {
+        se_rt::sleep_reset(it.first);
+        it.first->frame += (int32_t)it.second;
+        it.first->cur ^= 1;
+    }
+}
+
 int ensure_streams(se_batch* b, int n) {
     for (int i = 0; i < n && i < 8; i++)
         if (!b->streams[i]) HIPCHECK(hipStreamCreateWithFlags(&b->streams[i], hipStreamNonBlocking));
@@ -222,39 +438,118 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
     std::map<se_module*, std::vector<std::pair<se_world*, uint32_t>>> groups;
     for (auto& it : work) groups[it.first->mod.get()].push_back(it);
     std::vector<std::unique_ptr<Plan>> plans;
+    std::vector<std::unique_ptr<SlicedPlan>> sliced;
+    size_t squares = 0;  // of the whole batch: its lists run side by side
+    for (auto& it : work)
+        if (it.second) squares += se_rt::sliced_squares(it.first->W, it.first->H);
     for (auto& g : groups) {
         se_module* mod = g.first;
         int vi = variant;
         uint32_t kk = k;
         int la = launch;
         auto t = b->tuned.find(mod);
+        bool chosen = vi >= 0;
         if (vi < 0) {
             if (t != b->tuned.end()) {
                 vi = t->second.vi;
+                chosen = true;
                 if (kk == 0) kk = t->second.k;
             } else {
                 vi = se_rt::default_lds_index(mod);
             }
         }
         if (la < 0) la = t != b->tuned.end() ? (int)t->second.persistent : 0;
-        if (vi < 0 || vi >= (int)mod->lds.size() || mod->lds[vi].first.sliced) return fail(SE_ERR_ARG, "LDS variant out of range");
+        if (vi < 0 || vi >= (int)mod->lds.size()) return fail(SE_ERR_ARG, "LDS variant out of range");
+        uint32_t most = 0;
+        for (auto& it : g.second) most = std::max(most, it.second);
+        const bool want = mod->lds[vi].first.sliced || (!chosen && la != 1 && se_rt::sliced_pays(mod, most));
+        if (want && most > 0) {
+            std::unique_ptr<SlicedPlan> one(new SlicedPlan()), many(new SlicedPlan());
+            one->mod = many->mod = mod;
+            for (auto& it : g.second)
+                if (it.second)
+                    (se_rt::sliced_one_tile(it.first->W, it.first->H, false).nw ? one : many)->list.push_back(it);
+            if ((one->list.empty() || make_sliced(*one, true, kk, squares)) && (many->list.empty() || make_sliced(*many, false, kk, squares))) {
+                if (!many->list.empty()) sliced.push_back(std::move(many));
+                if (!one->list.empty()) sliced.push_back(std::move(one));
+                continue;
+            }
+        }
+        if (mod->lds[vi].first.sliced) vi = se_rt::default_lds_index(mod);
         plans.emplace_back(new Plan());
         plans.back()->persistent = la == 1;
         int rc = make_plan(ctx, mod, vi, kk, g.second, *plans.back());
         if (rc) return rc;
     }
-    int rc = ensure_streams(b, 2 * (int)plans.size());
+    if (!sliced.empty()) {
+        size_t bytes = 0;
+        for (auto& p : sliced) bytes += p->meta_bytes + p->packed_bytes + p->hash_bytes;
+        if (bytes > b->arena_bytes) {
+            bytes += bytes / 8;  // worlds that drift apart in frames take a little more each run
+            if (b->arena) HIPCHECK(hipFree(b->arena));
+            b->arena = nullptr;
+            b->arena_bytes = 0;
+            if (hipMalloc(&b->arena, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                b->arena = nullptr;
+            } else {
+                b->arena_bytes = bytes;
+            }
+        }
+        if (b->arena) {
+            char* p = (char*)b->arena;
+            for (auto& q : sliced) {
+                int rc = place_sliced(*q, p);
+                if (rc) return rc;
+                p += q->meta_bytes + q->packed_bytes + q->hash_bytes;
+            }
+        } else {  // no memory for them: the LDS kernels
+            std::map<se_module*, std::vector<std::pair<se_world*, uint32_t>>> back;
+            for (auto& q : sliced) back[q->mod].insert(back[q->mod].end(), q->list.begin(), q->list.end());
+            sliced.clear();
+            for (auto& g : back) {
+                plans.emplace_back(new Plan());
+                int rc = make_plan(ctx, g.first, se_rt::default_lds_index(g.first), 0, g.second, *plans.back());
+                if (rc) return rc;
+            }
+        }
+    }
+    // Sliced plans: worlds beyond one tile on a stream per plan, two at most, the longest
+    // chain first; their hash planes on the context's stream, idle until the joins; and all
+    // worlds inside one tile, a few long launches with planes of their own, on a third
+    // stream ahead of everything.
+    std::vector<int> lane(sliced.size());
+    {
+        auto chain = [](const SlicedPlan& p) { return (double)p.list[0].second * p.mod->sliced.planes; };
+        std::stable_sort(sliced.begin(), sliced.end(),
+                         [&](const std::unique_ptr<SlicedPlan>& x, const std::unique_ptr<SlicedPlan>& y) {
+                             return chain(*x) > chain(*y);
+                         });
+        double sum[2] = {0, 0};
+        for (size_t i = 0; i < sliced.size(); i++) {
+            lane[i] = !sliced[i]->shape.halo ? 2 : sum[0] <= sum[1] ? 0 : 1;
+            if (lane[i] < 2) sum[lane[i]] += chain(*sliced[i]);
+        }
+    }
+    const size_t n_streams = 2 * plans.size() + (sliced.empty() ? 0 : 3);
+    int rc = ensure_streams(b, (int)n_streams);
     if (rc) return rc;
     RunResources res;  // declared after `plans`: destroyed (and the stream drained) first
     res.streams.assign(b->streams, b->streams + 8);
     res.streams.push_back(ctx->stream);
     hipEvent_t e0, e1, fork;
-    std::vector<hipEvent_t> joins(2 * plans.size());
+    std::vector<hipEvent_t> joins(n_streams);
     rc = res.event(&e0, hipEventDefault);
     if (!rc) rc = res.event(&e1, hipEventDefault);
     if (!rc) rc = res.event(&fork, hipEventDisableTiming);
     for (auto& j : joins)
         if (!rc) rc = res.event(&j, hipEventDisableTiming);
+    std::vector<std::vector<hipEvent_t>> chunk_events(sliced.size());
+    for (size_t i = 0; i < sliced.size(); i++) {
+        chunk_events[i].resize(2 * sliced[i]->chunks.size());
+        for (auto& e : chunk_events[i])
+            if (!rc) rc = res.event(&e, hipEventDisableTiming);
+    }
     if (rc) return rc;
     auto submit = [&]() -> int {
         HIPCHECK(hipEventRecord(fork, ctx->stream));
@@ -267,9 +562,53 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
             HIPCHECK(hipEventRecord(joins[2 * i], sa));
             HIPCHECK(hipEventRecord(joins[2 * i + 1], sb));
         }
+        if (!sliced.empty()) {
+            hipStream_t st[3];
+            for (int i = 0; i < 3; i++) {
+                st[i] = b->streams[(2 * plans.size() + i) % 8];
+                HIPCHECK(hipStreamWaitEvent(st[i], fork, 0));
+            }
+            for (size_t i = 0; i < sliced.size(); i++) {
+                if (lane[i] < 2) continue;
+                int r2 = sliced_pack(*sliced[i], st[2]);
+                for (size_t c = 0; !r2 && c < sliced[i]->chunks.size(); c++)
+                    r2 = sliced_chunk(*sliced[i], c, st[2], st[2], chunk_events[i]);
+                if (!r2) r2 = sliced_unpack(*sliced[i], st[2]);
+                if (r2) return r2;
+            }
+            // the others two at a time, chunk by chunk
+            for (size_t next[2] = {0, 0};;) {
+                int at[2] = {-1, -1};
+                size_t chunks = 0;
+                for (int l = 0; l < 2; l++) {
+                    while (next[l] < sliced.size() && lane[next[l]] != l) next[l]++;
+                    if (next[l] == sliced.size()) continue;
+                    at[l] = (int)next[l]++;
+                    int r2 = sliced_pack(*sliced[at[l]], st[l]);
+                    if (r2) return r2;
+                    chunks = std::max(chunks, sliced[at[l]]->chunks.size());
+                }
+                if (at[0] < 0 && at[1] < 0) break;
+                for (size_t c = 0; c < chunks; c++)
+                    for (int l = 0; l < 2; l++) {
+                        if (at[l] < 0 || c >= sliced[at[l]]->chunks.size()) continue;
+                        int r2 = sliced_chunk(*sliced[at[l]], c, st[l], ctx->stream, chunk_events[at[l]]);
+                        if (r2) return r2;
+                    }
+                for (int l = 0; l < 2; l++) {
+                    int r2 = at[l] < 0 ? SE_OK : sliced_unpack(*sliced[at[l]], st[l]);
+                    if (r2) return r2;
+                }
+            }
+            for (int i = 0; i < 3; i++) HIPCHECK(hipEventRecord(joins[2 * plans.size() + i], st[i]));
+        }
         for (auto& j : joins) HIPCHECK(hipStreamWaitEvent(ctx->stream, j, 0));
         return SE_OK;
     };
+    // Sliced plans are submitted directly: they make some forty launches where the
+    // rounds of the LDS kernels make hundreds, and capturing them has ended in heap
+    // corruption inside one of the HIP runtimes that programs load.
+    if (!sliced.empty()) graph = 0;
     if (graph) {
         HIPCHECK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
         int r2 = submit();
@@ -290,6 +629,7 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
     float ms = 0;
     HIPCHECK(hipEventElapsedTime(&ms, e0, e1));
     for (auto& p : plans) finish_plan(*p);
+    for (auto& p : sliced) finish_sliced(*p);
     if (gpu_ms) *gpu_ms = ms;
     return SE_OK;
 }
@@ -341,6 +681,10 @@ int se_batch_add(se_batch* b, se_world* w, uint32_t nsteps) {
 int se_batch_clear(se_batch* b) {
     if (!b) return fail(SE_ERR_ARG, "null batch");
     b->items.clear();
+    DeviceGuard dg(b->ctx->device);
+    (void)hipFree(b->arena);
+    b->arena = nullptr;
+    b->arena_bytes = 0;
     return SE_OK;
 }
 
@@ -425,10 +769,9 @@ int se_batch_autotune(se_batch* b, uint32_t rounds, int32_t* best_variant, uint3
         uint32_t bk = 0;
         bool bp = false;
         for (int vi = 0; vi < (int)mod->lds.size(); vi++) {
-            if (mod->lds[vi].first.sliced) continue;  // single worlds only
             const int hb = mod->lds[vi].first.hb;
             for (uint32_t kk : {(uint32_t)hb, (uint32_t)std::max(2, hb / 2)})
-            for (int la = 0; la < 2; la++) {
+            for (int la = 0; la < (mod->lds[vi].first.sliced ? 1 : 2); la++) {
                 std::vector<std::pair<se_world*, uint32_t>> trial;
                 double cells = 0;
                 for (auto& it : g.second) {

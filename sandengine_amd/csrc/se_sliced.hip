@@ -732,6 +732,7 @@ struct se_slworld {  // == SlicedWorld (se_sliced.hpp)
         se_slworld one, const se_slworld* __restrict__ worlds, const int* __restrict__ prefix, int n,          \
         const se_slgrid* __restrict__ groups, int from, int done, int k) {                                     \
         __shared__ se_slshare<R, S> sh;                                                                        \
+        if (S > 1) __builtin_amdgcn_s_setprio(3); /* a chain of steps beside the planes of a later chunk */    \
         se_slworld v = one;                                                                                    \
         int tile;                                                                                              \
         if (n == 0) {                                                                                          \
@@ -767,8 +768,7 @@ SE_SL_STEP(2, 2, 1, 4, 3, 2x2)
 SE_SL_STEP(4, 2, 1, 2, 3, 4x2)
 #endif
 
-// Batch forms of the other kernels: prefix sums count 64 x 64 tiles (pack, unpack);
-// grid z over the groups (hash).
+// Batch forms of the other kernels: prefix sums count 64 x 64 tiles (pack, unpack).
 extern "C" __global__ __launch_bounds__(256) void se_sl_bpack(const se_slworld* __restrict__ worlds,
                                                               const int* __restrict__ prefix, int n) {
     __shared__ u32 lds[4][64 * 17];
@@ -791,8 +791,13 @@ extern "C" __global__ __launch_bounds__(256) void se_sl_bunpack(const se_slworld
     if (i % cols > 0) se_sl_unpack_tile(g, worlds[w].result, i % cols - 1, (i / cols) * 64, lds[wave]);
 }
 
-extern "C" __global__ __launch_bounds__(256) void se_sl_bhash(const se_slgrid* __restrict__ groups) {
-    const se_slgrid g = groups[blockIdx.z];
-    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
-    if (i < g.hash_words && (int)blockIdx.y < g.hash_sets) se_sl_hash_word(g, i, (int)blockIdx.y);
+// The words of all groups in one row of workgroups (prefix counts 256 of them): a grid
+// over the largest group's extents would be mostly empty workgroups (25 groups of a
+// 48-world batch: 103 us a launch, and the work in it some 15).
+extern "C" __global__ __launch_bounds__(256) void se_sl_bhash(const se_slgrid* __restrict__ groups,
+                                                              const int* __restrict__ prefix, int n) {
+    const int w = se_owner(prefix, n, (int)blockIdx.x);
+    const se_slgrid g = groups[w];
+    const u32 t = (u32)((int)blockIdx.x - prefix[w]) * 256u + threadIdx.x, set = t / (u32)g.hash_words;
+    if (set < (u32)g.hash_sets) se_sl_hash_word(g, (int)(t - set * (u32)g.hash_words), (int)set);
 }

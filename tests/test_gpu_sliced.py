@@ -97,6 +97,34 @@ def test_sliced_equals_oracle(name):
     w.close()
 
 
+@pytest.mark.parametrize("graph", [False, True], ids=["streams", "graph"])
+@pytest.mark.parametrize("k", [0, 5, 16])
+def test_sliced_batch_equals_per_world_plain(graph, k):
+    """A batch of both rule-set forms: worlds inside one tile and beyond it, with
+    equal and with different first frames and step counts, one of them 0."""
+    print(f"\n[gpu] sliced batch graph={graph} k={k}", flush=True)
+    b, pairs = S.Batch(rs("four_materials").ctx), []
+    for i, (W, H) in enumerate([(64, 64), (123, 126), (124, 126), (1, 300), (300, 1), (389, 211), (640, 193), (17, 90)]):
+        for name, first, steps in (("four_materials", 2, 40 + 13 * i), ("twelve_materials", 2 + i % 3, 9 + 31 * (i % 4)),
+                                   ("features", 2147483000 if i == 5 else 7, 60 if i else 0)):
+            x, y = S.World(_ctx, rs(name), W, H), S.World(_ctx, rs(name), W, H)
+            for w in (x, y):
+                w.upload(grid(name, W, H, 20 + i))
+                w.frame = first
+            pairs.append((x, y, steps))
+            b.add(x, steps)
+    for _ in range(2):
+        b.run(mode=1, k=k, graph=graph)
+        for x, y, steps in pairs:
+            y.step(steps)
+            assert x.frame == y.frame
+            np.testing.assert_array_equal(x.download(), y.download(), err_msg=f"{x.W}x{x.H} {x.rules.nmat} {steps}")
+    b.close()
+    for x, y, _ in pairs:
+        x.close()
+        y.close()
+
+
 def test_sliced_long_run_of_a_small_world():
     """More steps in one call than one launch hashes ahead."""
     print("\n[gpu] sliced 40000 steps of a 20x14 world", flush=True)
