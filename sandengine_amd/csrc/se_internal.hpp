@@ -86,7 +86,7 @@ struct se_module {
     std::vector<int> lds_waves;      // resident wavefronts per CU per LDS variant
     int default_lds = 0;             // LDS variant of se_world_step_blocked when none is set
     hipFunction_t plain = nullptr, fill = nullptr, fill_seeded = nullptr, copy = nullptr, fill_spec = nullptr;
-    hipFunction_t render = nullptr;  // se_render: colour and light side-outputs of a step
+    hipFunction_t render[3] = {};  // se_render_r1/2/4: colour and light side-outputs of a step
     hipFunction_t noise_fill = nullptr;  // se_noise_fill: the colour noise image
     hipFunction_t plain_v[6] = {};  // se_step_plain_r{1,2,4}_nt{0,1}
     std::vector<std::pair<se::LdsVariant, hipFunction_t>> lds;

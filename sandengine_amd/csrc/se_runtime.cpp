@@ -335,7 +335,8 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
     HIPCHECK(hipModuleGetFunction(&m->fill_seeded, m->mod, "se_fill_seeded"));
     HIPCHECK(hipModuleGetFunction(&m->copy, m->mod, "se_copy"));
     HIPCHECK(hipModuleGetFunction(&m->fill_spec, m->mod, "se_fill_spec"));
-    HIPCHECK(hipModuleGetFunction(&m->render, m->mod, "se_render"));
+    for (int i = 0; i < 3; i++)
+        HIPCHECK(hipModuleGetFunction(&m->render[i], m->mod, ("se_render_r" + std::to_string(1 << i)).c_str()));
     HIPCHECK(hipModuleGetFunction(&m->noise_fill, m->mod, "se_noise_fill"));
     int max_lds = 65536;
     hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device);
@@ -480,14 +481,19 @@ int launch_fill(se_world* w, uint32_t* g, uint32_t v) {
 }
 
 // Colour and light of the step that turned `prev` into `cur` (render enabled).
-constexpr int kRenderRows = 8;  // rows per wavefront of se_render (SE_RENDER_ROWS)
-
 int render_step(se_world* w, const uint32_t* prev, const uint32_t* cur) {
     if (!w->color) return SE_OK;
-    dim3 grid((w->W + 255) / 256, (w->H + kRenderRows - 1) / kRenderRows);
+    // Rows a wavefront.  One until there are two wavefronts per SIMD (512x256: 9.1 us a frame
+    // against 9.5 with two; 512x512 11.6 against 10.3), then two, so that half as many rows are
+    // read twice, and four once the outputs outgrow the caches (2048x1024: 33.1 against 32.8 with
+    // two; 2560x1440 51.4 against 53.0; 3840x2160 103 against 106).
+    const uint64_t waves = (uint64_t)((w->W + 63) / 64) * w->H;
+    const int v = waves <= 2048 ? 0 : waves <= 32768 ? 1 : 2;
+    const uint32_t rows = 1u << v;
+    const uint32_t groups = (w->W + 255) / 256 * ((w->H + rows - 1) / rows);
     void* args[] = {(void*)&prev, (void*)&cur, &w->light[w->lcur], &w->light[w->lcur ^ 1], &w->color,
                     (void*)&w->noise, (void*)&w->W, (void*)&w->H, (void*)&w->pitch};
-    HIPCHECK(hipModuleLaunchKernel(w->mod->render, grid.x, grid.y, 1, 256, 1, 1, 0, w->stream, args, nullptr));
+    HIPCHECK(hipModuleLaunchKernel(w->mod->render[v], groups, 1, 1, 256, 1, 1, 0, w->stream, args, nullptr));
     w->lcur ^= 1;
     return SE_OK;
 }
