@@ -41,7 +41,8 @@ __device__ __forceinline__ bool se_sqrt_le(float s, float R) {
 // Modification override for cell (x, y): returns the id or -1
 // (falling_sand.glsl:134-179: last matching entry wins, a NULL material hides
 // earlier matches, the list was cut at the first size-0 entry by the host).
-__device__ __forceinline__ int se_mod_override(const se_mod* __restrict__ mods, int nmods, int x, int y) {
+template <class Mods>
+__device__ __forceinline__ int se_mod_override(Mods mods, int nmods, int x, int y) {
     int fin = -1;
     for (int i = 0; i < nmods; i++) {
         const int mx = mods[i].x, my = mods[i].y, sz = mods[i].size, sh = mods[i].shape;
@@ -67,8 +68,8 @@ __device__ __forceinline__ int se_mod_override(const se_mod* __restrict__ mods, 
 }
 
 // Does any modification's bounding box touch rows [ya, yb] x columns [xa, xb]?
-__device__ __forceinline__ bool se_mods_touch(const se_mod* __restrict__ mods, int nmods, int xa, int xb, int ya,
-                                              int yb) {
+template <class Mods>
+__device__ __forceinline__ bool se_mods_touch(Mods mods, int nmods, int xa, int xb, int ya, int yb) {
     for (int i = 0; i < nmods; i++) {
         const long r = mods[i].size < 0 ? 0 : mods[i].size;
         const long mx = mods[i].x, my = mods[i].y;
@@ -112,8 +113,8 @@ __device__ __forceinline__ uint4 se_load_quad(const u32* __restrict__ row, int x
     return q;
 }
 
-__device__ __forceinline__ void se_apply_mods_quad(uint4& q, const se_mod* __restrict__ mods, int nmods, int x0,
-                                                   int y) {
+template <class Mods>
+__device__ __forceinline__ void se_apply_mods_quad(uint4& q, Mods mods, int nmods, int x0, int y) {
     int o;
     if ((o = se_mod_override(mods, nmods, x0, y)) >= 0) q.x = (u32)o;
     if ((o = se_mod_override(mods, nmods, x0 + 1, y)) >= 0) q.y = (u32)o;
@@ -132,6 +133,24 @@ __device__ __forceinline__ void se_store_quad(u32* p, const uint4& q) {
     }
 }
 
+// Up to SE_PLAIN_MODS modifications, more than a frame of brushes queues, travel in the
+// plain kernel's arguments.  Copied ahead of the step they cost a launch of the copy's own
+// kernel and the host's way to it: a frame with one brush 8.6 us and now 5.6 at 256x256, 15.6
+// and 13.2 at 3001x2003.  Longer lists come in `mods`, copied as before.
+#define SE_PLAIN_MODS 8
+struct se_few {
+    se_mod m[SE_PLAIN_MODS];
+};
+struct se_plain_args {  // the arguments as they lie in the kernel's argument segment
+    const u32* in;
+    u32* out;
+    int W, H, pitch, frame, offx, offy, strips, brows;
+    const se_mod* mods;
+    int nmods;
+    se_few few;
+};
+typedef const __attribute__((address_space(4))) se_mod* se_cmods;  // read by scalar loads
+
 typedef float se_f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void se_store_f4(float4* p, const float4& v) {
@@ -144,7 +163,7 @@ __device__ __forceinline__ void se_store_f4(float4* p, const float4& v) {
 template <int R, bool NT>
 __device__ __forceinline__ void se_plain_body(const u32* __restrict__ in, u32* __restrict__ out, int W, int H,
                                               int pitch, int frame, int offx, int offy, int strips, int brows,
-                                              const se_mod* __restrict__ mods, int nmods) {
+                                              se_cmods mods, int nmods) {
     const int lane = threadIdx.x & 63;
     const int wave = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
     const int strip = wave % strips;
@@ -239,11 +258,18 @@ __device__ __forceinline__ void se_plain_body(const u32* __restrict__ in, u32* _
     }
 }
 
+// A list in the arguments is read where it lies, in the constant address space like a
+// list in memory (nothing writes either while the kernel runs): an index into the
+// by-value `few` would copy it to scratch.
 #define SE_PLAIN_KERNEL(R, NT)                                                                                   \
     extern "C" __global__ __launch_bounds__(256) void se_step_plain_r##R##_nt##NT(                              \
         const u32* __restrict__ in, u32* __restrict__ out, int W, int H, int pitch, int frame, int offx,       \
-        int offy, int strips, int brows, const se_mod* __restrict__ mods, int nmods) {                         \
-        se_plain_body<R, NT != 0>(in, out, W, H, pitch, frame, offx, offy, strips, brows, mods, nmods);         \
+        int offy, int strips, int brows, const se_mod* __restrict__ mods, int nmods, se_few) {                 \
+        const se_cmods few = (se_cmods)((const __attribute__((address_space(4))) char*)                        \
+                                            __builtin_amdgcn_kernarg_segment_ptr() +                           \
+                                        __builtin_offsetof(se_plain_args, few));                               \
+        se_plain_body<R, NT != 0>(in, out, W, H, pitch, frame, offx, offy, strips, brows,                       \
+                                  nmods <= SE_PLAIN_MODS ? few : (se_cmods)mods, nmods);                        \
     }
 SE_PLAIN_KERNEL(1, 0)
 SE_PLAIN_KERNEL(2, 0)

@@ -460,13 +460,21 @@ struct ModsArg {
 
 // Uploads the queued modifications (cut at the first size-0 entry, as the
 // kernel's loop stops there, falling_sand.glsl:139-141) and clears the queue.
-int take_mods(se_world* w, ModsArg& m) {
+// Up to kFewMods of them go to `few` instead, where the kernel takes them by value.
+constexpr int kFewMods = 8;  // SE_PLAIN_MODS of the kernel source
+struct FewMods {
+    se_modification m[kFewMods];
+};
+
+int take_mods(se_world* w, ModsArg& m, FewMods* few = nullptr) {
     m.ptr = w->d_mods;
     m.n = 0;
     if (w->pending.empty()) return SE_OK;
     int n = 0;
     while (n < (int)w->pending.size() && n < SE_MAX_MODIFICATIONS && w->pending[n].mod_size != 0) n++;
-    if (n > 0)
+    if (few && n <= kFewMods)
+        std::memcpy(few->m, w->pending.data(), sizeof(se_modification) * n);
+    else if (n > 0)
         HIPCHECK(hipMemcpyAsync(w->d_mods, w->pending.data(), sizeof(se_modification) * n, hipMemcpyHostToDevice,
                                 w->stream));
     w->pending.clear();
@@ -515,7 +523,8 @@ int se_rt::plain_step(se_world* w) {
         return SE_OK;
     }
     ModsArg m;
-    int rc = take_mods(w, m);
+    FewMods few{};
+    int rc = take_mods(w, m, &few);
     if (rc) return rc;
     int ox, oy;
     offset_of(w->frame, ox, oy);
@@ -527,7 +536,7 @@ int se_rt::plain_step(se_world* w) {
     unsigned blocks = (unsigned)((waves + 3) / 4);
     int rc2 = launch(w->mod->plain_v[w->plain_variant], blocks, w->stream, (const uint32_t*)in, out, (int)w->W,
                      (int)w->H,
-                     (int)w->pitch, (int)w->frame, ox, oy, strips, brows, (const void*)m.ptr, m.n);
+                     (int)w->pitch, (int)w->frame, ox, oy, strips, brows, (const void*)m.ptr, m.n, few);
     if (!rc2) rc2 = render_step(w, in, out);
     if (rc2) return rc2;
     w->cur ^= 1;
