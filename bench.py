@@ -5,12 +5,14 @@ four-material rule set, seed 1, bottom 30% of rows stone and the rest i.i.d.
 60% EMPTY / 25% sand / 15% water; --steps timed steps after --warmup untimed
 ones.  Both step paths run from the same initial grid:
   plain   : one HBM pass per step (se_step_plain)
-  blocked : LDS temporal blocking, several sub-steps per launch (se_step_lds_*)
+  blocked : several sub-steps per launch: the sliced kernels (se_sl_step_*: bit planes,
+            32 blocks to a word) from 9 steps on, else LDS temporal blocking (se_step_lds_*)
 and their final grids must be identical (checked after the timed region).
 
 Prints ONE JSON line: value = whole-job Gcell-updates/s of the faster path,
 roofline of that path's kernel (algorithmic bytes: 8 B per cell per launch --
-one u32 read and one u32 write), per-step latency p50/p99 for both paths, and
+one u32 read and one u32 write -- and 1 B for the sliced kernels' packed cells),
+per-step latency p50/p99 for both paths, and
 the CPU baseline (the reference's GLSL program under Mesa llvmpipe on a bounded
 sample, or the oracle's C restatement where the llvmpipe build is absent).
 """
@@ -34,6 +36,9 @@ WORKLOADS = {
     "single256": (256, "four_materials", 0, [0, 3, 4, 5], [50, 25, 15, 10], (0, 1), 0),
     "rich8k": (8192, "twelve_materials", 2, [0] + list(range(3, 15)), [40] + [5] * 12, (0, 1), 0),
 }
+# Step kernel and deepest launch of the sliced form, by the world's size and planes
+SLICED = {"single16k": ("se_sl_step_4x2", 12), "rich8k": ("se_sl_step_4x2s", 16), "single256": ("se_sl_step_2x2s", 32)}
+SLICED_PAYS = 9  # steps from which the default choice is the sliced kernels
 BATCH = {
     # name: (n worlds, side range, step range, seed)
     "batch4096": (4096, (64, 1024), (100, 1000), 3),
@@ -180,8 +185,8 @@ def run_serve(args):
 
 
 def run_batch(args):
-    """Batched multi-world workload: autotuned batched LDS kernel (one hipGraph)
-    against looping the plain kernel world by world, from identical grids."""
+    """Batched multi-world workload: the batch as autotuned (sliced kernels, or LDS kernels in
+    one hipGraph) against looping the plain kernel world by world, from identical grids."""
     import sandengine_amd as S
     ctx = S.Context(0)
     rsets = {k: S.RuleSet(ctx, S.bundled_ruleset(k)) for k in BATCH_FILLS}
@@ -251,7 +256,7 @@ def run_batch(args):
         "n_gpus": 1, "steps": int(sum(s[2] for s in specs)), "warmup": 0,
         "ms_per_step": None, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "u32", "data": "synthetic (seeded SplitMix64 fills generated on the device)",
-        "config": {"workload": DESCR[args.workload], "path": "batched LDS kernel, autotuned, one hipGraph",
+        "config": {"workload": DESCR[args.workload], "path": "batched sliced kernels or LDS kernels as autotuned",
                    "tuned_variant": tuned_by_rules},
         "batched": {"gpu_ms": ms_batch, "wall_s": wall_batch, "gcups_gpu": cells / (ms_batch / 1e3) / 1e9,
                     "gcups_wall": cells / wall_batch / 1e9, "autotune_s": tune_s},
@@ -309,7 +314,7 @@ def run_render(args):
         wp.close()
         log(f"grid with render outputs == grid without: {identical}")
     w.close()
-    kernel = "se_render"
+    kernel = "se_render_r4"
     prof = load_profile(kernel, args.workload)
     achieved = RENDER_BYTES_PER_CELL * cells / (render_ms / 1e3) / 1e9
     cpu = None if args.no_cpu_baseline else cpu_baseline(
@@ -358,6 +363,18 @@ def time_path(S, w, mode, steps, warmup, sub):
     gpu_ms = w.step_timed(steps, 0 if mode == "plain" else 1, sub)
     wall = time.perf_counter() - t0
     return wall, gpu_ms
+
+
+def sliced_variant(S, w):
+    """Index that names the sliced kernels (the last LDS index, without LDS), or None."""
+    last, found = 0, None
+    while True:
+        try:
+            if w.variant_info(3, last)[1] == 0:
+                found = last
+        except S.SandengineError:
+            return found
+        last += 1
 
 
 def latencies(w, mode, sub, n):
@@ -511,7 +528,7 @@ def main():
     ap.add_argument("--plain-drain", type=float, default=5.0)
     ap.add_argument("--verify", type=int, default=0, help="serve: replay every n-th request alone (0: none)")
     ap.add_argument("--budget-gb", type=float, default=200.0)
-    ap.add_argument("--sub", type=int, default=8, help="sub-steps per LDS launch")
+    ap.add_argument("--sub", type=int, default=8, help="sub-steps per launch of the blocked path")
     ap.add_argument("--paths", default="plain,blocked,blocked_dense,blocked_tuned")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-check", action="store_true")
@@ -548,7 +565,7 @@ def main():
     log(f"copy reference: {copy_ms:.3f} ms per 2x{4 * cells / 2**30:.2f} GiB -> {copy_gbs:.0f} GB/s")
     for mode in args.paths.split(","):
         w = make_world(S, ctx, rs, args.workload)
-        if mode == "blocked_dense":  # the LDS kernel with tile sleeping off: every tile loaded and stored
+        if mode == "blocked_dense":  # tile sleeping off: LDS tiles are all loaded and stored
             w.set_sleep(False)
         sub, tune, lds_kernel = args.sub, None, None
         if mode == "blocked_tuned":  # the variant se_world_autotune picks for this run length (untimed)
@@ -557,9 +574,16 @@ def main():
             tune = {"variant": vi, "tile": list(w.variant_info(1, vi)[:2]), "halo": sub,
                     "trial_ms_per_step": trial_ms, "seconds": time.perf_counter() - t0}
             log(f"autotune for {args.steps} steps: variant {vi} {w.variant_info(1, vi)}, {sub} sub-steps per launch")
+        sliced = False
         if mode.startswith("blocked"):
-            tw, th, c = w.variant_info(1, w.variant_info(2, sub)[0])
+            which = tune["variant"] if tune else w.variant_info(2, sub)[0]
+            tw, th, c = w.variant_info(1, which)
             lds_kernel = f"se_step_lds_{tw}x{th}_h{c // 1000}_t{c % 1000}"
+            sl = sliced_variant(S, w)
+            sliced = sl is not None and (which == sl if tune else args.steps >= SLICED_PAYS)
+            if sliced:
+                lds_kernel = SLICED[args.workload][0]
+                sub = min(sub, SLICED[args.workload][1])
         wall, gpu_ms = time_path(S, w, mode, args.steps, args.warmup, sub)
         launches = args.steps if mode == "plain" else -(-args.steps // sub)
         avg_launch_ms = gpu_ms / launches
@@ -577,7 +601,8 @@ def main():
         else:
             full_ms = avg_launch_ms
         r["full_launch_ms"] = full_ms
-        r["achieved_gbs"] = 8.0 * cells / (full_ms / 1e3) / 1e9
+        r["bytes_per_launch"] = (1 if sliced else 8) * cells
+        r["achieved_gbs"] = r["bytes_per_launch"] / (full_ms / 1e3) / 1e9
         r["roofline_frac"] = r["achieved_gbs"] / HBM_PEAK_GBS
         r["frac_of_copy"] = r["achieved_gbs"] / copy_gbs
         p50, p99 = latencies(w, mode, sub, args.latency_samples)
@@ -607,21 +632,26 @@ def main():
         log(f"blocked paths vs plain after frame {top}: {check}")
     for w in worlds.values():
         w.close()
-    # headline: the fastest of the plain kernel, the LDS kernel at the default
-    # variant and sub-steps, and the LDS kernel as se_world_autotune picks it for
+    # headline: the fastest of the plain kernel, the blocked path at its default
+    # variant and --sub sub-steps, and the blocked path as se_world_autotune picks it for
     # this run length (its trials run before the warmup, outside the timed steps)
     best = max((m for m in results if m in ("plain", "blocked", "blocked_tuned")), key=lambda m: results[m]["gcups"])
     R = results[best]
     kernel = R["kernel"]
+    kernel_ms = R["full_launch_ms"]
     prof = load_profile(kernel, args.workload)
     traffic = prof.get("bytes_per_launch")
     valu = None
     if prof.get("valu_wave_instr_per_launch"):
-        rate = prof["valu_wave_instr_per_launch"] / (R["full_launch_ms"] / 1e3)
+        # the sliced kernels' launches are profiled by themselves: the timed ones include
+        # the planes, packing and unpacking
+        kernel_ms = prof["avg_us"] / 1e3 if kernel.startswith("se_sl_") else R["full_launch_ms"]
+        rate = prof["valu_wave_instr_per_launch"] / (kernel_ms / 1e3)
         valu = {"bound": "valu", "kernel": kernel, "achieved": rate, "peak": VALU_PEAK_WAVE_INSTR_PER_S,
                 "unit": "wave64 VALU instructions/s", "frac": rate / VALU_PEAK_WAVE_INSTR_PER_S,
                 "instr_per_launch": prof["valu_wave_instr_per_launch"],
-                "source": "SQ_INSTS_VALU per launch from profiles/traffic.json over this run's launch time"}
+                "source": "SQ_INSTS_VALU per launch from profiles/traffic.json over " +
+                          ("the traced launch time there" if kernel.startswith("se_sl_") else "this run's launch time")}
     cpu = None if args.no_cpu_baseline else cpu_baseline(
         single_sample(args.workload), steps=40,
         what=f"2048x2048 world of the same fill and rules as {args.workload} (llvmpipe holds at most 8192^2 RGBA32F)")
@@ -642,11 +672,12 @@ def main():
                    "steps_per_launch": R["steps_per_launch"], "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "kernel": kernel, "achieved": R["achieved_gbs"], "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": R["achieved_gbs"] / HBM_PEAK_GBS, "traffic": traffic,
-                     "algorithmic_bytes_per_launch": 8 * cells, "avg_launch_ms": R["full_launch_ms"],
+                     "algorithmic_bytes_per_launch": R["bytes_per_launch"], "avg_launch_ms": R["full_launch_ms"],
                      "launch_timing": ("the timed steps' launches" if best == "plain" else
                                        f"{args.roofline_launches} launches of {R['steps_per_launch']} sub-steps "
-                                       f"after the timed steps"),
-                     "binding_limit": binding_limit(best, traffic, R["full_launch_ms"], valu)},
+                                       f"after the timed steps" + (", their hash planes, packing and unpacking "
+                                       "included" if kernel.startswith("se_sl_") else "")),
+                     "binding_limit": binding_limit(best, traffic, kernel_ms, valu)},
         "roofline_valu": valu,
         "cpu_baseline": cpu,
         "copy_reference": {"gbs": copy_gbs, "ms": copy_ms, "frac_of_peak": copy_gbs / HBM_PEAK_GBS},

@@ -130,7 +130,7 @@ int se_world_step_blocked(se_world* w, uint32_t nsteps, uint32_t sub);
  * a=workgroups of LDS variant `index` resident at once on the device (the
  * batch's persistent launch shape), b=its LDS bytes per workgroup).  The last
  * LDS index of a rule set with a sliced form (bit planes, se_world_step_blocked's
- * choice for longer runs) names those kernels: LDS bytes 0, single worlds only. */
+ * choice for longer runs) names those kernels: LDS bytes 0. */
 int se_world_set_variant(se_world* w, int32_t plain_variant, int32_t lds_variant);
 /* Tile sleeping of se_world_step_blocked (no reference counterpart; on by
  * default): an LDS tile whose cells, halo included, all hold one material whose
