@@ -85,6 +85,8 @@ struct se_module {
     std::vector<int> lds_grid;       // resident workgroups per LDS variant at full occupancy (multiple of 8)
     std::vector<int> lds_waves;      // resident wavefronts per CU per LDS variant
     int default_lds = 0;             // LDS variant of se_world_step_blocked when none is set
+    int wide_lds = 0;  // of the default's tile and halo, the variant with the most threads
+    int cus = 0;
     hipFunction_t plain = nullptr, fill = nullptr, fill_seeded = nullptr, copy = nullptr, fill_spec = nullptr;
     hipFunction_t render[3] = {};  // se_render_r1/2/4: colour and light side-outputs of a step
     hipFunction_t noise_fill = nullptr;  // se_noise_fill: the colour noise image

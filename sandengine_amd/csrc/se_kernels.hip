@@ -1245,7 +1245,7 @@ struct se_bworld {
     int cur0;
     const se_mod* mods;  // modifications for the world's first step in this run
     int nmods;
-    int pad;
+    int per;  // steps a round where not the launch's k (worlds inside one tile), else 0
 };
 
 // Index of the world owning item `item`: prefix[w] <= item < prefix[w+1].
@@ -1356,8 +1356,8 @@ __device__ __forceinline__ bool se_tile_sleeps(const unsigned char* __restrict__
         for (int item = (int)blockIdx.x; item < n_items; item += (int)gridDim.x) {                            \
             const int w = se_owner(prefix, n_active, item);                                                   \
             const se_bworld& B = worlds[w];                                                                   \
-            const int done = round * k;                                                                       \
-            const int nsub = min(k, B.steps - done);                                                          \
+            const int per = B.per ? B.per : k, done = round * per;                                            \
+            const int nsub = min(per, B.steps - done);                                                        \
             const int cur = (B.cur0 + round) & 1;                                                             \
             se_lds_body<TW, TH, HB, NT>(B.buf[cur], B.buf[cur ^ 1], B.W, B.H, B.pitch, B.frame0 + done, nsub,  \
                                         B.tiles_x, item - prefix[w], done == 0 ? B.mods : nullptr,            \

@@ -37,7 +37,7 @@ struct BWorld {
     int W, H, pitch, tiles_x, ntiles;
     int frame0, steps, cur0;
     const void* mods;
-    int nmods, pad;
+    int nmods, per;
 };
 static_assert(sizeof(BWorld) == 64, "se_bworld layout");
 
@@ -139,15 +139,35 @@ extern "C" int se_grids_step_noalloc(se_ctx* ctx, const se_ruleset* rs, se_grid_
 
     // single-tile grids first (all their steps in one work item), then the
     // multi-tile ones, longest first, so that each round's active set is a prefix
-    uint32_t order[SE_NOALLOC_MAX_GRIDS];
-    uint32_t ns = 0, nl = 0;
+    uint32_t order[SE_NOALLOC_MAX_GRIDS], per[SE_NOALLOC_MAX_GRIDS];
+    uint32_t ns = 0, nl = 0, most = 0;
+    size_t tiles = 0;
     auto single = [&](uint32_t i) { return grids[i].w <= (uint32_t)v.tw && grids[i].h <= (uint32_t)v.th; };
+    auto rounds_of = [&](uint32_t i) { return (steps[i] + per[i] - 1) / per[i]; };
+    for (uint32_t i = 0; i < n; i++) {
+        if (!steps[i]) continue;
+        tiles += (size_t)((grids[i].w + v.tw - 1) / v.tw) * ((grids[i].h + v.th - 1) / v.th);
+        per[i] = single(i) ? steps[i] : k;
+        most = std::max(most, rounds_of(i));
+    }
+    // Single-tile grids beside the rounds of the others, where the device holds all tiles
+    // at once: a launch of their own ahead of the rounds keeps a few workgroups busy for as
+    // long as their longest chain takes (40 grids of 64 to 512 cells a side, one of them
+    // inside a tile: 897 us so, 675 beside).  They have no halo, so any number of steps a
+    // round is right; an odd number of rounds leaves the grid in the buffer that one
+    // launch would.
+    const bool merge = most > 1 && tiles <= (size_t)mod->lds_grid[vi];
+    for (uint32_t i = 0; i < n; i++) {
+        if (!merge || !steps[i] || !single(i)) continue;
+        per[i] = (steps[i] + most - 1) / most;
+        while (rounds_of(i) % 2 == 0) per[i]++;
+    }
     for (uint32_t i = 0; i < n; i++)
-        if (steps[i] && single(i)) order[ns++] = i;
+        if (steps[i] && single(i) && !merge) order[ns++] = i;
     for (uint32_t i = 0; i < n; i++)
-        if (steps[i] && !single(i)) order[ns + nl++] = i;
+        if (steps[i] && (merge || !single(i))) order[ns + nl++] = i;
     std::sort(order + ns, order + ns + nl, [&](uint32_t a, uint32_t b) {  // in place: no temporary buffer
-        return steps[a] != steps[b] ? steps[a] > steps[b] : a < b;
+        return rounds_of(a) != rounds_of(b) ? rounds_of(a) > rounds_of(b) : a < b;
     });
     pre_small[0] = 0;
     pre_large[0] = 0;
@@ -165,6 +185,7 @@ extern "C" int se_grids_step_noalloc(se_ctx* ctx, const se_ruleset* rs, se_grid_
         b.frame0 = g.frame + 1;
         b.steps = (int)steps[i];
         b.cur0 = g.cur;
+        b.per = j < ns || per[i] == k ? 0 : (int)per[i];
         int nm = 0;  // the kernels' modification loop ends at a size-0 entry (falling_sand.glsl:139-141)
         while (nm < (int)mcount[i] && hm[g.mod_first + nm].mod_size != 0) nm++;
         b.nmods = nm;
@@ -178,27 +199,34 @@ extern "C" int se_grids_step_noalloc(se_ctx* ctx, const se_ruleset* rs, se_grid_
     HIPCHECK(hipEventRecord(ctx->staging_done, st));
 
     const uint32_t* tbl = mod->table;
-    hipFunction_t f = mod->batch[vi];
+    // Up to three tiles a CU the same tile with more wavefronts is ahead (160 steps, four
+    // materials: 72 tiles 529 us with 256 threads and 397 with 512, 252 tiles 578 / 449, 720
+    // 800 / 730, 1080 1028 / 1145; chain form: 252 tiles 1586 / 1050): a tile's sub-steps are
+    // a serial chain of LDS reads and barriers, which more wavefronts shorten
+    // until the CU's others fill the waits.
+    auto launch_tiles = [&](int items, const void* r, const void* prefix, int active, int round, int steps_each) {
+        const int use = items <= 3 * mod->cus ? mod->wide_lds : vi;
+        return launch_ex(mod->batch[use], (unsigned)items, (unsigned)mod->lds[use].first.nt, 0u, st, r,
+                         (const int*)prefix, active, round, steps_each, tbl);
+    };
     if (ns) {
-        int rc = launch_ex(f, (unsigned)pre_small[ns], (unsigned)v.nt, 0u, st, (const void*)dev,
-                           (const int*)(dev + kOffPreSmall), (int)ns, 0, (int)(1 << 30), tbl);
+        int rc = launch_tiles(pre_small[ns], dev, dev + kOffPreSmall, (int)ns, 0, 1 << 30);
         if (rc) return rc;
     }
     if (nl) {
         const BWorld* lrec = (const BWorld*)dev + ns;
-        uint32_t rounds = (steps[order[ns]] + k - 1) / k;
+        const uint32_t rounds = rounds_of(order[ns]);
         for (uint32_t r = 0; r < rounds; r++) {
             int act = 0;
-            while (act < (int)nl && steps[order[ns + act]] > r * k) act++;
-            int rc = launch_ex(f, (unsigned)pre_large[act], (unsigned)v.nt, 0u, st, (const void*)lrec,
-                               (const int*)(dev + kOffPreLarge), act, (int)r, (int)k, tbl);
+            while (act < (int)nl && rounds_of(order[ns + act]) > r) act++;
+            int rc = launch_tiles(pre_large[act], lrec, dev + kOffPreLarge, act, (int)r, (int)k);
             if (rc) return rc;
         }
     }
     for (uint32_t j = 0; j < ns + nl; j++) {
         const uint32_t i = order[j];
         grids[i].frame += (int32_t)steps[i];
-        grids[i].cur ^= j < ns ? 1 : (int32_t)(((steps[i] + k - 1) / k) & 1);
+        grids[i].cur ^= (int32_t)(rounds_of(i) & 1);
     }
     return SE_OK;
 }

@@ -388,6 +388,7 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         int per_cu = 0, cus = 0;
         HIPCHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, v.nt, 0));
         HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+        m->cus = cus;
         m->lds.push_back({v, f});
         m->batch.push_back(fb);
         m->lds_bytes.push_back(bytes);
@@ -414,6 +415,11 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         else if (!enough && !d_enough && m->lds_waves[i] > m->lds_waves[d]) m->default_lds = (int)i;
     }
     if (m->default_lds < 0) m->default_lds = 0;
+    m->wide_lds = m->default_lds;
+    for (size_t i = 0; i < m->lds.size(); i++) {
+        const se::LdsVariant &v = m->lds[i].first, &d = m->lds[m->default_lds].first;
+        if (v.tw == d.tw && v.th == d.th && v.hb == d.hb && v.nt > m->lds[m->wide_lds].first.nt) m->wide_lds = (int)i;
+    }
     if (info.sliced.ok) {
         se_rt::SlicedKernels& K = m->sliced;
         HIPCHECK(hipModuleGetFunction(&K.pack, m->mod, "se_sl_pack"));
