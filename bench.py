@@ -274,17 +274,15 @@ def run_batch(args):
         sys.exit(1)
 
 
-# se_render per cell: id after and before the step (4 + 4), light in (16), colour
+# A step with its outputs per cell: id before and after the step (4 + 4), light in (16), colour
 # noise (4, precomputed per world), light and colour out (16 + 16)
 RENDER_BYTES_PER_CELL = 60
 
 
 def run_render(args):
     """Grid step plus the render side-outputs of every step (colour noise and
-    light propagation) on the 16384^2 four-material world: the plain step kernel
-    then se_render, per step.  se_render dominates; its roofline uses 60
-    algorithmic bytes per cell and its launch time is measured alone with HIP
-    events.  The grid must equal a world stepped without render outputs."""
+    light propagation) on the 16384^2 four-material world, in one launch (se_frame_b2) per
+    step: 60 algorithmic bytes per cell over the time of a step by HIP events.  The grid must equal a world stepped without render outputs."""
     import sandengine_amd as S
     ctx = S.Context(0)
     side, rsname = WORKLOADS["single16k"][:2]
@@ -304,8 +302,8 @@ def run_render(args):
     step_ms = gpu_ms / args.steps
     p50, p99 = latencies(w, "plain", 0, args.latency_samples)
     log(f"step+render: {cells * args.steps / wall / 1e9:.1f} Gcell-upd/s wall, {step_ms:.3f} ms/step by events; "
-        f"se_render alone {render_ms:.3f} ms/launch -> {RENDER_BYTES_PER_CELL * cells / (render_ms / 1e3) / 1e9:.0f} "
-        f"GB/s algorithmic")
+        f"{RENDER_BYTES_PER_CELL * cells / (step_ms / 1e3) / 1e9:.0f} GB/s algorithmic; se_render alone "
+        f"{render_ms:.3f} ms/launch")
     identical = None
     if not args.no_check:
         wp = make_world(S, ctx, rs, "single16k")
@@ -314,9 +312,9 @@ def run_render(args):
         wp.close()
         log(f"grid with render outputs == grid without: {identical}")
     w.close()
-    kernel = "se_render_r4"
+    kernel = "se_frame_b2"
     prof = load_profile(kernel, args.workload)
-    achieved = RENDER_BYTES_PER_CELL * cells / (render_ms / 1e3) / 1e9
+    achieved = RENDER_BYTES_PER_CELL * cells / (step_ms / 1e3) / 1e9
     cpu = None if args.no_cpu_baseline else cpu_baseline(
         single_sample("single16k"), steps=40,
         what="2048x2048 world of the same fill and rules as single16k (the reference program computes colour and "
@@ -328,10 +326,10 @@ def run_render(args):
         "scaling": "weak", "vs_baseline": None, "dtype": "u32 grid, f32 colour and light",
         "data": "synthetic (seeded SplitMix64 fill generated on the device)",
         "config": {"workload": DESCR["single16k"] + "; colour and light side-outputs of every step",
-                   "path": "plain step + se_render per step", "rules": rsname, "parallelism": "single GPU"},
+                   "path": "step, colour and light in one launch per step", "rules": rsname, "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": prof.get("bytes_per_launch"),
-                     "algorithmic_bytes_per_launch": RENDER_BYTES_PER_CELL * cells, "avg_launch_ms": render_ms},
+                     "algorithmic_bytes_per_launch": RENDER_BYTES_PER_CELL * cells, "avg_launch_ms": step_ms},
         "cpu_baseline": cpu,
         "copy_reference": {"gbs": copy_gbs, "ms": copy_ms, "frac_of_peak": copy_gbs / HBM_PEAK_GBS},
         "paths": {"step_and_render": {"gpu_ms_per_step": step_ms, "render_ms_per_launch": render_ms,

@@ -88,7 +88,8 @@ struct se_module {
     int wide_lds = 0;  // of the default's tile and halo, the variant with the most threads
     int cus = 0;
     hipFunction_t plain = nullptr, fill = nullptr, fill_seeded = nullptr, copy = nullptr, fill_spec = nullptr;
-    hipFunction_t render[3] = {};  // se_render_r1/2/4: colour and light side-outputs of a step
+    hipFunction_t frame[2] = {};   // se_frame_b1/2: plain step with its colour and light
+    hipFunction_t render = nullptr;  // se_render: colour and light alone
     hipFunction_t noise_fill = nullptr;  // se_noise_fill: the colour noise image
     hipFunction_t plain_v[6] = {};  // se_step_plain_r{1,2,4}_nt{0,1}
     std::vector<std::pair<se::LdsVariant, hipFunction_t>> lds;

@@ -1600,39 +1600,19 @@ __device__ __forceinline__ float4 se_cell_light(u32 c, int x, int y, int W, int 
     return make_float4(avg.x * 0.5f + mx.x * 0.5f, avg.y * 0.5f + mx.y * 0.5f, avg.z * 0.5f + mx.z * 0.5f, avg.w);
 }
 
-// One wavefront per 64-column strip and R rows.  All loads of the R + 2 rows are
-// issued before the first light term, at addresses clamped into the world: no
-// branch stands between them, so a wavefront waits for memory once.  (A walk down 8
-// rows, loading one ahead, took 1.4 us a row by its waits, however small the world:
-// 20 us a launch at 960x540, 9 at 64x64.)  Stores past the caches: with ordinary ones
-// 4096x4096 takes 4 % longer and 1920x1080 the same.  A frame of step and outputs, before and
-// now: 64x64 14.9 and 6.2 us, 960x540 25.3 and 14.7, 1920x1080 41.8 and 33.1, 4096x4096 245 and
-// 208, of which 155 are its 60 bytes a cell at the rate of a large copy.
+// The R + 2 rows around rows y0 .. y0 + R - 1 of a 64-column strip, at addresses
+// clamped into the world: no branch stands between the loads, so a wavefront that issues
+// them first waits for memory once.
 template <int R>
-__device__ __forceinline__ void se_render_body(const u32* __restrict__ prev, const u32* __restrict__ cur,
-                                               const float4* __restrict__ light_in, float4* __restrict__ light_out,
-                                               float4* __restrict__ color_out, const float* __restrict__ noise, int W,
-                                               int H, int pitch) {
-    const int lane = (int)(threadIdx.x & 63);
-    const int across = (W + 255) / 256, by = (int)blockIdx.x / across;  // 1-D grid, rows of 4 strips
-    const int sx = (((int)blockIdx.x - by * across) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * 64;
-    if (sx >= W) return;
-    const int x = sx + lane, xc = min(x, W - 1);
-    const int y0 = by * R;
-    se_lraw raw[R + 2];
-    u32 id[R];
-    float nz[R];
+__device__ __forceinline__ void se_light_rows(se_lraw (&raw)[R + 2], const u32* __restrict__ prev,
+                                              const float4* __restrict__ light_in, int x, int y0, int lane, int W,
+                                              int H, int pitch) {
+    const int xc = min(x, W - 1);
 #pragma unroll
     for (int j = 0; j < R + 2; j++) {
         const size_t at = (size_t)min(max(y0 - 1 + j, 0), H - 1) * pitch + xc;
         raw[j].L = raw[j].Le = light_in[at];
         raw[j].P = raw[j].Pe = prev[at];
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const size_t at = (size_t)min(y0 + r, H - 1) * pitch + xc;
-        id[r] = cur[at];
-        nz[r] = noise[at];
     }
     if (lane == 0 || lane == 63) {
         const int xe = lane == 0 ? max(x - 1, 0) : min(x + 1, W - 1);
@@ -1643,6 +1623,42 @@ __device__ __forceinline__ void se_render_body(const u32* __restrict__ prev, con
             raw[j].Pe = prev[at];
         }
     }
+}
+
+// Colour of id c with the cell's noise.
+__device__ __forceinline__ float4 se_cell_color(u32 c, float nz) {
+    float4 col = se_color(c);
+    if (c != SE_EMPTY) {
+        const float d = nz * 0.25f;
+        col.x = fminf(fmaxf(col.x - d, 0.0f), 1.0f);
+        col.y = fminf(fmaxf(col.y - d, 0.0f), 1.0f);
+        col.z = fminf(fmaxf(col.z - d, 0.0f), 1.0f);
+    }
+    return col;
+}
+
+// Colour and light alone (of a clearing frame, and for timing): one wavefront per
+// 64-column strip and R rows.
+template <int R>
+__device__ __forceinline__ void se_render_body(const u32* __restrict__ prev, const u32* __restrict__ cur,
+                                               const float4* __restrict__ light_in, float4* __restrict__ light_out,
+                                               float4* __restrict__ color_out, const float* __restrict__ noise, int W,
+                                               int H, int pitch) {
+    const int lane = (int)(threadIdx.x & 63);
+    const int across = (W + 255) / 256, by = (int)blockIdx.x / across;  // 1-D grid, rows of 4 strips
+    const int sx = (((int)blockIdx.x - by * across) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * 64;
+    if (sx >= W) return;
+    const int x = sx + lane, y0 = by * R;
+    se_lraw raw[R + 2];
+    u32 id[R];
+    float nz[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const size_t at = (size_t)min(y0 + r, H - 1) * pitch + min(x, W - 1);
+        id[r] = cur[at];
+        nz[r] = noise[at];
+    }
+    se_light_rows<R>(raw, prev, light_in, x, y0, lane, W, H, pitch);
     const bool inner = sx > 0 && sx + 64 < W && y0 > 0 && y0 + R < H;  // uniform
     se_lrow up = se_light_row(raw[0], lane), mid = se_light_row(raw[1], lane);
 #pragma unroll
@@ -1652,14 +1668,7 @@ __device__ __forceinline__ void se_render_body(const u32* __restrict__ prev, con
         if (x < W && y < H) {
             const size_t p = (size_t)y * pitch + x;
             const u32 c = se_decode(id[r]);
-            float4 col = se_color(c);
-            if (c != SE_EMPTY) {
-                const float d = nz[r] * 0.25f;
-                col.x = fminf(fmaxf(col.x - d, 0.0f), 1.0f);
-                col.y = fminf(fmaxf(col.y - d, 0.0f), 1.0f);
-                col.z = fminf(fmaxf(col.z - d, 0.0f), 1.0f);
-            }
-            se_store_f4(color_out + p, col);
+            se_store_f4(color_out + p, se_cell_color(c, nz[r]));
             se_store_f4(light_out + p, inner ? se_cell_light<true>(c, x, y, W, H, up, mid, dn)
                                              : se_cell_light<false>(c, x, y, W, H, up, mid, dn));
         }
@@ -1668,13 +1677,116 @@ __device__ __forceinline__ void se_render_body(const u32* __restrict__ prev, con
     }
 }
 
-#define SE_RENDER_KERNEL(R)                                                                                          \
-    extern "C" __global__ __launch_bounds__(256) void se_render_r##R(                                                \
-        const u32* __restrict__ prev, const u32* __restrict__ cur, const float4* __restrict__ light_in,              \
-        float4* __restrict__ light_out, float4* __restrict__ color_out, const float* __restrict__ noise, int W, int H, \
-        int pitch) {                                                                                                 \
-        se_render_body<R>(prev, cur, light_in, light_out, color_out, noise, W, H, pitch);                            \
+extern "C" __global__ __launch_bounds__(256) void se_render(
+    const u32* __restrict__ prev, const u32* __restrict__ cur, const float4* __restrict__ light_in,
+    float4* __restrict__ light_out, float4* __restrict__ color_out, const float* __restrict__ noise, int W, int H,
+    int pitch) {
+    se_render_body<4>(prev, cur, light_in, light_out, color_out, noise, W, H, pitch);
+}
+
+// The plain step and its outputs in one pass, one wavefront per 64-column strip and B
+// block rows: what the light needs of the grid before the step, the cells of the rows and
+// of their neighbours, is what the step reads.  A lane evaluates the block of its own
+// column (each block twice, by both its lanes) and keeps its own two cells.  Bound by
+// memory for large worlds, by one wait for it and the light terms for small ones, so all
+// loads come first (a walk down 8 rows, loading one ahead, waited 1.4 us a row).  Images
+// are stored past the caches: with ordinary stores 4096x4096 takes 4 % longer.
+// A frame, by the plain kernel and a walk over its output / by the plain kernel and
+// such loads / in one pass: 64x64 14.9 / 6.4 / 4.8 us, 960x540 25.3 / 14.9 / 9.8, 1920x1080
+// 41.8 / 33.8 / 28.0, 4096x4096 245 / 207 / 184, where 60 bytes a cell take 155 at the rate
+// of a large copy.
+struct se_frame_args {  // the arguments as they lie in the kernel's argument segment
+    const u32* in;
+    u32* out;
+    const float4* light_in;
+    float4 *light_out, *color_out;
+    const float* noise;
+    int W, H, pitch, frame, offx, offy;
+    const se_mod* mods;
+    int nmods;
+    se_few few;
+};
+
+template <int B>
+__device__ __forceinline__ void se_frame_body(const u32* __restrict__ in, u32* __restrict__ out,
+                                              const float4* __restrict__ light_in, float4* __restrict__ light_out,
+                                              float4* __restrict__ color_out, const float* __restrict__ noise, int W,
+                                              int H, int pitch, int frame, int offx, int offy, se_cmods mods,
+                                              int nmods) {
+    constexpr int R = 2 * B;
+    const int lane = (int)(threadIdx.x & 63);
+    const int across = (W + 255) / 256, by = (int)blockIdx.x / across;
+    const int sx = (((int)blockIdx.x - by * across) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * 64;
+    if (sx >= W) return;
+    const int x = sx + lane, y0 = by * R - offy;
+    se_lraw raw[R + 2];
+    u32 id[R];
+    float nz[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) nz[r] = noise[(size_t)min(max(y0 + r, 0), H - 1) * pitch + min(x, W - 1)];
+    se_light_rows<R>(raw, in, light_in, x, y0, lane, W, H, pitch);
+    const bool left = ((lane ^ offx) & 1) == 0;  // the lane's column is its block's left one
+    const int xe = lane == 0 ? x - 1 : x + 1;
+    const bool has_edge = (lane == 0 || lane == 63) && offx == 1;
+#pragma unroll
+    for (int r = 0; r < R; r++) {  // own cell and the other of its row in the block
+        const int y = y0 + r;
+        const bool row = y >= 0 && y < H;
+        id[r] = row && x < W ? se_decode(raw[r + 1].P) : SE_WALLID;
     }
-SE_RENDER_KERNEL(1)
-SE_RENDER_KERNEL(2)
-SE_RENDER_KERNEL(4)
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        u32 o[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int r = 2 * b + i, y = y0 + r;
+            const u32 v = id[r];
+            const u32 fl = (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xf, 0xf, false);
+            const u32 fr = (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, false);
+            const u32 e = y >= 0 && y < H && xe >= 0 && xe < W ? se_decode(raw[r + 1].Pe) : SE_WALLID;
+            o[i] = has_edge ? e : left ? fr : fl;
+        }
+        u32 a = left ? id[2 * b] : o[0], bb = left ? o[0] : id[2 * b];
+        u32 c = left ? id[2 * b + 1] : o[1], d = left ? o[1] : id[2 * b + 1];
+        se_block(a, bb, c, d, (u32)(left ? x : x - 1), (u32)(y0 + 2 * b), (u32)frame);
+        id[2 * b] = left ? a : bb;
+        id[2 * b + 1] = left ? c : d;
+    }
+    const bool touched = nmods > 0 && se_mods_touch(mods, nmods, sx, sx + 63, y0, y0 + R - 1);
+    const bool inner = sx > 0 && sx + 64 < W && y0 > 0 && y0 + R < H;  // uniform
+    se_lrow up = se_light_row(raw[0], lane), mid = se_light_row(raw[1], lane);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int y = y0 + r;
+        const se_lrow dn = se_light_row(raw[r + 2], lane);
+        if (x < W && y >= 0 && y < H) {
+            const size_t p = (size_t)y * pitch + x;
+            u32 c = id[r];
+            if (touched) {
+                const int m = se_mod_override(mods, nmods, x, y);
+                if (m >= 0) c = (u32)m;
+            }
+            out[p] = c;
+            c = se_decode(c);
+            se_store_f4(color_out + p, se_cell_color(c, nz[r]));
+            se_store_f4(light_out + p, inner ? se_cell_light<true>(c, x, y, W, H, up, mid, dn)
+                                             : se_cell_light<false>(c, x, y, W, H, up, mid, dn));
+        }
+        up = mid;
+        mid = dn;
+    }
+}
+
+#define SE_FRAME_KERNEL(B)                                                                                           \
+    extern "C" __global__ __launch_bounds__(256) void se_frame_b##B(                                                 \
+        const u32* __restrict__ in, u32* __restrict__ out, const float4* __restrict__ light_in,                      \
+        float4* __restrict__ light_out, float4* __restrict__ color_out, const float* __restrict__ noise, int W, int H, \
+        int pitch, int frame, int offx, int offy, const se_mod* __restrict__ mods, int nmods, se_few) {              \
+        const se_cmods few = (se_cmods)((const __attribute__((address_space(4))) char*)                              \
+                                            __builtin_amdgcn_kernarg_segment_ptr() +                                 \
+                                        __builtin_offsetof(se_frame_args, few));                                     \
+        se_frame_body<B>(in, out, light_in, light_out, color_out, noise, W, H, pitch, frame, offx, offy,             \
+                         nmods <= SE_PLAIN_MODS ? few : (se_cmods)mods, nmods);                                      \
+    }
+SE_FRAME_KERNEL(1)
+SE_FRAME_KERNEL(2)

@@ -335,8 +335,9 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
     HIPCHECK(hipModuleGetFunction(&m->fill_seeded, m->mod, "se_fill_seeded"));
     HIPCHECK(hipModuleGetFunction(&m->copy, m->mod, "se_copy"));
     HIPCHECK(hipModuleGetFunction(&m->fill_spec, m->mod, "se_fill_spec"));
-    for (int i = 0; i < 3; i++)
-        HIPCHECK(hipModuleGetFunction(&m->render[i], m->mod, ("se_render_r" + std::to_string(1 << i)).c_str()));
+    for (int i = 0; i < 2; i++)
+        HIPCHECK(hipModuleGetFunction(&m->frame[i], m->mod, ("se_frame_b" + std::to_string(1 << i)).c_str()));
+    HIPCHECK(hipModuleGetFunction(&m->render, m->mod, "se_render"));
     HIPCHECK(hipModuleGetFunction(&m->noise_fill, m->mod, "se_noise_fill"));
     int max_lds = 65536;
     hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device);
@@ -497,17 +498,10 @@ int launch_fill(se_world* w, uint32_t* g, uint32_t v) {
 // Colour and light of the step that turned `prev` into `cur` (render enabled).
 int render_step(se_world* w, const uint32_t* prev, const uint32_t* cur) {
     if (!w->color) return SE_OK;
-    // Rows a wavefront.  One until there are two wavefronts per SIMD (512x256: 9.1 us a frame
-    // against 9.5 with two; 512x512 11.6 against 10.3), then two, so that half as many rows are
-    // read twice, and four once the outputs outgrow the caches (2048x1024: 33.1 against 32.8 with
-    // two; 2560x1440 51.4 against 53.0; 3840x2160 103 against 106).
-    const uint64_t waves = (uint64_t)((w->W + 63) / 64) * w->H;
-    const int v = waves <= 2048 ? 0 : waves <= 32768 ? 1 : 2;
-    const uint32_t rows = 1u << v;
-    const uint32_t groups = (w->W + 255) / 256 * ((w->H + rows - 1) / rows);
+    const uint32_t groups = (w->W + 255) / 256 * ((w->H + 3) / 4);  // 4 rows a wavefront
     void* args[] = {(void*)&prev, (void*)&cur, &w->light[w->lcur], &w->light[w->lcur ^ 1], &w->color,
                     (void*)&w->noise, (void*)&w->W, (void*)&w->H, (void*)&w->pitch};
-    HIPCHECK(hipModuleLaunchKernel(w->mod->render[v], groups, 1, 1, 256, 1, 1, 0, w->stream, args, nullptr));
+    HIPCHECK(hipModuleLaunchKernel(w->mod->render, groups, 1, 1, 256, 1, 1, 0, w->stream, args, nullptr));
     w->lcur ^= 1;
     return SE_OK;
 }
@@ -534,6 +528,21 @@ int se_rt::plain_step(se_world* w) {
     if (rc) return rc;
     int ox, oy;
     offset_of(w->frame, ox, oy);
+    if (w->color) {  // the step and its outputs in one launch
+        // One block row a wavefront; two, which read fewer rows twice, once the images outgrow
+        // the caches (us a frame with one and two, four materials and twelve: 960x540 9.8 / 10.7 and
+        // 10.3 / 11.4, 1920x1080 28.0 / 27.9 and 28.6 / 30.3, 3840x2160 92.7 / 88.1 and 98.6 / 94.3).
+        const int v = (uint64_t)((w->W + 63) / 64) * w->H > 32768;
+        const uint32_t rows = 2u << v;
+        const unsigned groups = (unsigned)((w->W + 255) / 256 * ((w->H + (uint32_t)oy + rows - 1) / rows));
+        rc = launch(w->mod->frame[v], groups, w->stream, (const uint32_t*)in, out, (const void*)w->light[w->lcur],
+                    (void*)w->light[w->lcur ^ 1], (void*)w->color, (const void*)w->noise, (int)w->W, (int)w->H,
+                    (int)w->pitch, (int)w->frame, ox, oy, (const void*)m.ptr, m.n, few);
+        if (rc) return rc;
+        w->lcur ^= 1;
+        w->cur ^= 1;
+        return SE_OK;
+    }
     int strips = (int)((w->W + 255) / 256);
     int brows = (int)((w->H + (uint32_t)oy + 1) / 2);
     static const int kRows[3] = {1, 2, 4};
@@ -543,7 +552,6 @@ int se_rt::plain_step(se_world* w) {
     int rc2 = launch(w->mod->plain_v[w->plain_variant], blocks, w->stream, (const uint32_t*)in, out, (int)w->W,
                      (int)w->H,
                      (int)w->pitch, (int)w->frame, ox, oy, strips, brows, (const void*)m.ptr, m.n, few);
-    if (!rc2) rc2 = render_step(w, in, out);
     if (rc2) return rc2;
     w->cur ^= 1;
     return SE_OK;

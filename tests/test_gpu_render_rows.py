@@ -1,10 +1,11 @@
-"""Light and colour at the edges of the render kernels' strips and row groups.
+"""Grid, light and colour at the edges of the frame kernels' strips and row groups.
 
-The kernels take 1, 2 or 4 rows a wavefront by the world's size; each is run on worlds
-whose height leaves a remainder and whose width leaves a partial strip.  Light is compared,
-bit for bit, with the same float32 formula in numpy (every operation is one
+The kernels step one or two block rows a wavefront, by the world's size, and write their
+colour and light in the same pass; each is run at all four offsets on worlds
+whose height leaves a remainder and whose width leaves a partial strip.  The grid is compared with
+a world stepped without outputs, with short and long modification lists; light, bit for bit, with the same float32 formula in numpy (every operation is one
 IEEE operation in the shader's order, setCell's light loop, math.glsl:154-166); colour with that of
-a short world of one row a wavefront whose first rows hold the same cells.
+a short world whose first rows hold the same cells.
 """
 import numpy as np
 import pytest
@@ -42,9 +43,9 @@ def light_step(prev, light):
     return out
 
 
-# strips of 64 columns x rows: up to 2048 one row a wavefront, up to 32768 two, then four
-@pytest.mark.parametrize("w,h", [(1, 1), (63, 2), (65, 1024), (64, 2049), (129, 683), (65, 16385), (1, 32771)])
-def test_light_and_colour_over_row_groups(w, h):
+# strips of 64 columns x rows: up to 32768 one block row a wavefront, then two
+@pytest.mark.parametrize("w,h", [(1, 1), (2, 1), (63, 2), (64, 3), (65, 1024), (129, 683), (257, 6), (65, 16385), (1, 32771)])
+def test_frames_over_row_groups(w, h):
     print(f"\n[gpu] render rows {w}x{h}", flush=True)
     ctx = S.Context(0)
     rules = S.RuleSet(ctx, S.bundled_ruleset("four_materials"))
@@ -59,14 +60,22 @@ def test_light_and_colour_over_row_groups(w, h):
         a.frame = 1
         return a
 
-    big, small = world(cells), world(cells[:top])
-    for _ in range(4):
+    big, small, plain = world(cells), world(cells[:top]), world(cells)
+    plain.set_render(False)
+    rng = np.random.RandomState(w + h)
+    for f in range(5):
         prev, light = big.download(), big.render_download()[1]
-        big.step(1)
-        small.step(1)
+        for _ in range((0, 2, 0, 9, 1)[f] if h > top else 0):  # below the rows that `small` holds
+            m = (int(rng.randint(w)), int(rng.randint(top + 9, h + 9)), int(rng.randint(2)), int(rng.randint(1, 9)),
+                 int(rng.choice([0, 3, 4])))
+            big.push_modification(*m)
+            plain.push_modification(*m)
+        for a in (big, small, plain):
+            a.step(1)
+        np.testing.assert_array_equal(big.download(), plain.download())
         col, new = big.render_download()
         np.testing.assert_array_equal(new, light_step(prev, light))
-    same = h if top == h else top - 12  # a step reaches two rows, light one
+    same = h if top == h else top - 12  # a step reaches at most two rows
     np.testing.assert_array_equal(col[:same], small.render_download()[0][:same])
-    big.close()
-    small.close()
+    for a in (big, small, plain):
+        a.close()
