@@ -145,7 +145,7 @@ int se_variant_info(const se_world* w, int32_t kind, int32_t index, int32_t* a, 
  * Simulation::output_color / output_light, simulation.rs:109-114).  Enable before
  * the first step to match the reference, whose light starts at zero
  * (simulation.rs:180-181) and then propagates one cell per step.  While
- * enabled, every step runs the plain kernel and then the render kernel (the
+ * enabled, every step writes its colour and light in the same launch (the
  * light needs each step's grid), and the world cannot join a batch.  Images are
  * RGBA f32 per cell, W*H*4 floats row-major on download.  Colour noise uses this
  * platform's sinf, so it matches a GL implementation only to within its sin

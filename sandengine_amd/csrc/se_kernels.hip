@@ -1455,7 +1455,7 @@ extern "C" __global__ __launch_bounds__(256) void se_fill_seeded(u32* __restrict
 // Float arithmetic follows the GLSL expression order with no contraction; sin
 // is this platform's sinf, so the noise matches the GL implementation's only
 // to within its sin error.  The noise depends on the position alone: se_noise_fill
-// evaluates it once per world into an f32 image that se_render reads.
+// evaluates it once per world into an f32 image that the kernels below read.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float se_fract(float x) { return x - floorf(x); }
 __device__ __forceinline__ float2 se_old_hash2(float px, float py) {
@@ -1638,12 +1638,12 @@ __device__ __forceinline__ float4 se_cell_color(u32 c, float nz) {
 }
 
 // Colour and light alone (of a clearing frame, and for timing): one wavefront per
-// 64-column strip and R rows.
-template <int R>
-__device__ __forceinline__ void se_render_body(const u32* __restrict__ prev, const u32* __restrict__ cur,
-                                               const float4* __restrict__ light_in, float4* __restrict__ light_out,
-                                               float4* __restrict__ color_out, const float* __restrict__ noise, int W,
-                                               int H, int pitch) {
+// 64-column strip and 4 rows.
+extern "C" __global__ __launch_bounds__(256) void se_render(
+    const u32* __restrict__ prev, const u32* __restrict__ cur, const float4* __restrict__ light_in,
+    float4* __restrict__ light_out, float4* __restrict__ color_out, const float* __restrict__ noise, int W, int H,
+    int pitch) {
+    constexpr int R = 4;
     const int lane = (int)(threadIdx.x & 63);
     const int across = (W + 255) / 256, by = (int)blockIdx.x / across;  // 1-D grid, rows of 4 strips
     const int sx = (((int)blockIdx.x - by * across) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * 64;
@@ -1675,13 +1675,6 @@ __device__ __forceinline__ void se_render_body(const u32* __restrict__ prev, con
         up = mid;
         mid = dn;
     }
-}
-
-extern "C" __global__ __launch_bounds__(256) void se_render(
-    const u32* __restrict__ prev, const u32* __restrict__ cur, const float4* __restrict__ light_in,
-    float4* __restrict__ light_out, float4* __restrict__ color_out, const float* __restrict__ noise, int W, int H,
-    int pitch) {
-    se_render_body<4>(prev, cur, light_in, light_out, color_out, noise, W, H, pitch);
 }
 
 // The plain step and its outputs in one pass, one wavefront per 64-column strip and B

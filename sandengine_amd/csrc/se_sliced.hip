@@ -342,9 +342,10 @@ extern "C" __global__ __launch_bounds__(256) void se_sl_hash(se_slgrid g) {
 //   * x offset 1: the O words move up by one block (alignbit over the word
 //     columns) and the blocks are (O, E) instead of (E, O).
 // Blocks are never split between lanes otherwise, so one wavefront needs no barriers
-// and no LDS; two that share a tile exchange a word column at odd x offsets.  What the shifts bring in at the tile's sides is wrong inside the world and
-// right at its border (WALL, code 0), so the valid region shrinks by one cell per
-// sub-step on the sides that cut into the world: 16 or 32 columns and `halo` rows
+// and no LDS; two that share a tile exchange a word column at odd x offsets.  What
+// the shifts bring in at the tile's sides is wrong inside the world and right at its
+// border (WALL, code 0), so the valid region shrinks by one cell per sub-step on the
+// sides that cut into the world: 16 or 32 columns and `halo` rows
 // are given up on each side of a tile, none of a world that fits one tile.
 // ---------------------------------------------------------------------------
 template <int NW, int R>
