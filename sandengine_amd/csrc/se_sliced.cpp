@@ -156,6 +156,22 @@ size_t se_rt::sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int
     return ((size_t)g.hash_sets * g.hash_words + past) * classes * sizeof(uint32_t);
 }
 
+// As many whole launches at a time as the budget holds, at least one.  A later chunk
+// can need more room than the first: it may be shorter and take the direct form, whose
+// frames loaded ahead are larger than the shared form's.
+se_rt::SlicedAhead se_rt::sliced_ahead(const SlicedShape& s, SlicedGrid g, int32_t frame0, uint32_t n, int classes) {
+    const uint32_t per_launch = std::min(s.max_sub, n);
+    SlicedAhead a;
+    a.frames = std::min(n, kSlicedMostFrames);
+    while (sliced_hash_layout(g, frame0, a.frames, classes) > kHashBudget && a.frames > (s.halo ? per_launch : 1u)) {
+        a.frames = a.frames / 2;
+        if (s.halo) a.frames = std::max(a.frames / per_launch, 1u) * per_launch;
+    }
+    for (uint32_t at = 0; at < n; at += a.frames)
+        a.bytes = std::max(a.bytes, sliced_hash_layout(g, frame0 + (int32_t)at, std::min(a.frames, n - at), classes));
+    return a;
+}
+
 // Packing, hashing and unpacking cost three launches more than the LDS kernels
 // have, and from the largest worlds a pass over the grid.  The LDS kernels' default
 // tile advances 8 steps in one launch and stays for those; the generated chain,
@@ -184,17 +200,9 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     sliced_geometry(shape, w->W, w->H, g);
     g.pitch = (int)w->pitch;
     const size_t packed = sliced_packed_bytes(g);
-    const uint32_t per_launch = std::min(shape.max_sub, n);
-    // frames hashed at a time: as many whole launches as the budget holds
-    uint32_t ahead = std::min(n, kSlicedMostFrames);
-    size_t hash = sliced_hash_layout(g, w->frame + 1, ahead, K.classes);
-    while (hash > kHashBudget && ahead > (shape.halo ? per_launch : 1u)) {
-        ahead = ahead / 2;
-        if (shape.halo) ahead = std::max(ahead / per_launch, 1u) * per_launch;
-        hash = sliced_hash_layout(g, w->frame + 1, ahead, K.classes);
-    }
-    // later chunks start at another phase of the cycle: a word or two more
-    const size_t bytes = 2 * packed + hash + (size_t)64 * 464 * K.classes;
+    const SlicedAhead plan = sliced_ahead(shape, g, w->frame + 1, n, K.classes);
+    const uint32_t ahead = plan.frames;
+    const size_t bytes = 2 * packed + plan.bytes;
 
     // The scratch belongs to the context: its worlds share one stream, and the
     // launches of one call are enqueued together under the lock.
@@ -229,8 +237,7 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     int from = 0;
     for (uint32_t at = 0; at < n && !rc;) {
         const uint32_t nf = std::min(ahead, n - at);
-        const size_t need = sliced_hash_layout(g, w->frame + 1 + (int)at, nf, K.classes);
-        if (2 * packed + need > ctx->sliced_bytes) return fail(SE_ERR_STATE, "internal: hash planes exceed their scratch");
+        sliced_hash_layout(g, w->frame + 1 + (int)at, nf, K.classes);
         rc = launch2(K.hash, (unsigned)(g.hash_words + 255) / 256, (unsigned)g.hash_sets, 256, w->stream, g);
         for (uint32_t d = 0; d < nf && !rc;) {
             // a launch after the first starts at the head of a cycle where that costs

@@ -58,6 +58,14 @@ constexpr uint32_t kSlicedMostFrames = 32768;  // hashed in one launch (a grid's
 // kernel loads ahead.
 size_t sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int classes);
 
+// How a run of n steps of one world hashes its frames: so many at a time, and the bytes
+// that the planes of every such chunk fit.
+struct SlicedAhead {
+    uint32_t frames = 0;
+    size_t bytes = 0;
+};
+SlicedAhead sliced_ahead(const SlicedShape& s, SlicedGrid g, int32_t frame0, uint32_t n, int classes);
+
 // Is the sliced path taken for n steps of a world whose caller chose no variant?
 bool sliced_pays(const se_module* m, uint32_t n);
 // Wavefronts (64 columns x 64 rows each) that pack and that unpack a world.
