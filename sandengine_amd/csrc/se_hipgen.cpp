@@ -947,6 +947,8 @@ public:
         if (t >= 0xFFFFFFFFll) return Net::kOne;
         for (size_t i = 0; i < classes.size(); i++)
             if (classes[i] == std::make_pair(lane, (uint32_t)t)) return class_lit[i];
+        // here and not after the chain: its last check goes through all class words
+        if (classes.size() == (size_t)kSlicedMaxClasses) throw NotSliced();
         classes.push_back({lane, (uint32_t)t});
         class_lit.push_back(net.input());
         return class_lit.back();
@@ -1208,7 +1210,6 @@ std::string hip_sliced_source(const ParsingResult& r, SlicedInfo& out) {
         return "";
     }
     const int P = (int)sl.classes.size();
-    if (P > kSlicedMaxClasses) return "";
     // does any block change a WALL cell?  (every tuple of codes, every class word)
     bool kept = true;
     {
