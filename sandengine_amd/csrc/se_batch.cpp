@@ -318,7 +318,7 @@ bool make_sliced(SlicedPlan& P, bool single, uint32_t k, size_t squares) {
     // least one launch's.  Each group's planes lie where its largest chunk has room.
     P.n_groups = extent.size();
     const uint32_t least = std::min(single ? 32u : deep, most);
-    for (uint32_t ahead = single ? se_rt::kSlicedMostFrames : std::max(1u, kBatchChunkMost / deep) * deep;;) {
+    for (uint32_t ahead = single ? std::min(most, se_rt::kSlicedMostFrames) : std::max(1u, kBatchChunkMost / deep) * deep;;) {
         uint32_t length = std::min(ahead, single ? ahead : std::max(1u, kBatchChunk / deep) * deep);
         P.groups.clear();
         P.words.clear();

@@ -122,9 +122,11 @@ size_t se_rt::sliced_hash_layout(SlicedGrid& g, int32_t frame0, uint32_t nf, int
     const int wcols = (g.bcols + 3) / 4;
     g.hash_frame0 = frame0;
     // shared form: the range of n of each parity over the frames, and the words of b
-    // that cover it (one more than a tile's last word, for the shifted read)
+    // that cover it (one more than a tile's last word, for the shifted read).  n grows by
+    // 4.5 M a frame and the offsets change it by some thousands, and any four frames hold
+    // both parities, so the first four and the last four frames bound it.
     int64_t lo[2] = {0, 0}, hi[2] = {-1, -1};
-    for (uint32_t i = 0; i < nf; i++) {
+    for (uint32_t i = 0; i < nf; i = i == 3 && nf > 8 ? nf - 4 : i + 1) {
         const int64_t f = (int64_t)frame0 + i;
         const int ox = (int)(f & 1), oy = (f & 3) == 1 || (f & 3) == 2;
         const int64_t n = 461ll * (-ox - g.xpad) + 2131ll * (oy - g.ypad) + 4541161ll * f;
