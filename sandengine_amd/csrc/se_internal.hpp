@@ -87,7 +87,7 @@ struct se_module {
     int default_lds = 0;             // LDS variant of se_world_step_blocked when none is set
     int wide_lds = 0;  // of the default's tile and halo, the variant with the most threads
     int cus = 0;
-    hipFunction_t plain = nullptr, fill = nullptr, fill_seeded = nullptr, copy = nullptr, fill_spec = nullptr;
+    hipFunction_t plain = nullptr, fill = nullptr, fill_seeded = nullptr, copy = nullptr, fill_spec = nullptr, fill_narrow = nullptr;
     hipFunction_t frame[2] = {};   // se_frame_b1/2: plain step with its colour and light
     hipFunction_t render = nullptr;  // se_render: colour and light alone
     hipFunction_t noise_fill = nullptr;  // se_noise_fill: the colour noise image
@@ -174,6 +174,8 @@ inline void sleep_reset(se_world* w) { w->sleep_variant = -1; }
 // Index of the default LDS tile variant of a module (batches and serving use it
 // unless tuned).
 int default_lds_index(const se_module* m);
+// Enqueues the seeded fill of a grid of w.
+int fill_spec(const se_world* w, uint32_t* grid, uint64_t seed, const FillSpec& fs);
 // Device address of the no-allocation scratch array on `device` (current).
 int noalloc_scratch(int device, void** out);
 }  // namespace se_rt

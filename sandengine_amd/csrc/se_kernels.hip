@@ -1383,16 +1383,51 @@ struct se_fillspec {  // fill parameters passed by value
     u32 ids[16], thr[16];
 };
 
-// Up to 16 ids, passed by value.  One wavefront per 256 cells, a quad a lane, leaving
-// as 16-byte stores.  In a row of more than 128 cells they are one row's, and the row
-// and its term of the generator's input are uniform: 16384^2 with three ids takes 187
-// us, at the rate of plain stores (se_fill: 175); with thirteen ids the compares bound
-// it (8192^2: 100 us).  Narrower worlds give a row 2 to 32 lanes and a wavefront 32 to 2
-// rows (8x100000 17 us, and 41 with a wavefront a row); in worlds of up to 4 columns,
-// which have no whole quads, a lane takes a cell (3x1000000 26 us, 49 by quads and 234
-// with a wavefront a row).
+// Up to 16 ids, passed by value.  One wavefront per 256 cells of a row, a quad a
+// lane: the row and its term of the generator's input are uniform, and cells leave
+// as 16-byte stores.  16384^2 with three ids takes 187 us, at the rate of plain
+// stores (se_fill: 175); with thirteen ids the compares bound it (8192^2: 100 us).
 // The form below divides each cell's index by W and reads the tables per cell: 554
-// and 520 us, 22 and 32 for the narrow ones.
+// and 520 us.
+extern "C" __global__ __launch_bounds__(256) void se_fill_spec(u32* __restrict__ g, int W, int H, int pitch,
+                                                               u64 seed, se_fillspec sp) {
+    const int lane = (int)(threadIdx.x & 63), strips = (W + 255) / 256;
+    const int items = strips * H, stride = (int)gridDim.x * 4;
+    for (int i = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); i < items; i += stride) {
+        const int y = i / strips, x = (i - y * strips) * 256 + 4 * lane;
+        if (x >= W) continue;
+        u32 v[4] = {sp.stone_id, sp.stone_id, sp.stone_id, sp.stone_id};
+        if ((long)y < (long)H - sp.stone_rows) {
+            const u64 i0 = (u64)y * (u64)W + (u64)x;
+            u32 r[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                r[j] = (u32)(se_splitmix64((seed << 40) ^ (i0 + (u64)j)) >> 32);
+                v[j] = sp.ids[sp.n - 1];
+            }
+            for (int k = sp.n - 2; k >= 0; k--) {  // the first threshold above r decides
+                const u32 t = sp.thr[k], id = sp.ids[k];
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = r[j] < t ? id : v[j];
+            }
+        }
+        u32* d = g + (size_t)y * (size_t)pitch + x;
+        if (x + 3 < W) {
+            se_store_quad<true>(d, make_uint4(v[0], v[1], v[2], v[3]));
+        } else {
+            d[0] = v[0];
+            if (x + 1 < W) d[1] = v[1];
+            if (x + 2 < W) d[2] = v[2];
+        }
+    }
+}
+
+// The same for worlds of up to 128 columns, of whose rows a wavefront above takes one: a
+// row gets 1 to 32 lanes, a quad each, and in worlds of up to 4 columns, which have no
+// whole quads, a cell each (us a fill, with a wavefront a row / a division per cell / so:
+// 8x100000 41 / 22 / 17, 128x30000 - / 33 / 22, 3x1000000 234 / 32 / 26, by quads 49).
+// A kernel of its own: in one with the form above, that one took 5.1 us and not 4.1 for
+// 1000x1000.
 template <int N>
 __device__ __forceinline__ void se_fill_cells(u32 (&v)[N], int W, int H, u64 seed, const se_fillspec& sp, int x, int y) {
 #pragma unroll
@@ -1405,50 +1440,36 @@ __device__ __forceinline__ void se_fill_cells(u32 (&v)[N], int W, int H, u64 see
         r[j] = (u32)(se_splitmix64((seed << 40) ^ (i0 + (u64)j)) >> 32);
         v[j] = sp.ids[sp.n - 1];
     }
-    for (int k = sp.n - 2; k >= 0; k--) {  // the first threshold above r decides
+    for (int k = sp.n - 2; k >= 0; k--) {
         const u32 t = sp.thr[k], id = sp.ids[k];
 #pragma unroll
         for (int j = 0; j < N; j++) v[j] = r[j] < t ? id : v[j];
     }
 }
 
-__device__ __forceinline__ void se_fill_quad(u32* __restrict__ g, int W, int H, int pitch, u64 seed,
-                                             const se_fillspec& sp, int x, int y) {
-    u32 v[4];
-    se_fill_cells<4>(v, W, H, seed, sp, x, y);
-    u32* d = g + (size_t)y * (size_t)pitch + x;
-    if (x + 3 < W) {
-        se_store_quad<true>(d, make_uint4(v[0], v[1], v[2], v[3]));
-    } else {
-        d[0] = v[0];
-        if (x + 1 < W) d[1] = v[1];
-        if (x + 2 < W) d[2] = v[2];
-    }
-}
-
-extern "C" __global__ __launch_bounds__(256) void se_fill_spec(u32* __restrict__ g, int W, int H, int pitch,
-                                                               u64 seed, se_fillspec sp) {
-    const int lane = (int)(threadIdx.x & 63), stride = (int)gridDim.x * 4;
-    const int wave = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (W > 128) {
-        const int strips = (W + 255) / 256, items = strips * H;
-        for (int i = wave; i < items; i += stride) {
-            const int y = i / strips, x = (i - y * strips) * 256 + 4 * lane;
-            if (x < W) se_fill_quad(g, W, H, pitch, seed, sp, x, y);
-        }
-        return;
-    }
+extern "C" __global__ __launch_bounds__(256) void se_fill_narrow(u32* __restrict__ g, int W, int H, int pitch,
+                                                                 u64 seed, se_fillspec sp) {
     // 1 << bits lanes hold a row, the least that do
     const int bits = W == 1 ? 0 : W <= 4 ? 32 - __builtin_clz((u32)(W - 1)) : 30 - __builtin_clz((u32)(W - 1));
-    const int at = lane & ((1 << bits) - 1), x = W <= 4 ? at : 4 * at;
+    const int at = (int)threadIdx.x & ((1 << bits) - 1), x = W <= 4 ? at : 4 * at;
     if (x >= W) return;
-    for (int y = (wave << (6 - bits)) + (lane >> bits); y < H; y += stride << (6 - bits)) {
+    const int step = (int)gridDim.x << (8 - bits);
+    for (int y = (int)((blockIdx.x * 256u + threadIdx.x) >> bits); y < H; y += step) {
+        u32* d = g + (size_t)y * (size_t)pitch + x;
         if (W <= 4) {
             u32 v[1];
             se_fill_cells<1>(v, W, H, seed, sp, x, y);
-            g[(size_t)y * (size_t)pitch + x] = v[0];
+            d[0] = v[0];
+            continue;
+        }
+        u32 v[4];
+        se_fill_cells<4>(v, W, H, seed, sp, x, y);
+        if (x + 3 < W) {
+            se_store_quad<true>(d, make_uint4(v[0], v[1], v[2], v[3]));
         } else {
-            se_fill_quad(g, W, H, pitch, seed, sp, x, y);
+            d[0] = v[0];
+            if (x + 1 < W) d[1] = v[1];
+            if (x + 2 < W) d[2] = v[2];
         }
     }
 }

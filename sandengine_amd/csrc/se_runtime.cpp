@@ -335,6 +335,7 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
     HIPCHECK(hipModuleGetFunction(&m->fill_seeded, m->mod, "se_fill_seeded"));
     HIPCHECK(hipModuleGetFunction(&m->copy, m->mod, "se_copy"));
     HIPCHECK(hipModuleGetFunction(&m->fill_spec, m->mod, "se_fill_spec"));
+    HIPCHECK(hipModuleGetFunction(&m->fill_narrow, m->mod, "se_fill_narrow"));
     for (int i = 0; i < 2; i++)
         HIPCHECK(hipModuleGetFunction(&m->frame[i], m->mod, ("se_frame_b" + std::to_string(1 << i)).c_str()));
     HIPCHECK(hipModuleGetFunction(&m->render, m->mod, "se_render"));
@@ -555,6 +556,13 @@ int se_rt::plain_step(se_world* w) {
     if (rc2) return rc2;
     w->cur ^= 1;
     return SE_OK;
+}
+
+int se_rt::fill_spec(const se_world* w, uint32_t* grid, uint64_t seed, const FillSpec& fs) {
+    const size_t cells = (size_t)w->W * w->H;
+    const unsigned blocks = (unsigned)std::min<size_t>((cells + 255) / 256, 1u << 16);
+    return launch(w->W > 128 ? w->mod->fill_spec : w->mod->fill_narrow, blocks, w->stream, grid, (int)w->W, (int)w->H,
+                  (int)w->pitch, (unsigned long long)seed, fs);
 }
 
 namespace {
@@ -1216,8 +1224,6 @@ int se_world_fill_seeded(se_world* w, uint64_t seed, const uint32_t* ids, const 
     if (!w || !ids || !thresholds || n < 1 || n > 64) return fail(SE_ERR_ARG, "bad fill arguments");
     DeviceGuard dg(w->ctx->device);
     se_rt::sleep_reset(w);
-    size_t cells = (size_t)w->W * w->H;
-    unsigned blocks = (unsigned)std::min<size_t>((cells + 255) / 256, 1u << 16);
     int rc;
     if (n <= 16) {
         se_rt::FillSpec fs{};
@@ -1226,10 +1232,11 @@ int se_world_fill_seeded(se_world* w, uint64_t seed, const uint32_t* ids, const 
         fs.stone_id = stone_id;
         std::memcpy(fs.ids, ids, n * 4);
         std::memcpy(fs.thr, thresholds, n * 4);
-        rc = launch(w->mod->fill_spec, blocks, w->stream, w->buf[w->cur], (int)w->W, (int)w->H, (int)w->pitch,
-                    (unsigned long long)seed, fs);
+        rc = se_rt::fill_spec(w, w->buf[w->cur], seed, fs);
     } else {
         // ids and thresholds are staged in the world's modification buffer (8 KiB)
+        const size_t cells = (size_t)w->W * w->H;
+        const unsigned blocks = (unsigned)std::min<size_t>((cells + 255) / 256, 1u << 16);
         void* d = w->d_mods;
         uint32_t host[128] = {0};
         std::memcpy(host, ids, n * 4);

@@ -394,10 +394,7 @@ int admit(se_serve* S, Request& r, Arena& A) {
     r.bytes = need;
     r.state = 1;
     const se_rt::FillSpec& fs = S->fills[r.rs];
-    size_t cells = (size_t)r.side * r.side;
-    unsigned blocks = (unsigned)std::min<size_t>((cells + 255) / 256, 1u << 16);
-    return launch(w->mod->fill_spec, blocks, w->stream, w->buf[0], (int)r.side, (int)r.side, (int)pitch,
-                  (unsigned long long)r.fill_seed, fs);
+    return se_rt::fill_spec(w, w->buf[0], r.fill_seed, fs);
 }
 
 int lds_index(const se_module* m) { return se_rt::default_lds_index(m); }
