@@ -136,8 +136,12 @@ int se_world_set_variant(se_world* w, int32_t plain_variant, int32_t lds_variant
  * default): an LDS tile whose cells, halo included, all hold one material whose
  * uniform 2x2 block no rule changes skips its sub-steps, and when it and its
  * eight neighbours were already so in the previous launch it also skips its
- * loads and stores (its output buffer already holds those cells).  Results are
- * identical either way; any other write to the grids restarts the record. */
+ * loads and stores (its output buffer already holds those cells).  The sliced
+ * kernels, in worlds of some 4 M cells and more, do the same by tiles for the
+ * sub-steps, and by squares of 64 x 64 cells for reading and writing the grid,
+ * the latter only while the caller has not asked for the grid's address
+ * (se_world_device_ptr).  Results are identical either way; any other write to
+ * the grids restarts the record. */
 int se_world_set_sleep(se_world* w, int enable);
 int se_variant_info(const se_world* w, int32_t kind, int32_t index, int32_t* a, int32_t* b, int32_t* c);
 /* Render side-outputs of every step: the colour and light images that

@@ -1234,6 +1234,23 @@ std::string hip_sliced_source(const ParsingResult& r, SlicedInfo& out) {
             }
         }
     }
+    // ids whose uniform block no class word changes, as codes
+    for (int i = 0; i < n; i++) {
+        std::vector<uint32_t> in(sl.net.inputs()), got;
+        bool stays = true;
+        for (int c = 0; c < 4; c++)
+            for (int k = 0; k < K; k++) in[c * K + k] = (code[i] >> k) & 1 ? ~0u : 0u;
+        for (uint32_t m = 0; m < (1u << P) && stays; m += 32) {
+            for (int j = 0; j < P; j++) {
+                uint32_t w = 0;
+                for (uint32_t b = 0; b < 32; b++) w |= (((m + b) >> j) & 1u) << b;
+                in[4 * K + j] = w;
+            }
+            sl.net.eval(in, outs, got);
+            for (int c = 0; c < 4 * K; c++) stays = stays && got[c] == in[c];
+        }
+        if (stays) out.stable |= 1u << code[i];
+    }
     out.ok = true;
     out.planes = K;
     out.code = code;

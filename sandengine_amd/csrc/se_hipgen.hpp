@@ -33,6 +33,7 @@ struct SlicedInfo {
     std::vector<int> code;                          // material id -> code
     std::vector<std::pair<int, uint32_t>> classes;  // hash planes: bit set when the lane is <= the threshold
     bool wall_kept = false;                         // no block changes a WALL cell
+    uint32_t stable = 0;                            // bit c: no class word changes a block of four cells of code c
 };
 
 struct HipGenInfo {

@@ -66,7 +66,8 @@ struct FillSpec {  // == se_fillspec in se_kernels.hip
 struct SlicedKernels {
     bool ok = false;
     int planes = 0, classes = 0;  // bit planes of a cell, hash planes of a frame
-    hipFunction_t pack = nullptr, unpack = nullptr, hash = nullptr;
+    uint32_t stable = 0;          // SlicedInfo::stable
+    hipFunction_t pack = nullptr, unpack = nullptr, hash = nullptr, brush = nullptr;
     hipFunction_t bpack = nullptr, bunpack = nullptr, bhash = nullptr;  // the worlds of a batch
     hipFunction_t step[4] = {};  // 2x2 and 4x2 tiles by one wavefront (up to three planes), 2x2 by two, 4x2 by four
 };
@@ -154,23 +155,41 @@ struct se_world {
     void* color = nullptr;
     int lcur = 0;
     // tile sleeping of the LDS kernel (se_tile_sleeps): per tile of variant
-    // sleep_variant, the settled code in the last launch or 0xff; valid only while
-    // nothing but that kernel has written either grid buffer (sleep_variant -1
-    // otherwise)
+    // sleep_variant, the settled code in the last launch or 0xff; of the sliced kernels
+    // (se_slknown), whose variant is the last: per 64 x 64 square, laid out as
+    // sleep_layout says.  Valid only while nothing but those kernels has written either
+    // grid buffer (sleep_variant -1 otherwise)
     unsigned char* d_sleep[2] = {nullptr, nullptr};
     size_t sleep_cap = 0;
     int sleep_variant = -1;
+    int sleep_layout = 0;
     int sleep_p = 0;
+    bool exposed = false;  // the caller has a grid's address and may write through it at any time
     bool sleep_enabled = true;
 };
 
 
 namespace se_rt {
+constexpr int kFewMods = 8;  // SE_PLAIN_MODS of the kernel source
+struct FewMods {             // == se_few
+    se_modification m[kFewMods];
+};
+struct ModsArg {
+    void* ptr;
+    int n;
+};
+// Takes the queued modifications (cut at the first size-0 entry, as the
+// kernel's loop stops there, falling_sand.glsl:139-141) and clears the queue: up to
+// kFewMods go to `few`, if given, where the kernel takes them by value, more to device
+// memory.
+int take_mods(se_world* w, ModsArg& m, FewMods* few = nullptr);
 // One Simulation::run of `w` with the plain kernel (frame += 1, mods, step).
 int plain_step(se_world* w);
 // The grids of `w` were written by something other than the LDS kernel: its
 // tile-sleeping record no longer describes them.
 inline void sleep_reset(se_world* w) { w->sleep_variant = -1; }
+// Room for n bytes in each of w->d_sleep.
+int sleep_room(se_world* w, size_t n);
 // Index of the default LDS tile variant of a module (batches and serving use it
 // unless tuned).
 int default_lds_index(const se_module* m);

@@ -427,6 +427,7 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         HIPCHECK(hipModuleGetFunction(&K.pack, m->mod, "se_sl_pack"));
         HIPCHECK(hipModuleGetFunction(&K.unpack, m->mod, "se_sl_unpack"));
         HIPCHECK(hipModuleGetFunction(&K.hash, m->mod, "se_sl_hash"));
+        HIPCHECK(hipModuleGetFunction(&K.brush, m->mod, "se_sl_brush"));
         HIPCHECK(hipModuleGetFunction(&K.step[2], m->mod, "se_sl_step_2x2s"));
         HIPCHECK(hipModuleGetFunction(&K.step[3], m->mod, "se_sl_step_4x2s"));
         if (info.sliced.planes <= 3) {
@@ -438,6 +439,7 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         HIPCHECK(hipModuleGetFunction(&K.bhash, m->mod, "se_sl_bhash"));
         K.planes = info.sliced.planes;
         K.classes = (int)info.sliced.classes.size();
+        K.stable = info.sliced.stable;
         K.ok = true;
         // listed after the LDS instantiations (never the default among them)
         m->lds.push_back({{128, 128, 32, 128, true}, K.step[2]});
@@ -461,20 +463,9 @@ void offset_of(int32_t frame, int& ox, int& oy) {
     oy = (m == 1 || m == 2) ? 1 : 0;
 }
 
-struct ModsArg {
-    void* ptr;
-    int n;
-};
+}  // namespace
 
-// Uploads the queued modifications (cut at the first size-0 entry, as the
-// kernel's loop stops there, falling_sand.glsl:139-141) and clears the queue.
-// Up to kFewMods of them go to `few` instead, where the kernel takes them by value.
-constexpr int kFewMods = 8;  // SE_PLAIN_MODS of the kernel source
-struct FewMods {
-    se_modification m[kFewMods];
-};
-
-int take_mods(se_world* w, ModsArg& m, FewMods* few = nullptr) {
+int se_rt::take_mods(se_world* w, ModsArg& m, FewMods* few) {
     m.ptr = w->d_mods;
     m.n = 0;
     if (w->pending.empty()) return SE_OK;
@@ -489,6 +480,11 @@ int take_mods(se_world* w, ModsArg& m, FewMods* few = nullptr) {
     m.n = n;
     return SE_OK;
 }
+
+namespace {
+using se_rt::FewMods;
+using se_rt::ModsArg;
+using se_rt::take_mods;
 
 int launch_fill(se_world* w, uint32_t* g, uint32_t v) {
     size_t n = (size_t)w->pitch * w->H;
@@ -565,6 +561,22 @@ int se_rt::fill_spec(const se_world* w, uint32_t* grid, uint64_t seed, const Fil
                   (int)w->pitch, (unsigned long long)seed, fs);
 }
 
+int se_rt::sleep_room(se_world* w, size_t n) {
+    if (n <= w->sleep_cap) return SE_OK;
+    hipFree(w->d_sleep[0]);
+    hipFree(w->d_sleep[1]);
+    w->d_sleep[0] = w->d_sleep[1] = nullptr;
+    w->sleep_cap = 0;
+    w->sleep_variant = -1;
+    for (auto& p : w->d_sleep)
+        if (hipMalloc(&p, n) != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(SE_ERR_HIP, "hipMalloc of a sleep record failed");
+        }
+    w->sleep_cap = n;
+    return SE_OK;
+}
+
 namespace {
 using se_rt::plain_step;
 
@@ -611,17 +623,8 @@ int lds_launch(se_world* w, const std::pair<se::LdsVariant, hipFunction_t>& v, i
     const unsigned char* s_in = nullptr;
     unsigned char* s_out = nullptr;
     if (w->sleep_enabled) {
-        const size_t ntiles = (size_t)tiles_x * tiles_y;
-        if (ntiles > w->sleep_cap) {
-            hipFree(w->d_sleep[0]);
-            hipFree(w->d_sleep[1]);
-            w->d_sleep[0] = w->d_sleep[1] = nullptr;
-            w->sleep_cap = 0;
-            w->sleep_variant = -1;
-            HIPCHECK(hipMalloc(&w->d_sleep[0], ntiles));
-            HIPCHECK(hipMalloc(&w->d_sleep[1], ntiles));
-            w->sleep_cap = ntiles;
-        }
+        rc = se_rt::sleep_room(w, (size_t)tiles_x * tiles_y);
+        if (rc) return rc;
         if (w->sleep_variant == vi) s_in = w->d_sleep[w->sleep_p];
         s_out = w->d_sleep[w->sleep_p ^ 1];
     }
@@ -650,9 +653,9 @@ int blocked_steps(se_world* w, uint32_t nsteps, uint32_t sub) {
     auto* v = pick_lds(w, sub);
     if (!v) return fail(SE_ERR_ARG, "no LDS variant supports " + std::to_string(sub) + " sub-steps");
     if (v->first.sliced || (w->lds_variant < 0 && se_rt::sliced_pays(w->mod.get(), nsteps))) {
-        // the sliced kernels take neither the clearing frame nor modifications: the
-        // step that carries them is a plain one
-        if (nsteps && (w->frame + 1 == 1 || !w->pending.empty())) {
+        // the clearing frame is a step of its own, and so are modifications where a plain
+        // step is faster than the launches that take them into the packed grid
+        if (nsteps && (w->frame + 1 == 1 || (!w->pending.empty() && !se_rt::sliced_takes_mods(w, nsteps)))) {
             int rc = plain_step(w);
             if (rc) return rc;
             nsteps--;
@@ -1214,6 +1217,7 @@ int se_world_sync(se_world* w) {
 int se_world_device_ptr(se_world* w, void** ptr, uint32_t* pitch) {
     if (!w) return fail(SE_ERR_ARG, "null world");
     se_rt::sleep_reset(w);  // the caller may write through the pointer
+    w->exposed = true;
     if (ptr) *ptr = w->buf[w->cur];
     if (pitch) *pitch = w->pitch;
     return SE_OK;

@@ -15,6 +15,7 @@ using se_rt::fail;
 
 namespace {
 
+constexpr size_t kKnownSquares = 1024;      // from so many 64 x 64 squares on a world keeps what is known of them
 constexpr size_t kHashBudget = 128u << 20;  // hash planes made ahead, unless one launch needs more
 
 struct Tile {
@@ -35,6 +36,17 @@ int launch2(hipFunction_t f, unsigned gx, unsigned gy, unsigned block, hipStream
     hipError_t e = hipModuleLaunchKernel(f, gx, gy, 1, block, 1, 1, 0, s, p, nullptr);
     if (e != hipSuccess) return fail(SE_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
     return SE_OK;
+}
+
+// Workgroups a modification for se_sl_brush: the largest box of `list` at 16 cells a
+// thread, or a fixed number where the list is in device memory; they stride over more.
+unsigned brush_blocks(const se_world& w, const se_modification* list, int n) {
+    uint64_t most = list ? 1 : 64;
+    for (int i = 0; list && i < n; i++) {
+        const uint64_t side = 2ull * (uint64_t)std::max(list[i].mod_size, 0) + 1;
+        most = std::max(most, (std::min<uint64_t>(side, w.W) / 16 + 2) * std::min<uint64_t>(side, w.H) / 256 + 1);
+    }
+    return (unsigned)std::min<uint64_t>(most, 4096);
 }
 
 }  // namespace
@@ -68,6 +80,8 @@ se_rt::SlicedShape se_rt::sliced_one_tile(uint32_t W, uint32_t H, bool wide) {
 //   1537x1111  150 steps  221 / 191 / 199 / 203
 //   4096^2      64 steps  433 / 366 / 338 / 341
 //   8192^2      64 steps    -  /  -  / 703 / 646
+// The deepest launch of one wavefront is 12 sub-steps; a run of up to 16 takes them in one
+// launch and not in two (settled 16384^2: 201 us a call, 236 in two).
 void se_rt::sliced_choice(size_t few, const SlicedKernels& K, int* kernel, uint32_t* deep) {
     const bool one_wave = K.step[0] != nullptr;
     if (few <= 2048) {
@@ -185,6 +199,14 @@ bool se_rt::sliced_pays(const se_module* m, uint32_t n) {
     return m->sliced.ok && n >= (m->table_form == 0 ? 4u : 9u);
 }
 
+// A launch of one sub-step and se_sl_brush take some 10 us and a pass over the packed
+// grid, a plain step 5 us and a pass over the ids, and it ends what is known of the
+// grids (us a call with a brush, plain step / packed: four materials 256^2 9 steps 35 / 42,
+// 1024^2 39 / 44, settled 4096^2 92 / 62, 16384^2 829 / 171).
+bool se_rt::sliced_takes_mods(const se_world* w, uint32_t n) {
+    return n > 1 && sliced_squares(w->W, w->H) >= kKnownSquares;
+}
+
 int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     *done = false;
     const SlicedKernels& K = w->mod->sliced;
@@ -193,6 +215,7 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
         int kernel;
         uint32_t deep;
         sliced_choice(sliced_squares(w->W, w->H), K, &kernel, &deep);
+        if (deep < n && n <= 16) deep = 16;
         shape = sliced_tiles(w->W, w->H, kernel, sub ? std::min(sub, deep) : deep);
     } else if (sub) {
         shape.max_sub = sub;
@@ -221,6 +244,10 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
         }
         ctx->sliced_bytes = bytes;
     }
+    ModsArg mods;
+    FewMods few{};
+    int rc = take_mods(w, mods, &few);
+    if (rc) return rc;
     *done = true;
     one.frame0 = w->frame + 1;
     one.steps = (int)n;
@@ -235,7 +262,28 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
 
     const int ptiles = sliced_pack_tiles(g), pcols = ptiles / (g.rows / 64);
     const int ucols = sliced_unpack_columns(g), utiles = ucols * (g.rows / 64);
-    int rc = launch2(K.pack, (unsigned)(ptiles + 3) / 4, 1, 256, w->stream, g, pcols, ptiles);
+    // Sleeping, from some 4 M cells on (below, a call is a chain of launches and steps that
+    // a settled tile does not shorten): settled tiles are only written, known squares are
+    // not packed or unpacked.  us a call of 12 steps of a settled world (stone below, nothing
+    // above), sleeping LDS tiles / sliced kernels without / with this: four materials 4096^2
+    // 61 / 76 / 57, 8192^2 88 / 166 / 80, 16384^2 174 / 540 / 139, twelve at 16384^2 312 / 748
+    // / 240; a dense world pays up to 1 % (8192^2 twelve 749 / 755).
+    // A caller who holds a grid's address may write it between two calls: nothing is known
+    // from one to the next then.
+    SlicedKnown known;
+    const int variant = (int)w->mod->lds.size() - 1, layout = (g.xpad << 8 | g.ypad) << 16 | pcols;
+    const size_t each = ((size_t)ptiles + 255) & ~(size_t)255;  // calm is read by whole words
+    if (w->sleep_enabled && sliced_squares(w->W, w->H) >= kKnownSquares && sleep_room(w, 2 * each) == SE_OK) {
+        if (!w->exposed) known.same = w->d_sleep[0];
+        known.was = w->d_sleep[1];
+        known.calm = w->d_sleep[1] + each;
+        known.valid = known.same && w->sleep_variant == variant && w->sleep_layout == layout;
+        one.stable = K.stable;
+        one.calm = known.calm;
+        one.calm_cols = pcols;
+    }
+    sleep_reset(w);  // until the run is enqueued
+    rc = launch2(K.pack, (unsigned)(ptiles + 3) / 4, 1, 256, w->stream, g, pcols, ptiles, known);
     int from = 0;
     for (uint32_t at = 0; at < n && !rc;) {
         const uint32_t nf = std::min(ahead, n - at);
@@ -249,17 +297,26 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
             if (m < nf - d && lead < m && (nf - d - (m - lead) + shape.max_sub - 1) / shape.max_sub ==
                                               (nf - d - m + shape.max_sub - 1) / shape.max_sub)
                 m -= lead;
+            if (at + d == 0 && mods.n > 0) m = 1;  // modifications follow the first step
             rc = launch2(K.step[shape.kernel], (unsigned)(shape.tiles_x * shape.tiles_y), 1, shape.threads, w->stream, one,
                          (const SlicedWorld*)nullptr, (const int*)nullptr, 0, (const SlicedGrid*)nullptr, from,
                          (int)(at + d), (int)m);
             from ^= 1;
+            if (at + d == 0 && mods.n > 0 && !rc) {
+                const unsigned blocks = brush_blocks(*w, mods.n <= kFewMods ? few.m : nullptr, mods.n);
+                rc = launch2(K.brush, blocks, (unsigned)mods.n, 256, w->stream, g, from, (const void*)mods.ptr, mods.n,
+                             (void*)known.calm, pcols, few);
+            }
             d += m;
         }
         at += nf;
     }
-    if (!rc) rc = launch2(K.unpack, (unsigned)(utiles + 3) / 4, 1, 256, w->stream, g, from, ucols, utiles);
+    if (!rc) rc = launch2(K.unpack, (unsigned)(utiles + 3) / 4, 1, 256, w->stream, g, from, ucols, utiles, pcols, known);
     if (rc) return rc;
-    sleep_reset(w);
+    if (known.same) {
+        w->sleep_variant = variant;
+        w->sleep_layout = layout;
+    }
     w->frame += (int32_t)n;
     w->cur ^= 1;
     return SE_OK;

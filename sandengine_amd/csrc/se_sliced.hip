@@ -156,52 +156,93 @@ __device__ __forceinline__ void se_sl_planes(const uint2* c, u32* e, u32* o) {
     }
 }
 
-__device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int m0, u32* lds) {
+// The code that all 64 x 64 cells of a wavefront's square hold, else 0xff.
+__device__ __forceinline__ u32 se_sl_uniform(const u32* e, const u32* o) {
+    u32 code = 0u, differ = 0u;
+#pragma unroll
+    for (int k = 0; k < SE_SL_K; k++) {
+        const u32 bit = (u32)__builtin_amdgcn_readfirstlane((int)e[k]) & 1u;
+        code |= bit << k;
+        differ |= (e[k] ^ (0u - bit)) | (o[k] ^ (0u - bit));
+    }
+    return __builtin_amdgcn_ballot_w64(differ != 0u) ? 0xffu : code;
+}
+
+// What a run of one world knows of its 64 x 64 squares (null: nothing is kept).
+// same: the code that both grids held all over the square when the last run ended,
+// else 0xff; all 0xff when `valid` is 0, which is so once anything else has written a
+// grid.  was: the code that the run's first grid held; calm: the same, for tiles that sleep.
+// Packing does not read a square whose code it knows, and unpacking does not write one that holds it already: a run of
+// 12 steps of a settled 16384^2 world took 540 us, of which 412 were these two passes.
+struct se_slknown {
+    unsigned char *same, *was, *calm;
+    int valid;
+};
+
+__device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int m0, u32* lds, const se_slknown& known,
+                                                int sq) {
     const int lane = (int)(threadIdx.x & 63);
     const int x = 16 * se_sl_bcol(g, wc) - g.xpad + 4 * (lane & 15);
     const int y0 = m0 - g.ypad, xw = 16 * se_sl_bcol(g, wc) - g.xpad;
-    uint4 v[16];
-    if (y0 >= 0 && y0 + 64 <= g.H && xw >= 0 && xw + 64 <= g.W) {  // all of the tile inside the world
-        const u32* s = se_sl_ptr<const u32>(g.in) + (size_t)(y0 + (lane >> 4)) * g.pitch + x;
+    const bool inside = y0 >= 0 && y0 + 64 <= g.H && xw >= 0 && xw + 64 <= g.W;  // all of the tile inside the world
+    const u32 code = known.valid && inside ? known.same[sq] : 0xffu;
+    u32 e[SE_SL_K], o[SE_SL_K];
+    if (code != 0xffu) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = se_load_nt(s + (size_t)(4 * i) * g.pitch);
+        for (int k = 0; k < SE_SL_K; k++) e[k] = o[k] = 0u - ((code >> k) & 1u);
+        if (lane == 0) known.was[sq] = known.calm[sq] = (unsigned char)code;
     } else {
+        uint4 v[16];
+        if (inside) {
+            const u32* s = se_sl_ptr<const u32>(g.in) + (size_t)(y0 + (lane >> 4)) * g.pitch + x;
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = se_load_nt(s + (size_t)(4 * i) * g.pitch);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int y = y0 + 4 * i + (lane >> 4);
+                const bool in = y >= 0 && y < g.H && x >= 0 && x < g.W;
+                uint4 t = *reinterpret_cast<const uint4*>(se_sl_ptr<const u32>(g.in) + (in ? (size_t)y * g.pitch + x : 0));
+                t.x = in ? t.x : SE_WALLID;
+                t.y = in && x + 1 < g.W ? t.y : SE_WALLID;
+                t.z = in && x + 2 < g.W ? t.z : SE_WALLID;
+                t.w = in && x + 3 < g.W ? t.w : SE_WALLID;
+                v[i] = t;
+            }
+        }
+        bool exact = true;  // no id beyond the materials: the codes say what the grid holds
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            const int y = y0 + 4 * i + (lane >> 4);
-            const bool in = y >= 0 && y < g.H && x >= 0 && x < g.W;
-            uint4 t = *reinterpret_cast<const uint4*>(se_sl_ptr<const u32>(g.in) + (in ? (size_t)y * g.pitch + x : 0));
-            t.x = in ? t.x : SE_WALLID;
-            t.y = in && x + 1 < g.W ? t.y : SE_WALLID;
-            t.z = in && x + 2 < g.W ? t.z : SE_WALLID;
-            t.w = in && x + 3 < g.W ? t.w : SE_WALLID;
-            v[i] = t;
+            const u32 mx = max(max(v[i].x, v[i].y), max(v[i].z, v[i].w));
+            u32 q;
+            if (__builtin_expect(mx >= SE_NMAT, 0)) {
+                q = se_pack4(se_decode(v[i].x), se_decode(v[i].y), se_decode(v[i].z), se_decode(v[i].w));
+                exact = false;
+            } else {
+                q = se_pack4(v[i].x, v[i].y, v[i].z, v[i].w);
+            }
+            lds[(4 * i + (lane >> 4)) * 17 + (lane & 15)] = se_sl_codes(q);
+        }
+        __builtin_amdgcn_wave_barrier();
+        u32 q[16], de[8], dd[8];
+#pragma unroll
+        for (int m = 0; m < 16; m++) q[m] = lds[lane * 17 + m];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            se_sl_bytes4(q[t], q[4 + t], q[8 + t], q[12 + t]);
+            de[2 * t] = q[t];
+            dd[2 * t] = q[4 + t];
+            de[2 * t + 1] = q[8 + t];
+            dd[2 * t + 1] = q[12 + t];
+        }
+        se_sl_slice(de, e);
+        se_sl_slice(dd, o);
+        if (known.was != nullptr) {
+            const u32 all = se_sl_uniform(e, o);
+            const bool keep = inside && __builtin_amdgcn_ballot_w64(!exact) == 0;
+            if (lane == 0) known.was[sq] = known.calm[sq] = (unsigned char)(keep ? all : 0xffu);
         }
     }
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const u32 mx = max(max(v[i].x, v[i].y), max(v[i].z, v[i].w));
-        u32 q;
-        if (__builtin_expect(mx >= SE_NMAT, 0))
-            q = se_pack4(se_decode(v[i].x), se_decode(v[i].y), se_decode(v[i].z), se_decode(v[i].w));
-        else
-            q = se_pack4(v[i].x, v[i].y, v[i].z, v[i].w);
-        lds[(4 * i + (lane >> 4)) * 17 + (lane & 15)] = se_sl_codes(q);
-    }
-    __builtin_amdgcn_wave_barrier();
-    u32 q[16], e[SE_SL_K], o[SE_SL_K], de[8], dd[8];
-#pragma unroll
-    for (int m = 0; m < 16; m++) q[m] = lds[lane * 17 + m];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        se_sl_bytes4(q[t], q[4 + t], q[8 + t], q[12 + t]);
-        de[2 * t] = q[t];
-        dd[2 * t] = q[4 + t];
-        de[2 * t + 1] = q[8 + t];
-        dd[2 * t + 1] = q[12 + t];
-    }
-    se_sl_slice(de, e);
-    se_sl_slice(dd, o);
     const int row = m0 + lane;
     const bool around_y = row < g.ypad || row >= g.ypad + g.H;
     uint2 cols[4];
@@ -217,7 +258,8 @@ __device__ __forceinline__ void se_sl_pack_tile(const se_slgrid& g, int wc, int 
 }
 
 // packed grid `from` -> u32 grid (the cells of the world only)
-__device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, int wc, int m0, u32* lds) {
+__device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, int wc, int m0, u32* lds,
+                                                  const se_slknown& known, int sq) {
     const int lane = (int)(threadIdx.x & 63);
     u32 e[SE_SL_K], o[SE_SL_K], de[8], dd[8], q[16];
     uint2 cols[4];
@@ -226,6 +268,13 @@ __device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, 
         cols[c] = se_sl_bcol(g, wc) + c < g.bcols ? *se_sl_at(g, from, se_sl_bcol(g, wc) + c, m0 + lane)
                                                    : make_uint2(0u, 0u);
     se_sl_planes(cols, e, o);
+    if (known.same != nullptr) {
+        const u32 was = known.was[sq], all = was != 0xffu ? se_sl_uniform(e, o) : 0xffu;  // 0xff: not all inside the world
+        const bool stays = all != 0xffu && was == all;  // the first grid holds it
+        const bool held = stays && known.valid && known.same[sq] == all;
+        if (lane == 0) known.same[sq] = (unsigned char)(stays ? all : 0xffu);
+        if (held) return;
+    }
     se_sl_unslice(e, de);
     se_sl_unslice(o, dd);
 #pragma unroll
@@ -258,19 +307,21 @@ __device__ __forceinline__ void se_sl_unpack_tile(const se_slgrid& g, int from, 
 }
 
 // wtiles columns of 64 cells, from the one left of the world on (se_sl_pack: the
-// margin is packed too), tiles in all
-extern "C" __global__ __launch_bounds__(256) void se_sl_pack(se_slgrid g, int wtiles, int tiles) {
+// margin is packed too), tiles in all; unpacking leaves that column out
+extern "C" __global__ __launch_bounds__(256) void se_sl_pack(se_slgrid g, int wtiles, int tiles, se_slknown known) {
     __shared__ u32 lds[4][64 * 17];
-    const int wave = (int)(threadIdx.x >> 6), t = (int)blockIdx.x * 4 + wave;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), t = (int)blockIdx.x * 4 + wave;
     if (t >= tiles) return;
-    se_sl_pack_tile(g, t % wtiles - 1, (t / wtiles) * 64, lds[wave]);
+    se_sl_pack_tile(g, t % wtiles - 1, (t / wtiles) * 64, lds[wave], known, t);
 }
 
-extern "C" __global__ __launch_bounds__(256) void se_sl_unpack(se_slgrid g, int from, int wtiles, int tiles) {
+extern "C" __global__ __launch_bounds__(256) void se_sl_unpack(se_slgrid g, int from, int wtiles, int tiles, int packed_wtiles,
+                                                               se_slknown known) {
     __shared__ u32 lds[4][64 * 17];
-    const int wave = (int)(threadIdx.x >> 6), t = (int)blockIdx.x * 4 + wave;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), t = (int)blockIdx.x * 4 + wave;
     if (t >= tiles) return;
-    se_sl_unpack_tile(g, from, t % wtiles, (t / wtiles) * 64, lds[wave]);
+    se_sl_unpack_tile(g, from, t % wtiles, (t / wtiles) * 64, lds[wave], known,
+                      (t / wtiles) * packed_wtiles + t % wtiles + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -723,8 +774,42 @@ __device__ __forceinline__ void se_sl_tile(const se_slgrid& g, int from, int tx,
 struct se_slworld {  // == SlicedWorld (se_sliced.hpp)
     se_slgrid g;
     int frame0, steps, tiles_x, side, halo, group;
-    int result, pad;  // packed grid that holds the world after its last launch
+    int result;  // packed grid that holds the world after its last launch
+    u32 stable;  // codes of tiles that may sleep (se_sl_sleeps); 0 in a batch
+    u64 calm;    // squares' codes
+    int calm_cols, pad;
 };
+
+// Does the tile sleep through the launch?  Then its kept cells are written as they are.
+// A change travels a cell a step: a tile where all squares within `done` cells of it (it has
+// the launch's halo in it) held one code when the run began (calm, by packing; a
+// modification ends it), and no rule changes a block of four such cells, is as it was.
+// Others are mostly found out by the square at their middle, one scalar load.  Kept apart
+// from the tile's own loads and registers: a test of the cells once they are here, or one
+// path to the stores for both, cost a launch of a dense 16384^2 world 3 to 8 %.
+template <int NW, int R, int S>
+__device__ __forceinline__ bool se_sl_sleeps(const se_slworld& v, int from, int tx, int ty, int done) {
+    constexpr int W = 64 * NW * S, H = 64 * R;
+    const int bc0 = tx * (4 * NW * S - 2 * v.side), row0 = ty * (H - 2 * v.halo), x = 16 * bc0 - v.g.xpad;
+    const int mid = ((row0 + H / 2) >> 6) * v.calm_cols + ((x + W / 2) >> 6) + 1;  // inside the packed grid
+    const u32 code = ((const __attribute__((address_space(4))) u32*)v.calm)[mid >> 2] >> (8 * (mid & 3)) & 0xffu;
+    if (code == 0xffu || !((v.stable >> code) & 1u)) return false;
+    const int ca = (x - done) >> 6, cb = (x + W - 1 + done) >> 6, ra = (row0 - done) >> 6, rb = (row0 + H - 1 + done) >> 6;
+    if (ca < 0 || cb + 1 >= v.calm_cols || ra < 0 || 64 * rb >= v.g.rows) return false;
+    const unsigned char* calm = se_sl_ptr<const unsigned char>(v.calm);
+    const int wide = cb - ca + 1, n = wide * (rb - ra + 1);
+    bool other = false;
+    for (int i = (int)(threadIdx.x & 63); i < n; i += 64) other |= calm[(ra + i / wide) * v.calm_cols + ca + i % wide + 1] != code;
+    if (__builtin_amdgcn_ballot_w64(other)) return false;
+    u32 planes = 0u;
+#pragma unroll
+    for (int k = 0; k < SE_SL_K; k++) planes |= (code >> k) & 1u ? 0xffu << (8 * k) : 0u;
+    const int pairs = H / 2 - v.halo, columns = 4 * NW * S - 2 * v.side;  // pairs of rows
+    for (int i = (int)threadIdx.x; i < columns * pairs; i += 64 * S)
+        *reinterpret_cast<uint4*>(se_sl_at(v.g, from ^ 1, bc0 + v.side + i / pairs, row0 + v.halo + 2 * (i % pairs))) =
+            make_uint4(planes, planes, planes, planes);
+    return true;
+}
 
 // Steps [done, done + k) of `one` (n = 0), or of worlds [0, n) (longest first, their
 // tiles counted by prefix); one workgroup per tile.
@@ -738,6 +823,8 @@ struct se_slworld {  // == SlicedWorld (se_sliced.hpp)
         int tile;                                                                                              \
         if (n == 0) {                                                                                          \
             tile = se_xcd_tile((int)blockIdx.x, (int)gridDim.x);                                               \
+            if (one.stable != 0u &&                                                                            \
+                se_sl_sleeps<NW, R, S>(one, from, tile % one.tiles_x, tile / one.tiles_x, done)) return;       \
         } else {                                                                                               \
             const int w = se_owner(prefix, n, (int)blockIdx.x);                                                \
             tile = (int)blockIdx.x - prefix[w];                                                                \
@@ -769,6 +856,60 @@ SE_SL_STEP(2, 2, 1, 4, 3, 2x2)
 SE_SL_STEP(4, 2, 1, 2, 3, 4x2)
 #endif
 
+// ---------------------------------------------------------------------------
+// Modifications of a run's first step, on packed grid `to` after that step (one launch of
+// one sub-step).  blockIdx.y is a modification; a thread takes 16 cells of a row at a time
+// of its box, unless an earlier one's box has them too, and looks all modifications up for
+// each cell as the plain kernel does.  12 steps of a settled 16384^2 world with a brush take
+// 178 us, with the first step by the plain kernel instead, a pass over the ids that ends
+// what is known of them, 852, and with the LDS kernels 211.
+// ---------------------------------------------------------------------------
+struct se_slbrush_args {  // the arguments as they lie in the kernel's argument segment
+    se_slgrid g;
+    int to;
+    const se_mod* mods;
+    int nmods;
+    unsigned char* calm;
+    int cols;
+    se_few few;
+};
+
+extern "C" __global__ __launch_bounds__(256) void se_sl_brush(se_slgrid g, int to, const se_mod* __restrict__ list,
+                                                              int nmods, unsigned char* calm, int cols, se_few) {
+    const se_cmods few = (se_cmods)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() +
+                                    __builtin_offsetof(se_slbrush_args, few));
+    const se_cmods mods = nmods <= SE_PLAIN_MODS ? few : (se_cmods)list;
+    const int i = (int)blockIdx.y;
+    const long r = max(mods[i].size, 0), mx = mods[i].x, my = mods[i].y;
+    const long xa = max(mx - r, 0l), xb = min(mx + r, (long)g.W - 1), ya = max(my - r, 0l), yb = min(my + r, (long)g.H - 1);
+    if (xa > xb || ya > yb) return;
+    const int first = ((int)xa + g.xpad) >> 4, wide = (((int)xb + g.xpad) >> 4) - first + 1;
+    const u64 units = (u64)wide * (u64)(yb - ya + 1);
+    for (u64 u = (u64)blockIdx.x * 256 + threadIdx.x; u < units; u += (u64)gridDim.x * 256) {
+        const int bc = first + (int)(u % (u64)wide), y = (int)ya + (int)(u / (u64)wide), x0 = 16 * bc - g.xpad;
+        if (se_mods_touch(mods, i, x0, x0 + 15, y, y)) continue;
+        uint2* p = se_sl_at(g, to, bc, y + g.ypad);
+        uint2 v = *p;
+#pragma unroll 1
+        for (int c = 0; c < 16; c++) {
+            const int x = x0 + c;
+            const int id = x >= 0 && x < g.W ? se_mod_override(mods, nmods, x, y) : -1;
+            if (id < 0) continue;
+            const u32 code = se_sl_codes((u32)id) & 0xffu;
+            u32 w = c & 1 ? v.y : v.x;
+#pragma unroll
+            for (int k = 0; k < SE_SL_K; k++) {
+                const u32 bit = 1u << (8 * k + (c >> 1));
+                w = (code >> k) & 1u ? w | bit : w & ~bit;
+            }
+            if (c & 1) v.y = w;
+            else v.x = w;
+        }
+        *p = v;
+        if (calm != nullptr) calm[((y + g.ypad) >> 6) * cols + (x0 >> 6) + 1] = 0xffu;  // 16 cells of one square
+    }
+}
+
 // Batch forms of the other kernels: prefix sums count 64 x 64 tiles (pack, unpack).
 extern "C" __global__ __launch_bounds__(256) void se_sl_bpack(const se_slworld* __restrict__ worlds,
                                                               const int* __restrict__ prefix, int n) {
@@ -778,7 +919,7 @@ extern "C" __global__ __launch_bounds__(256) void se_sl_bpack(const se_slworld* 
     const int w = se_owner(prefix, n, t), i = t - prefix[w];
     const se_slgrid g = worlds[w].g;
     const int cols = 1 + (g.bcols - (g.xpad >> 4) + 3) / 4;
-    se_sl_pack_tile(g, i % cols - 1, (i / cols) * 64, lds[wave]);
+    se_sl_pack_tile(g, i % cols - 1, (i / cols) * 64, lds[wave], se_slknown{nullptr, nullptr, nullptr, 0}, 0);
 }
 
 extern "C" __global__ __launch_bounds__(256) void se_sl_bunpack(const se_slworld* __restrict__ worlds,
@@ -789,7 +930,7 @@ extern "C" __global__ __launch_bounds__(256) void se_sl_bunpack(const se_slworld
     const int w = se_owner(prefix, n, t), i = t - prefix[w];
     const se_slgrid g = worlds[w].g;
     const int cols = 1 + (g.bcols - (g.xpad >> 4) + 3) / 4;  // as packing: the first column holds no cells
-    if (i % cols > 0) se_sl_unpack_tile(g, worlds[w].result, i % cols - 1, (i / cols) * 64, lds[wave]);
+    if (i % cols > 0) se_sl_unpack_tile(g, worlds[w].result, i % cols - 1, (i / cols) * 64, lds[wave], se_slknown{nullptr, nullptr, nullptr, 0}, 0);
 }
 
 // The words of all groups in one row of workgroups (prefix counts 256 of them): a grid

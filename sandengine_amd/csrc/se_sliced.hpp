@@ -27,9 +27,17 @@ static_assert(sizeof(SlicedGrid) == 104, "se_slgrid layout");
 struct SlicedWorld {
     SlicedGrid g;
     int frame0 = 0, steps = 0, tiles_x = 0, side = 0, halo = 0, group = 0;
-    int result = 0, pad = 0;
+    int result = 0;
+    uint32_t stable = 0;
+    unsigned char* calm = nullptr;
+    int calm_cols = 0, pad = 0;
 };
-static_assert(sizeof(SlicedWorld) == 136, "se_slworld layout");
+static_assert(sizeof(SlicedWorld) == 152, "se_slworld layout");
+
+struct SlicedKnown {  // == se_slknown in se_sliced.hip
+    unsigned char *same = nullptr, *was = nullptr, *calm = nullptr;
+    int valid = 0;
+};
 
 // How a world is cut into tiles of one step kernel.
 struct SlicedShape {
@@ -71,8 +79,11 @@ bool sliced_pays(const se_module* m, uint32_t n);
 // Wavefronts (64 columns x 64 rows each) that pack and that unpack a world.
 int sliced_pack_tiles(const SlicedGrid& g);
 int sliced_unpack_columns(const SlicedGrid& g);
-// Advances w by n steps (no clearing frame and no queued modifications among
-// them), launches of up to `sub` sub-steps.  *done = false and nothing enqueued
+// Do the modifications of a run's first step go into the packed grid (else that step is
+// for the plain kernel)?
+bool sliced_takes_mods(const se_world* w, uint32_t n);
+// Advances w by n steps (no clearing frame among them; queued modifications follow the
+// first), launches of up to `sub` sub-steps.  *done = false and nothing enqueued
 // when the scratch memory cannot be had.
 int sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done);
 
