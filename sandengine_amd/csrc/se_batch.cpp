@@ -462,7 +462,12 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
         if (vi < 0 || vi >= (int)mod->lds.size()) return fail(SE_ERR_ARG, "LDS variant out of range");
         uint32_t most = 0;
         for (auto& it : g.second) most = std::max(most, it.second);
-        const bool want = mod->lds[vi].first.sliced || (!chosen && la != 1 && se_rt::sliced_pays(mod, most));
+        bool want = mod->lds[vi].first.sliced;
+        if (!want && !chosen && la != 1 && mod->sliced.ok) {
+            std::vector<se_rt::SlicedLoad> loads;
+            for (auto& it : g.second) loads.push_back({it.first->W, it.first->H, it.second, it.first->frame});
+            want = se_rt::sliced_batch_pays(mod->sliced, loads);
+        }
         if (want && most > 0) {
             std::unique_ptr<SlicedPlan> one(new SlicedPlan()), many(new SlicedPlan());
             one->mod = many->mod = mod;

@@ -1313,7 +1313,8 @@ std::string lds_kernel_name(const LdsVariant& v) {
 
 std::string hip_program_source(const ParsingResult& r, const std::vector<LdsVariant>& lds, bool allow_ctable,
                                uint64_t ct_x_words, SlicedInfo* sliced) {
-    std::string s = hip_rules_source(r, nullptr, allow_ctable, ct_x_words);
+    HipGenInfo form;
+    std::string s = hip_rules_source(r, &form, allow_ctable, ct_x_words);
     s += "\n";
     s += kKernelTemplates;
     s += "\n";
@@ -1324,6 +1325,10 @@ std::string hip_program_source(const ParsingResult& r, const std::vector<LdsVari
         SlicedInfo local;
         SlicedInfo& sl = sliced ? *sliced : local;
         const std::string rules = hip_sliced_source(r, sl);
+        // A network this large is never the faster one beside a transition table, whose
+        // cost does not grow with the rules (se_sliced.cpp: 1661 tables, 4096^2, 64 steps 920 us
+        // and 586 by the table), and takes seconds to compile.
+        if (sl.ok && (form.table || form.ctable) && sl.tables > 1000) sl = SlicedInfo();
         if (sl.ok) s += rules + kSlicedTemplates;
     }
     return s;

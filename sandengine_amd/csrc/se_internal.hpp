@@ -61,10 +61,20 @@ struct FillSpec {  // == se_fillspec in se_kernels.hip
     uint32_t ids[16], thr[16];
 };
 
+// What the choice between a rule set's kernels goes by (se_sliced.cpp).
+struct StepCost {
+    int form = 0;           // of the LDS kernels: 0 generated chain, 1 full table, 2 coded table
+    bool wall_kept = true;  // no block changes a WALL cell
+    int tables = 0;         // three-input tables of the sliced form
+    int hash_ops = 0;       // instructions that hash a block: 9 a lane, 2 a plane
+    bool one_wave = true;   // tiles of one wavefront are there (up to three planes)
+};
+
 // The sliced kernels of a module (se_sliced.hip); ok false where the rule set has
 // no sliced form.
 struct SlicedKernels {
     bool ok = false;
+    StepCost cost;
     int planes = 0, classes = 0;  // bit planes of a cell, hash planes of a frame
     uint32_t stable = 0;          // SlicedInfo::stable
     hipFunction_t pack = nullptr, unpack = nullptr, hash = nullptr, brush = nullptr;

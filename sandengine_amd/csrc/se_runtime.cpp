@@ -440,6 +440,13 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         K.planes = info.sliced.planes;
         K.classes = (int)info.sliced.classes.size();
         K.stable = info.sliced.stable;
+        K.cost.form = m->table_form;
+        K.cost.wall_kept = info.sliced.wall_kept;
+        K.cost.tables = info.sliced.tables;
+        unsigned lanes = 0;
+        for (auto& c : info.sliced.classes) lanes |= 1u << c.first;
+        K.cost.hash_ops = 9 * __builtin_popcount(lanes) + 2 * K.classes;
+        K.cost.one_wave = K.step[0] != nullptr;
         K.ok = true;
         // listed after the LDS instantiations (never the default among them)
         m->lds.push_back({{128, 128, 32, 128, true}, K.step[2]});
@@ -652,7 +659,7 @@ int blocked_steps(se_world* w, uint32_t nsteps, uint32_t sub) {
     }
     auto* v = pick_lds(w, sub);
     if (!v) return fail(SE_ERR_ARG, "no LDS variant supports " + std::to_string(sub) + " sub-steps");
-    if (v->first.sliced || (w->lds_variant < 0 && se_rt::sliced_pays(w->mod.get(), nsteps))) {
+    if (v->first.sliced || (w->lds_variant < 0 && se_rt::sliced_pays(w->mod->sliced, w->W, w->H, nsteps))) {
         // the clearing frame is a step of its own, and so are modifications where a plain
         // step is faster than the launches that take them into the packed grid
         if (nsteps && (w->frame + 1 == 1 || (!w->pending.empty() && !se_rt::sliced_takes_mods(w, nsteps)))) {

@@ -9,6 +9,7 @@
 #include "se_sliced.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 using se_rt::DeviceGuard;
 using se_rt::fail;
@@ -188,15 +189,163 @@ se_rt::SlicedAhead se_rt::sliced_ahead(const SlicedShape& s, SlicedGrid g, int32
     return a;
 }
 
-// Packing, hashing and unpacking cost three launches more than the LDS kernels
-// have, and from the largest worlds a pass over the grid.  The LDS kernels' default
-// tile advances 8 steps in one launch and stays for those; the generated chain,
-// where no table fits, does a step in the time of ten (measured per call, LDS
-// against sliced, us: four materials 256^2 8 steps 22 and 19, 12 steps 37 and 20;
-// 4096^2 46 and 55, 83 and 64; 16384^2 427 and 567, 831 and 607; twelve at 8192^2
+// ---------------------------------------------------------------- LDS or sliced kernels
+// Packing, hashing and unpacking cost three launches more than the LDS kernels have, and
+// from the largest worlds a pass over the grid.  The LDS kernels' default tile advances 8
+// steps in one launch and stays for those; the generated chain, where no table fits, does a
+// step in the time of ten (measured per call, LDS against sliced, us: four materials 4096^2
+// 8 steps 46 and 55, 12 steps 83 and 64; 16384^2 427 and 567, 831 and 607; twelve at 8192^2
 // 226 and 223, 368 and 261; feature rules 4096^2 2 steps 52 and 53, 4 steps 88 and 66).
-bool se_rt::sliced_pays(const se_module* m, uint32_t n) {
-    return m->sliced.ok && n >= (m->table_form == 0 ? 4u : 9u);
+// From there on the sliced kernels are ahead in worlds of at least 128 cells a side with
+// networks of up to 300 tables (1500^2 to 12000^2, 3000x8192, 200x40000 and the like, 9 to 32
+// steps: 1.1 to 2.2 times faster with four and twelve materials).  Elsewhere the path is the
+// one of the smaller estimate, which goes by times like these:
+//   * worlds inside one LDS tile take all their steps in one launch (four materials, LDS /
+//     sliced: 2x2 9 steps 19 / 27 us, 96 steps 56 / 53; 32x32 16 steps 27 / 28, 24 33 / 31;
+//     64x64 9 steps 26 / 28, 12 29 / 28; 90x90 9 steps 31 / 28);
+//   * worlds a few rows high fill a tenth of the sliced tiles, whose planes are hashed all
+//     the same (20000x16 16 steps 28 / 34, 32 45 / 43; chain form 20000x1 128 steps 172 / 219);
+//   * large networks beside a table (586 tables, 4096^2, 64 steps 487 / 475; 1661 565 / 901);
+//   * batches whose worlds all start at different frames share no planes (2048 worlds of 64^2,
+//     256 steps 956 / 2325 us, and 966 / 408 at one frame).
+// Fitted to some 700 calls of seven rule sets; the estimates' choice costs at most a third
+// more than the better path there, mostly in worlds a few rows high.
+namespace {
+
+bool one_lds_tile(uint32_t W, uint32_t H) { return W <= 112 && H <= 112; }
+
+// The generated chain grows with the rules, as the network does.
+double chain_scale(const se_rt::StepCost& c) { return c.form == 0 ? (c.tables + 100) / 200.0 : 1.0; }
+
+// us a step of a world alone: a serial chain of LDS reads and barriers, longer by the tile's rows
+double lds_latency(const se_rt::StepCost& c, uint32_t W, uint32_t H) {
+    static const double one[3][2] = {{.75, .060}, {.40, .0105}, {1.05, .0145}};
+    static const double many[3][2] = {{1.2, .056}, {.85, .0155}, {1.7, .018}};
+    const double t = one_lds_tile(W, H) ? one[c.form][0] + one[c.form][1] * std::sqrt((double)W * H)
+                                        : many[c.form][0] + many[c.form][1] * std::min(H, 112u);
+    return chain_scale(c) * (c.form == 1 && !c.wall_kept ? 1.15 : 1.0) * t;
+}
+
+// us a step of a world that shares a full device with others
+double lds_work(const se_rt::StepCost& c, uint32_t W, uint32_t H) {
+    static const double tile[3][2] = {{.004, 8e-7}, {.0008, 2.0e-7}, {.0027, 2.6e-7}};
+    const double* t = tile[c.form];
+    if (one_lds_tile(W, H)) return chain_scale(c) * (t[0] + t[1] * W * H);
+    return chain_scale(c) * (t[0] + t[1] * 16384) * ((W + 111) / 112) * ((H + 111) / 112);
+}
+
+// n steps, in steps of a long run: beyond one tile they come in launches of up to 8, and two
+// fifths of a full one's time are the launch's own
+double lds_steps(uint32_t W, uint32_t H, uint32_t n) {
+    return one_lds_tile(W, H) ? n : 3.2 * ((n + 7) / 8) + .6 * n;
+}
+
+double sliced_latency(const se_rt::StepCost& c, bool one) {
+    return (one ? .16 : .24) + .0021 * c.tables + (c.form == 0 && !c.wall_kept ? .06 : 0);
+}
+
+// us to hash a frame for planes of that geometry, n frames together
+double hash_time(const se_rt::StepCost& c, se_rt::SlicedGrid g, uint32_t n) {
+    n = std::min(n, 256u);
+    se_rt::sliced_hash_layout(g, 1, n, 1);
+    return .028e-6 * c.hash_ops * 32.0 * g.hash_words * g.hash_sets / n;
+}
+
+}  // namespace
+
+bool se_rt::sliced_pays(const SlicedKernels& K, uint32_t W, uint32_t H, uint32_t n) {
+    const StepCost& c = K.cost;
+    if (!K.ok || n < (c.form == 0 ? 4u : 9u)) return false;
+    if (std::min(W, H) >= 128 && (c.form == 0 || c.tables <= 300)) return true;
+    SlicedShape s = sliced_one_tile(W, H, true);
+    if (!s.nw) {
+        int kernel;
+        uint32_t deep;
+        sliced_choice(sliced_squares(W, H), K, &kernel, &deep);
+        s = sliced_tiles(W, H, kernel, deep);
+    }
+    SlicedGrid g;
+    sliced_geometry(s, W, H, g);
+    const double cells = 1e-6 * W * H, area = 16e-6 * g.bcols * g.rows;
+    const double tiles = 12544e-6 * ((W + 111) / 112) * ((H + 111) / 112) * (std::min(H, 112u) + 16) / 128;
+    const double work[3] = {1.0, c.wall_kept ? .20 : .42, .42};  // LDS kernels, us a step and M cells of its tiles
+    const double alone = lds_latency(c, W, H), full = chain_scale(c) * work[c.form] * tiles;
+    const double lds = (one_lds_tile(W, H) ? 15 : 12) + lds_steps(W, H, n) * (one_lds_tile(W, H) ? alone : std::hypot(alone, full));
+    const double step = std::max(sliced_latency(c, !s.halo), (.0003 * c.tables + .006) * area);
+    return 25 + (s.halo ? 2 : 0) + n * (step + hash_time(c, g, n)) + 1.55 * cells < lds;
+}
+
+bool se_rt::sliced_batch_pays(const SlicedKernels& K, const std::vector<SlicedLoad>& worlds) {
+    const StepCost& c = K.cost;
+    uint32_t most = 0;
+    size_t squares = 0;
+    for (auto& w : worlds) {
+        most = std::max(most, w.n);
+        if (w.n) squares += sliced_squares(w.W, w.H);
+    }
+    if (!K.ok || most < (c.form == 0 ? 4u : 9u)) return false;
+    int kernel;
+    uint32_t deep;
+    sliced_choice(squares, K, &kernel, &deep);
+    // The lists that advance side by side: worlds beyond one tile, and the others.  Worlds
+    // that start at the same frame share planes, as large as the largest needs.
+    struct List {
+        SlicedGrid most;      // extents
+        uint32_t n = 0;       // steps
+        size_t worlds = 0, groups = 0;
+        double hash = 0;  // us, were each world's planes its own
+    } lists[2];
+    size_t slots = 64;
+    while (slots < 4 * worlds.size()) slots *= 2;
+    std::vector<int32_t> seen[2];  // first frames, a hash table
+    SlicedLoad last{0, 0, 0, 0};
+    SlicedGrid g;
+    bool one = false;
+    double t = 0, cells = 0, lds_all = 0, lds_chain = 0, sliced_all = 0, sliced_chain = 0, count = 0;
+    for (auto& w : worlds) {
+        if (!w.n) continue;
+        if (w.W != last.W || w.H != last.H || w.n != last.n) {  // runs of equal worlds
+            last = w;
+            SlicedShape s = sliced_one_tile(w.W, w.H, false);
+            one = s.nw != 0;
+            if (!one) s = sliced_tiles(w.W, w.H, kernel, deep);
+            g = SlicedGrid();
+            sliced_geometry(s, w.W, w.H, g);
+            t = hash_time(c, g, w.n);
+        }
+        List& l = lists[one];
+        if (!l.worlds) l.most = g;
+        l.most.bcols = std::max(l.most.bcols, g.bcols);
+        l.most.brows = std::max(l.most.brows, g.brows);
+        l.n = std::max(l.n, w.n);
+        l.worlds++;
+        l.hash += w.n * t;
+        std::vector<int32_t>& at = seen[one];
+        if (at.empty()) at.assign(slots, INT32_MIN);
+        size_t i = (uint32_t)w.frame * 2654435761u & (slots - 1);
+        while (at[i] != INT32_MIN && at[i] != w.frame) i = (i + 1) & (slots - 1);
+        l.groups += at[i] == INT32_MIN;
+        at[i] = w.frame;
+        count++;
+        cells += 1e-6 * w.W * w.H;
+        const double steps = lds_steps(w.W, w.H, w.n);
+        lds_all += steps * lds_work(c, w.W, w.H);
+        lds_chain = std::max(lds_chain, steps * lds_latency(c, w.W, w.H));
+        sliced_all += w.n * c.tables * (one ? 3.9e-6 : 3.5e-6 * sliced_squares(w.W, w.H));
+        sliced_chain = std::max(sliced_chain, w.n * sliced_latency(c, one));
+    }
+    double host = 0;
+    for (int k = 0; k < 2; k++) {
+        const List& l = lists[k];
+        if (!l.worlds) continue;
+        const double us = l.groups == 1 ? l.n * hash_time(c, l.most, l.n) : l.hash * l.groups / l.worlds;
+        sliced_all += us * (k ? 1.5 : 1.0);  // one tile: few words a set, waiting workgroups
+        const double bytes = us / (.028e-6 * c.hash_ops) / 8 * K.classes;
+        const double chunks = k ? std::max(1.0, bytes / (64 << 20)) : l.n <= 64 ? 1 : l.n <= 192 ? 2 : 2 + (l.n + 63) / 256;
+        host += l.groups * (.08 + .12 * chunks) + (k ? 0 : 12 * (chunks - 1));
+    }
+    return 88 + .07 * count + host + std::max(sliced_chain, sliced_all) + 1.5 * cells <
+           76 + .045 * count + std::hypot(lds_chain, lds_all);
 }
 
 // A launch of one sub-step and se_sl_brush take some 10 us and a pass over the packed

@@ -75,7 +75,13 @@ struct SlicedAhead {
 SlicedAhead sliced_ahead(const SlicedShape& s, SlicedGrid g, int32_t frame0, uint32_t n, int classes);
 
 // Is the sliced path taken for n steps of a world whose caller chose no variant?
-bool sliced_pays(const se_module* m, uint32_t n);
+bool sliced_pays(const SlicedKernels& K, uint32_t W, uint32_t H, uint32_t n);
+// And for the worlds of a batch that share the rule set?
+struct SlicedLoad {
+    uint32_t W, H, n;
+    int32_t frame;
+};
+bool sliced_batch_pays(const SlicedKernels& K, const std::vector<SlicedLoad>& worlds);
 // Wavefronts (64 columns x 64 rows each) that pack and that unpack a world.
 int sliced_pack_tiles(const SlicedGrid& g);
 int sliced_unpack_columns(const SlicedGrid& g);
