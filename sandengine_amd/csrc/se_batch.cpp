@@ -82,11 +82,16 @@ struct se_batch {
     std::map<se_module*, Tuned> tuned;
     hipStream_t streams[8] = {};
     // records, packed grids and hash planes of the sliced plans, kept from run to run
-    // and freed by se_batch_clear (a run ends with the device idle)
-    void* arena = nullptr;
-    size_t arena_bytes = 0;
+    // (which end with the device idle), freed by se_batch_clear or when another allocation
+    // of the device fails
+    std::shared_ptr<se_rt::Pool> pool;
+    se_rt::Pool::Block arena;
     ~se_batch() {
-        (void)hipFree(arena);
+        if (pool) {
+            std::lock_guard<std::mutex> lk(pool->mu);
+            pool->arenas.erase(std::find(pool->arenas.begin(), pool->arenas.end(), &arena));
+            se_rt::Pool::drop(arena);
+        }
         for (auto s : streams)
             if (s) (void)hipStreamDestroy(s);
     }
@@ -437,6 +442,13 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
     se_ctx* ctx = b->ctx;
     std::map<se_module*, std::vector<std::pair<se_world*, uint32_t>>> groups;
     for (auto& it : work) groups[it.first->mod.get()].push_back(it);
+    struct Release {  // after the streams are drained: the arena may be given back again
+        se_batch* b;
+        ~Release() {
+            std::lock_guard<std::mutex> lk(b->pool->mu);
+            b->arena.busy = false;
+        }
+    } release{b};
     std::vector<std::unique_ptr<Plan>> plans;
     std::vector<std::unique_ptr<SlicedPlan>> sliced;
     size_t squares = 0;  // of the whole batch: its lists run side by side
@@ -489,20 +501,22 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
     if (!sliced.empty()) {
         size_t bytes = 0;
         for (auto& p : sliced) bytes += p->meta_bytes + p->packed_bytes + p->hash_bytes;
-        if (bytes > b->arena_bytes) {
-            bytes += bytes / 8;  // worlds that drift apart in frames take a little more each run
-            if (b->arena) HIPCHECK(hipFree(b->arena));
-            b->arena = nullptr;
-            b->arena_bytes = 0;
-            if (hipMalloc(&b->arena, bytes) != hipSuccess) {
-                (void)hipGetLastError();
-                b->arena = nullptr;
-            } else {
-                b->arena_bytes = bytes;
+        {
+            std::lock_guard<std::mutex> lk(b->pool->mu);
+            if (bytes > b->arena.bytes) {
+                bytes += bytes / 8;  // worlds that drift apart in frames take a little more each run
+                se_rt::Pool::drop(b->arena);
+                if (hipMalloc(&b->arena.mem, bytes) != hipSuccess) {
+                    (void)hipGetLastError();
+                    b->arena.mem = nullptr;
+                } else {
+                    b->arena.bytes = bytes;
+                }
             }
+            b->arena.busy = b->arena.mem != nullptr;
         }
-        if (b->arena) {
-            char* p = (char*)b->arena;
+        if (b->arena.mem) {
+            char* p = (char*)b->arena.mem;
             for (auto& q : sliced) {
                 int rc = place_sliced(*q, p);
                 if (rc) return rc;
@@ -662,13 +676,18 @@ int se_batch_create(se_ctx* ctx, se_batch** out) {
     if (!ctx || !out) return fail(SE_ERR_ARG, "null argument");
     auto* b = new se_batch();
     b->ctx = ctx;
+    {
+        std::lock_guard<std::mutex> lk(ctx->pool->mu);
+        ctx->pool->arenas.push_back(&b->arena);
+    }
+    b->pool = ctx->pool;
     *out = b;
     return SE_OK;
 }
 
 void se_batch_destroy(se_batch* b) {
     if (!b) return;
-    DeviceGuard dg(b->ctx->device);
+    DeviceGuard dg(b->pool->device);
     delete b;
 }
 
@@ -686,10 +705,9 @@ int se_batch_add(se_batch* b, se_world* w, uint32_t nsteps) {
 int se_batch_clear(se_batch* b) {
     if (!b) return fail(SE_ERR_ARG, "null batch");
     b->items.clear();
-    DeviceGuard dg(b->ctx->device);
-    (void)hipFree(b->arena);
-    b->arena = nullptr;
-    b->arena_bytes = 0;
+    DeviceGuard dg(b->pool->device);
+    std::lock_guard<std::mutex> lk(b->pool->mu);
+    se_rt::Pool::drop(b->arena);
     return SE_OK;
 }
 
@@ -760,7 +778,7 @@ int se_batch_autotune(se_batch* b, uint32_t rounds, int32_t* best_variant, uint3
             se_world* w = it.first;
             size_t bytes = (size_t)w->pitch * w->H * 4;
             void* p = nullptr;
-            if (hipMalloc(&p, bytes) != hipSuccess) {
+            if (se_rt::device_alloc(b->ctx->device, &p, bytes) != hipSuccess) {
                 for (auto& s : snaps) (void)hipFree(s.first);
                 return fail(SE_ERR_OOM, "autotune snapshot allocation failed");
             }

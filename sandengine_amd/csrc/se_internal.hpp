@@ -61,6 +61,35 @@ struct FillSpec {  // == se_fillspec in se_kernels.hip
     uint32_t ids[16], thr[16];
 };
 
+// Device memory that a context keeps from call to call.  Its worlds hold it too: they may
+// outlive the context.
+struct Pool {
+    struct Block {
+        void* mem = nullptr;
+        size_t bytes = 0;
+        bool busy = false;  // a batch's run is under way
+    };
+    int device = 0;
+    std::mutex mu;
+    // packed grids and hash planes of the sliced kernels (se_sliced.cpp), as large as the
+    // largest call needed, in use while mu is held and by what that enqueued
+    Block scratch;
+    int worlds = 0;              // live worlds made by se_world_create
+    std::vector<Block*> arenas;  // of the context's batches
+    // Frees a block that nothing uses (hipFree waits for the device); mu held.
+    static void drop(Block& b) {
+        (void)hipFree(b.mem);
+        b.mem = nullptr;
+        b.bytes = 0;
+    }
+    ~Pool();
+};
+// A context's pool, known to device_alloc while it lives.
+std::shared_ptr<Pool> make_pool(int device);
+// hipMalloc on the current device, `device`; where that fails, once more after the pools of
+// all contexts there gave back what is not in use.  The caller holds no pool's mu.
+hipError_t device_alloc(int device, void** p, size_t bytes);
+
 // What the choice between a rule set's kernels goes by (se_sliced.cpp).
 struct StepCost {
     int form = 0;           // of the LDS kernels: 0 generated chain, 1 full table, 2 coded table
@@ -130,12 +159,7 @@ struct se_ctx {
     void* staging = nullptr;
     hipEvent_t staging_done = nullptr;
     std::mutex staging_mu;
-    // packed grids and hash planes of the sliced kernels (se_sliced.cpp), as large
-    // as the largest call needed; freed with the context's last world
-    std::mutex sliced_mu;
-    void* sliced_mem = nullptr;
-    size_t sliced_bytes = 0;
-    int worlds = 0;  // live worlds made by se_world_create (under sliced_mu)
+    std::shared_ptr<se_rt::Pool> pool;
 };
 
 struct se_ruleset {
@@ -153,6 +177,7 @@ struct se_world {
     uint32_t* buf[2] = {nullptr, nullptr};
     int cur = 0;
     int32_t frame = 0;
+    std::shared_ptr<se_rt::Pool> pool;  // of the context (worlds from se_world_create)
     std::vector<se_modification> pending;
     void* d_mods = nullptr;
     hipStream_t stream = nullptr;

@@ -472,6 +472,58 @@ void offset_of(int32_t frame, int& ox, int& oy) {
 
 }  // namespace
 
+// ------------------------------------------------------------------ kept device memory
+namespace {
+std::mutex g_pools_mu;  // taken before any pool's mu
+std::vector<std::weak_ptr<se_rt::Pool>> g_pools;
+constexpr size_t kKeptScratch = 512u << 20;  // of a context without worlds
+}  // namespace
+
+se_rt::Pool::~Pool() {
+    if (!scratch.mem) return;
+    DeviceGuard dg(device);
+    drop(scratch);
+}
+
+std::shared_ptr<se_rt::Pool> se_rt::make_pool(int device) {
+    auto p = std::make_shared<Pool>();
+    p->device = device;
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    g_pools.erase(std::remove_if(g_pools.begin(), g_pools.end(), [](const std::weak_ptr<Pool>& w) { return w.expired(); }),
+                  g_pools.end());
+    g_pools.push_back(p);
+    return p;
+}
+
+hipError_t se_rt::device_alloc(int device, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    *p = nullptr;
+    std::vector<std::shared_ptr<Pool>> pools;  // released after the lock: the last owner frees
+    bool any = false;
+    {
+        std::lock_guard<std::mutex> lk(g_pools_mu);
+        for (auto& w : g_pools)
+            if (auto q = w.lock()) pools.push_back(std::move(q));
+    }
+    for (auto& q : pools) {
+        if (q->device != device) continue;
+        std::lock_guard<std::mutex> lk(q->mu);
+        any = any || q->scratch.mem;
+        if (q->scratch.mem) Pool::drop(q->scratch);
+        for (Pool::Block* b : q->arenas)
+            if (b->mem && !b->busy) {
+                any = true;
+                Pool::drop(*b);
+            }
+    }
+    if (!any) return e;
+    (void)hipGetLastError();  // of the first attempt
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) *p = nullptr;
+    return e;
+}
+
 int se_rt::take_mods(se_world* w, ModsArg& m, FewMods* few) {
     m.ptr = w->d_mods;
     m.n = 0;
@@ -570,16 +622,18 @@ int se_rt::fill_spec(const se_world* w, uint32_t* grid, uint64_t seed, const Fil
 
 int se_rt::sleep_room(se_world* w, size_t n) {
     if (n <= w->sleep_cap) return SE_OK;
-    hipFree(w->d_sleep[0]);
-    hipFree(w->d_sleep[1]);
+    hipFree(w->d_sleep[0]);  // both arrays
     w->d_sleep[0] = w->d_sleep[1] = nullptr;
     w->sleep_cap = 0;
     w->sleep_variant = -1;
-    for (auto& p : w->d_sleep)
-        if (hipMalloc(&p, n) != hipSuccess) {
-            (void)hipGetLastError();
-            return fail(SE_ERR_HIP, "hipMalloc of a sleep record failed");
-        }
+    n = (n + 255) & ~(size_t)255;
+    void* p = nullptr;
+    if (device_alloc(w->ctx->device, &p, 2 * n) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(SE_ERR_HIP, "hipMalloc of a sleep record failed");
+    }
+    w->d_sleep[0] = (unsigned char*)p;
+    w->d_sleep[1] = w->d_sleep[0] + n;
     w->sleep_cap = n;
     return SE_OK;
 }
@@ -762,6 +816,7 @@ int se_ctx_create(int device, se_ctx** out) {
     DeviceGuard dg(device);
     auto* c = new se_ctx();
     c->device = device;
+    c->pool = se_rt::make_pool(device);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         delete c;
         return fail(SE_ERR_HIP, "hipStreamCreate failed");
@@ -793,7 +848,8 @@ void se_ctx_destroy(se_ctx* ctx) {
             hipEventDestroy(ctx->staging_done);
         }
         if (ctx->staging) hipHostFree(ctx->staging);
-        hipFree(ctx->sliced_mem);
+        std::lock_guard<std::mutex> lk(ctx->pool->mu);
+        se_rt::Pool::drop(ctx->pool->scratch);
     }
     delete ctx;
 }
@@ -882,8 +938,9 @@ int se_world_create(se_ctx* ctx, const se_ruleset* rs, uint32_t w, uint32_t h, s
     W->pitch = (w + 63u) & ~63u;
     W->stream = ctx->stream;
     size_t bytes = (size_t)W->pitch * h * sizeof(uint32_t);
-    if (hipMalloc(&W->buf[0], bytes) != hipSuccess || hipMalloc(&W->buf[1], bytes) != hipSuccess ||
-        hipMalloc(&W->d_mods, sizeof(se_modification) * SE_MAX_MODIFICATIONS) != hipSuccess) {
+    auto alloc = [&](void* p, size_t n) { return se_rt::device_alloc(ctx->device, (void**)p, n) == hipSuccess; };
+    if (!alloc(&W->buf[0], bytes) || !alloc(&W->buf[1], bytes) ||
+        !alloc(&W->d_mods, sizeof(se_modification) * SE_MAX_MODIFICATIONS)) {
         hipFree(W->buf[0]);
         hipFree(W->buf[1]);
         hipFree(W->d_mods);
@@ -891,9 +948,10 @@ int se_world_create(se_ctx* ctx, const se_ruleset* rs, uint32_t w, uint32_t h, s
         hipGetLastError();
         return fail(SE_ERR_OOM, "hipMalloc of " + std::to_string(2 * bytes) + " bytes failed");
     }
+    W->pool = ctx->pool;
     {
-        std::lock_guard<std::mutex> lk(ctx->sliced_mu);
-        ctx->worlds++;
+        std::lock_guard<std::mutex> lk(ctx->pool->mu);
+        ctx->pool->worlds++;
     }
     int rc = launch_fill(W, W->buf[0], 0u);
     if (!rc) rc = launch_fill(W, W->buf[1], 0u);
@@ -908,7 +966,7 @@ int se_world_create(se_ctx* ctx, const se_ruleset* rs, uint32_t w, uint32_t h, s
 void se_world_destroy(se_world* w) {
     if (!w) return;
     {
-        DeviceGuard dg(w->ctx->device);
+        DeviceGuard dg(w->pool ? w->pool->device : w->ctx->device);
         hipStreamSynchronize(w->stream);
         if (w->owns) {
             hipFree(w->buf[0]);
@@ -919,13 +977,14 @@ void se_world_destroy(se_world* w) {
         hipFree(w->light[1]);
         hipFree(w->color);
         hipFree(w->noise);
-        hipFree(w->d_sleep[0]);
-        hipFree(w->d_sleep[1]);
-        std::lock_guard<std::mutex> lk(w->ctx->sliced_mu);
-        if (w->owns && --w->ctx->worlds == 0) {
-            hipFree(w->ctx->sliced_mem);
-            w->ctx->sliced_mem = nullptr;
-            w->ctx->sliced_bytes = 0;
+        hipFree(w->d_sleep[0]);  // both arrays
+        if (w->pool) {
+            // The last world's end gives the scratch back where it is larger than any up to
+            // 16384^2 needs.  Less stays with the context, or until an allocation fails: making and
+            // freeing it takes as long as the run (create, 16 steps, destroy, us, LDS kernels / with
+            // both / so: 4096^2 502 / 786 / 511, 8192^2 943 / 1197 / 946, 16384^2 1608 / 1867 / 1567).
+            std::lock_guard<std::mutex> lk(w->pool->mu);
+            if (--w->pool->worlds == 0 && w->pool->scratch.bytes > kKeptScratch) se_rt::Pool::drop(w->pool->scratch);
         }
     }
     delete w;
@@ -1038,8 +1097,8 @@ int se_world_set_render(se_world* w, int enable) {
     }
     if (w->color) return SE_OK;
     const size_t bytes = (size_t)w->pitch * w->H * 16;
-    if (hipMalloc(&w->light[0], bytes) != hipSuccess || hipMalloc(&w->light[1], bytes) != hipSuccess ||
-        hipMalloc(&w->color, bytes) != hipSuccess || hipMalloc(&w->noise, bytes / 4) != hipSuccess) {
+    auto alloc = [&](void* p, size_t n) { return se_rt::device_alloc(w->ctx->device, (void**)p, n) == hipSuccess; };
+    if (!alloc(&w->light[0], bytes) || !alloc(&w->light[1], bytes) || !alloc(&w->color, bytes) || !alloc(&w->noise, bytes / 4)) {
         hipGetLastError();
         release();
         return fail(SE_ERR_OOM, "hipMalloc of " + std::to_string(13 * bytes / 4) + " bytes for render outputs failed");
@@ -1337,7 +1396,7 @@ int se_world_autotune(se_world* w, uint32_t nsteps, uint32_t rounds, int32_t* be
         }
     } R;
     const size_t bytes = (size_t)w->pitch * w->H * 4;
-    if (hipMalloc(&R.snap, bytes) != hipSuccess) return fail(SE_ERR_OOM, "autotune snapshot allocation failed");
+    if (se_rt::device_alloc(w->ctx->device, &R.snap, bytes) != hipSuccess) return fail(SE_ERR_OOM, "autotune snapshot allocation failed");
     HIPCHECK(hipEventCreate(&R.ev[0]));
     HIPCHECK(hipEventCreate(&R.ev[1]));
     HIPCHECK(hipMemcpyAsync(R.snap, w->buf[w->cur], bytes, hipMemcpyDeviceToDevice, w->stream));

@@ -56,8 +56,8 @@ struct Arena {
     char* base = nullptr;
     size_t size = 0, used = 0, peak = 0;
     std::map<size_t, size_t> free_;  // offset -> length
-    int init(size_t bytes) {
-        HIPCHECK(hipMalloc((void**)&base, bytes));
+    int init(int device, size_t bytes) {
+        HIPCHECK(se_rt::device_alloc(device, (void**)&base, bytes));
         size = bytes;
         free_[0] = bytes;
         return SE_OK;
@@ -725,7 +725,7 @@ int se_serve_run(se_serve* S, se_serve_stats* stats) {
     DeviceGuard dg(S->ctx->device);
     const double slo = S->cfg.slo_ms;
     Arena A;
-    int rc = A.init(S->cfg.hbm_budget);
+    int rc = A.init(S->ctx->device, S->cfg.hbm_budget);
     if (rc) return rc;
     std::vector<Slot> slots(S->cfg.max_inflight);
     StreamDrain drain{S->ctx->stream};  // destroyed before the slots and the arena

@@ -378,37 +378,6 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     const uint32_t ahead = plan.frames;
     const size_t bytes = 2 * packed + plan.bytes;
 
-    // The scratch belongs to the context: its worlds share one stream, and the
-    // launches of one call are enqueued together under the lock.
-    se_ctx* ctx = w->ctx;
-    std::lock_guard<std::mutex> lk(ctx->sliced_mu);
-    if (bytes > ctx->sliced_bytes) {
-        if (ctx->sliced_mem) HIPCHECK(hipFree(ctx->sliced_mem));  // waits for the work that uses it
-        ctx->sliced_mem = nullptr;
-        ctx->sliced_bytes = 0;
-        if (hipMalloc(&ctx->sliced_mem, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            ctx->sliced_mem = nullptr;
-            return SE_OK;
-        }
-        ctx->sliced_bytes = bytes;
-    }
-    ModsArg mods;
-    FewMods few{};
-    int rc = take_mods(w, mods, &few);
-    if (rc) return rc;
-    *done = true;
-    one.frame0 = w->frame + 1;
-    one.steps = (int)n;
-    one.tiles_x = shape.tiles_x;
-    one.side = shape.side;
-    one.halo = shape.halo;
-    g.in = w->buf[w->cur];
-    g.out = w->buf[w->cur ^ 1];
-    g.pk0 = ctx->sliced_mem;
-    g.pk1 = (char*)ctx->sliced_mem + packed;
-    g.hash = (uint32_t*)((char*)ctx->sliced_mem + 2 * packed);
-
     const int ptiles = sliced_pack_tiles(g), pcols = ptiles / (g.rows / 64);
     const int ucols = sliced_unpack_columns(g), utiles = ucols * (g.rows / 64);
     // Sleeping, from some 4 M cells on (below, a call is a chain of launches and steps that
@@ -431,6 +400,37 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
         one.calm = known.calm;
         one.calm_cols = pcols;
     }
+
+    // The scratch belongs to the context: its worlds share one stream, and the
+    // launches of one call are enqueued together under the lock.
+    se_ctx* ctx = w->ctx;
+    std::lock_guard<std::mutex> lk(ctx->pool->mu);
+    Pool::Block& scratch = ctx->pool->scratch;
+    if (bytes > scratch.bytes) {
+        if (scratch.mem) Pool::drop(scratch);  // waits for the work that uses it
+        if (hipMalloc(&scratch.mem, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            scratch.mem = nullptr;
+            return SE_OK;
+        }
+        scratch.bytes = bytes;
+    }
+    ModsArg mods;
+    FewMods few{};
+    int rc = take_mods(w, mods, &few);
+    if (rc) return rc;
+    *done = true;
+    one.frame0 = w->frame + 1;
+    one.steps = (int)n;
+    one.tiles_x = shape.tiles_x;
+    one.side = shape.side;
+    one.halo = shape.halo;
+    g.in = w->buf[w->cur];
+    g.out = w->buf[w->cur ^ 1];
+    g.pk0 = scratch.mem;
+    g.pk1 = (char*)scratch.mem + packed;
+    g.hash = (uint32_t*)((char*)scratch.mem + 2 * packed);
+
     sleep_reset(w);  // until the run is enqueued
     rc = launch2(K.pack, (unsigned)(ptiles + 3) / 4, 1, 256, w->stream, g, pcols, ptiles, known);
     int from = 0;
