@@ -255,7 +255,7 @@ double hash_time(const se_rt::StepCost& c, se_rt::SlicedGrid g, uint32_t n) {
 
 bool se_rt::sliced_pays(const SlicedKernels& K, uint32_t W, uint32_t H, uint32_t n) {
     const StepCost& c = K.cost;
-    if (!K.ok || n < (c.form == 0 ? 4u : 9u)) return false;
+    if (!K.ok || n < sliced_least_steps(K)) return false;
     if (std::min(W, H) >= 128 && (c.form == 0 || c.tables <= 300)) return true;
     SlicedShape s = sliced_one_tile(W, H, true);
     if (!s.nw) {
@@ -283,7 +283,7 @@ bool se_rt::sliced_batch_pays(const SlicedKernels& K, const std::vector<SlicedLo
         most = std::max(most, w.n);
         if (w.n) squares += sliced_squares(w.W, w.H);
     }
-    if (!K.ok || most < (c.form == 0 ? 4u : 9u)) return false;
+    if (!K.ok || most < sliced_least_steps(K)) return false;
     int kernel;
     uint32_t deep;
     sliced_choice(squares, K, &kernel, &deep);
@@ -301,7 +301,7 @@ bool se_rt::sliced_batch_pays(const SlicedKernels& K, const std::vector<SlicedLo
     SlicedLoad last{0, 0, 0, 0};
     SlicedGrid g;
     bool one = false;
-    double t = 0, cells = 0, lds_all = 0, lds_chain = 0, sliced_all = 0, sliced_chain = 0, count = 0;
+    double t = 0, work = 0, chain = 0, sliced = 0, cells = 0, lds_all = 0, lds_chain = 0, sliced_all = 0, sliced_chain = 0, count = 0;
     for (auto& w : worlds) {
         if (!w.n) continue;
         if (w.W != last.W || w.H != last.H || w.n != last.n) {  // runs of equal worlds
@@ -312,6 +312,10 @@ bool se_rt::sliced_batch_pays(const SlicedKernels& K, const std::vector<SlicedLo
             g = SlicedGrid();
             sliced_geometry(s, w.W, w.H, g);
             t = hash_time(c, g, w.n);
+            const double steps = lds_steps(w.W, w.H, w.n);
+            work = steps * lds_work(c, w.W, w.H);
+            chain = steps * lds_latency(c, w.W, w.H);
+            sliced = w.n * c.tables * (one ? 3.9e-6 : 3.5e-6 * sliced_squares(w.W, w.H));
         }
         List& l = lists[one];
         if (!l.worlds) l.most = g;
@@ -328,10 +332,9 @@ bool se_rt::sliced_batch_pays(const SlicedKernels& K, const std::vector<SlicedLo
         at[i] = w.frame;
         count++;
         cells += 1e-6 * w.W * w.H;
-        const double steps = lds_steps(w.W, w.H, w.n);
-        lds_all += steps * lds_work(c, w.W, w.H);
-        lds_chain = std::max(lds_chain, steps * lds_latency(c, w.W, w.H));
-        sliced_all += w.n * c.tables * (one ? 3.9e-6 : 3.5e-6 * sliced_squares(w.W, w.H));
+        lds_all += work;
+        lds_chain = std::max(lds_chain, chain);
+        sliced_all += sliced;
         sliced_chain = std::max(sliced_chain, w.n * sliced_latency(c, one));
     }
     double host = 0;

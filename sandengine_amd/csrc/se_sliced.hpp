@@ -74,6 +74,8 @@ struct SlicedAhead {
 };
 SlicedAhead sliced_ahead(const SlicedShape& s, SlicedGrid g, int32_t frame0, uint32_t n, int classes);
 
+// The fewest steps that may leave the LDS kernels.
+inline uint32_t sliced_least_steps(const SlicedKernels& K) { return K.cost.form == 0 ? 4 : 9; }
 // Is the sliced path taken for n steps of a world whose caller chose no variant?
 bool sliced_pays(const SlicedKernels& K, uint32_t W, uint32_t H, uint32_t n);
 // And for the worlds of a batch that share the rule set?
