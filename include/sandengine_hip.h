@@ -224,8 +224,9 @@ int se_batch_clear(se_batch* b);
  * autotuned shape (else one workgroup per item).
  * lds_variant -1 / k 0: the autotuned (else default) choice, which for longer
  * runs of rule sets with a sliced form is the sliced kernels (modes 1 and 2).
- * graph != 0 captures a submission of LDS kernels in a hipGraph and launches
- * that; the sliced kernels' few launches are submitted directly.
+ * graph != 0 captures the LDS kernels' launches in a hipGraph and launches
+ * that; rule sets that take the sliced kernels submit their few launches directly
+ * beside it.
  * *gpu_ms: time between events around the submission. */
 int se_batch_run(se_batch* b, int mode, int32_t lds_variant, uint32_t k, int graph, float* gpu_ms);
 /* Autotuner: for each rule-set group, times every LDS variant with k = halo and

@@ -475,8 +475,9 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
         uint32_t most = 0;
         for (auto& it : g.second) most = std::max(most, it.second);
         bool want = mod->lds[vi].first.sliced;
-        if (!want && !chosen && la != 1 && mod->sliced.ok) {
+        if (!want && !chosen && la != 1 && mod->sliced.ok && most >= se_rt::sliced_least_steps(mod->sliced)) {
             std::vector<se_rt::SlicedLoad> loads;
+            loads.reserve(g.second.size());
             for (auto& it : g.second) loads.push_back({it.first->W, it.first->H, it.second, it.first->frame});
             want = se_rt::sliced_batch_pays(mod->sliced, loads);
         }
@@ -551,7 +552,7 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
         }
     }
     const size_t n_streams = 2 * plans.size() + (sliced.empty() ? 0 : 3);
-    int rc = ensure_streams(b, (int)n_streams);
+    int rc = ensure_streams(b, (int)n_streams + (graph && !sliced.empty() ? 1 : 0));  // one for a graph beside sliced plans
     if (rc) return rc;
     RunResources res;  // declared after `plans`: destroyed (and the stream drained) first
     res.streams.assign(b->streams, b->streams + 8);
@@ -570,7 +571,7 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
             if (!rc) rc = res.event(&e, hipEventDisableTiming);
     }
     if (rc) return rc;
-    auto submit = [&]() -> int {
+    auto submit_plans = [&]() -> int {  // forks from the context's stream and joins it
         HIPCHECK(hipEventRecord(fork, ctx->stream));
         for (size_t i = 0; i < plans.size(); i++) {
             hipStream_t sa = b->streams[(2 * i) % 8], sb = b->streams[(2 * i + 1) % 8];
@@ -581,11 +582,14 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
             HIPCHECK(hipEventRecord(joins[2 * i], sa));
             HIPCHECK(hipEventRecord(joins[2 * i + 1], sb));
         }
+        return SE_OK;
+    };
+    auto submit_sliced = [&](hipEvent_t begin) -> int {
         if (!sliced.empty()) {
             hipStream_t st[3];
             for (int i = 0; i < 3; i++) {
                 st[i] = b->streams[(2 * plans.size() + i) % 8];
-                HIPCHECK(hipStreamWaitEvent(st[i], fork, 0));
+                HIPCHECK(hipStreamWaitEvent(st[i], begin, 0));
             }
             for (size_t i = 0; i < sliced.size(); i++) {
                 if (lane[i] < 2) continue;
@@ -621,26 +625,50 @@ int run_batched(se_batch* b, const std::vector<std::pair<se_world*, uint32_t>>& 
             }
             for (int i = 0; i < 3; i++) HIPCHECK(hipEventRecord(joins[2 * plans.size() + i], st[i]));
         }
-        for (auto& j : joins) HIPCHECK(hipStreamWaitEvent(ctx->stream, j, 0));
         return SE_OK;
     };
-    // Sliced plans are submitted directly: they make some forty launches where the
-    // rounds of the LDS kernels make hundreds, and capturing them has ended in heap
-    // corruption inside one of the HIP runtimes that programs load.
-    if (!sliced.empty()) graph = 0;
-    if (graph) {
+    auto join = [&](size_t from, size_t to) -> int {
+        for (size_t i = from; i < to; i++) HIPCHECK(hipStreamWaitEvent(ctx->stream, joins[i], 0));
+        return SE_OK;
+    };
+    // A graph holds the LDS plans' launches, hundreds in their rounds.  Sliced plans make some
+    // forty and are submitted directly, beside the graph: a run that captured them ended in
+    // a host abort ("free(): invalid next size") under one HIP runtime, whose cause was not
+    // found.
+    const size_t n_plan_joins = 2 * plans.size();
+    hipStream_t beside = nullptr;  // of the graph, where sliced plans run too
+    hipEvent_t begin = nullptr, end = nullptr;
+    if (graph && !plans.empty()) {
         HIPCHECK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        int r2 = submit();
+        int r2 = submit_plans();
+        if (!r2) r2 = join(0, n_plan_joins);
         hipError_t ce = hipStreamEndCapture(ctx->stream, &res.graph);
         if (r2) return r2;
         if (ce != hipSuccess) return fail(SE_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(ce));
         HIPCHECK(hipGraphInstantiate(&res.exec, res.graph, nullptr, nullptr, 0));
+        if (!sliced.empty()) {
+            beside = b->streams[(n_plan_joins + 3) % 8];
+            rc = res.event(&begin, hipEventDisableTiming);
+            if (!rc) rc = res.event(&end, hipEventDisableTiming);
+            if (rc) return rc;
+        }
     }
     HIPCHECK(hipEventRecord(e0, ctx->stream));
-    if (graph) {
+    if (beside) {
+        HIPCHECK(hipEventRecord(begin, ctx->stream));
+        HIPCHECK(hipStreamWaitEvent(beside, begin, 0));
+        HIPCHECK(hipGraphLaunch(res.exec, beside));
+        HIPCHECK(hipEventRecord(end, beside));
+        rc = submit_sliced(begin);
+        if (!rc) rc = join(n_plan_joins, joins.size());
+        if (rc) return rc;
+        HIPCHECK(hipStreamWaitEvent(ctx->stream, end, 0));
+    } else if (res.exec) {
         HIPCHECK(hipGraphLaunch(res.exec, ctx->stream));
     } else {
-        rc = submit();
+        rc = submit_plans();
+        if (!rc) rc = submit_sliced(fork);
+        if (!rc) rc = join(0, joins.size());
         if (rc) return rc;
     }
     HIPCHECK(hipEventRecord(e1, ctx->stream));
