@@ -160,7 +160,8 @@ extern "C" int se_grids_step_noalloc(se_ctx* ctx, const se_ruleset* rs, se_grid_
     for (uint32_t i = 0; i < n; i++) {
         if (!merge || !steps[i] || !single(i)) continue;
         per[i] = (steps[i] + most - 1) / most;
-        while (rounds_of(i) % 2 == 0) per[i]++;
+        // the least number of steps a round that takes a round less, until their number is odd
+        for (uint32_t r = rounds_of(i); r % 2 == 0; r = rounds_of(i)) per[i] = (steps[i] + r - 2) / (r - 1);
     }
     for (uint32_t i = 0; i < n; i++)
         if (steps[i] && single(i) && !merge) order[ns++] = i;

@@ -11,6 +11,7 @@ import pytest
 import sandengine_amd as S
 from oracle import lang_ref as L
 from oracle import oracle as O
+from tests.test_zz_no_alloc import H2D, hip, ok
 
 pytestmark = pytest.mark.gpu
 
@@ -109,7 +110,8 @@ def test_a_caller_with_the_grids_address_writes_between_runs():
     """Once a grid's address was given out nothing is known of the grids: cells written
     through it between two runs are stepped."""
     print("\n[gpu] sliced sleep, a grid written through its address", flush=True)
-    a, b = world("four_materials", 2304, 2112) if rs("four_materials") else None, None
+    rs("four_materials")
+    a = world("four_materials", 2304, 2112)
     b = world("four_materials", 2304, 2112, sliced=False)
     ptrs = []
     for w in (a, b):
@@ -118,7 +120,7 @@ def test_a_caller_with_the_grids_address_writes_between_runs():
             assert S.lib().se_world_device_ptr(w._p, ctypes.byref(p), ctypes.byref(pitch)) == 0
             ptrs.append(p.value)
             w.step(1)
-    hip = ctypes.CDLL("libamdhip64.so")
+    H = hip()
     rows = np.full((200, 2304), 4, np.uint32)
     for run in range(3):
         for w, (p0, p1) in ((a, ptrs[:2]), (b, ptrs[2:])):
@@ -126,8 +128,7 @@ def test_a_caller_with_the_grids_address_writes_between_runs():
             w.sync()
             # 24 steps: an even number of plain steps, one exchange of the grids in a sliced run
             cur = (p0 if run % 2 == 1 else p1) if w is a else p0
-            assert hip.hipMemcpy(ctypes.c_void_p(cur + 4 * 2304 * 1500), rows.ctypes.data_as(ctypes.c_void_p),
-                                 ctypes.c_size_t(rows.nbytes), 1) == 0
+            ok(H.hipMemcpy(cur + 4 * 2304 * 1500, rows.ctypes.data, rows.nbytes, H2D))
         np.testing.assert_array_equal(a.download(), b.download())
     a.close()
     b.close()
