@@ -118,19 +118,22 @@ int se_world_push_modification(se_world* w, const se_modification* m);
 int se_world_step(se_world* w, uint32_t nsteps);
 /* Same result as se_world_step, advanced in launches of up to `sub` sub-steps (0 =
  * autotuned choice): by the sliced kernels (bit planes, 32 blocks to a word) for
- * longer runs of rule sets that have that form, else by the LDS temporal-blocked
- * kernel. */
+ * runs of rule sets that have that form where they are the faster ones (most from 9
+ * steps on), else by the LDS temporal-blocked kernel. */
 int se_world_step_blocked(se_world* w, uint32_t nsteps, uint32_t sub);
 /* Kernel variant selection (no reference counterpart; the autotuner drives it):
  * plain_variant indexes the plain-kernel instantiations (rows per wavefront x
  * store kind), lds_variant the LDS-tile instantiations (-1: default).
  * se_variant_info(kind 0 plain: a=rows, b=non-temporal; kind 1 lds: a=tile w,
  * b=tile h, c=max sub-steps * 1000 + threads per workgroup; kind 2: a=the LDS
- * variant se_world_step_blocked uses for `index` sub-steps per launch; kind 3:
- * a=workgroups of LDS variant `index` resident at once on the device (the
- * batch's persistent launch shape), b=its LDS bytes per workgroup).  The last
- * LDS index of a rule set with a sliced form (bit planes, se_world_step_blocked's
- * choice for longer runs) names those kernels: LDS bytes 0. */
+ * variant se_world_step_blocked uses for `index` sub-steps per launch where it
+ * takes the LDS kernels; kind 3: a=workgroups of LDS variant `index` resident at
+ * once on the device (the batch's persistent launch shape), b=its LDS bytes per
+ * workgroup; kind 4: a=1 if se_world_step_blocked takes the sliced kernels for
+ * `index` steps, by default or as chosen, b=their step kernel (0 to 3: tiles of
+ * 2x2 and 4x2 words by one wavefront, 2x2 by two, 4x2 by four), c=its steps a
+ * launch).  The last LDS index of a rule set with a sliced form (bit planes) names
+ * those kernels: LDS bytes 0. */
 int se_world_set_variant(se_world* w, int32_t plain_variant, int32_t lds_variant);
 /* Tile sleeping of se_world_step_blocked (no reference counterpart; on by
  * default): an LDS tile whose cells, halo included, all hold one material whose

@@ -1072,6 +1072,15 @@ int se_variant_info(const se_world* w, int32_t kind, int32_t index, int32_t* a, 
         if (!p) return fail(SE_ERR_ARG, "no LDS variant supports " + std::to_string(index) + " sub-steps");
         return put((int32_t)(p - &w->mod->lds[0]), 0, 0);
     }
+    if (kind == 4) {  // does se_world_step_blocked(w, index, 0) take the sliced kernels, and which
+        if (index < 1) return fail(SE_ERR_ARG, "number of steps out of range");
+        const se_rt::SlicedKernels& K = w->mod->sliced;
+        const bool takes = !w->color && (w->lds_variant < 0 ? se_rt::sliced_pays(K, w->W, w->H, (uint32_t)index)
+                                                            : w->mod->lds[w->lds_variant].first.sliced);
+        if (!takes) return put(0, 0, 0);
+        const se_rt::SlicedShape s = se_rt::sliced_shape(K, w->W, w->H, (uint32_t)index, 0);
+        return put(1, s.kernel, (int32_t)std::min(s.max_sub, (uint32_t)index));
+    }
     if (index < 0 || index >= (int)w->mod->lds.size()) return fail(SE_ERR_ARG, "lds variant out of range");
     const se::LdsVariant& v = w->mod->lds[index].first;
     if (kind == 1) return put(v.tw, v.th, v.hb * 1000 + v.nt);

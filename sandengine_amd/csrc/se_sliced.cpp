@@ -257,13 +257,7 @@ bool se_rt::sliced_pays(const SlicedKernels& K, uint32_t W, uint32_t H, uint32_t
     const StepCost& c = K.cost;
     if (!K.ok || n < sliced_least_steps(K)) return false;
     if (std::min(W, H) >= 128 && (c.form == 0 || c.tables <= 300)) return true;
-    SlicedShape s = sliced_one_tile(W, H, true);
-    if (!s.nw) {
-        int kernel;
-        uint32_t deep;
-        sliced_choice(sliced_squares(W, H), K, &kernel, &deep);
-        s = sliced_tiles(W, H, kernel, deep);
-    }
+    const SlicedShape s = sliced_shape(K, W, H, n, 0);
     SlicedGrid g;
     sliced_geometry(s, W, H, g);
     const double cells = 1e-6 * W * H, area = 16e-6 * g.bcols * g.rows;
@@ -351,6 +345,19 @@ bool se_rt::sliced_batch_pays(const SlicedKernels& K, const std::vector<SlicedLo
            76 + .045 * count + std::hypot(lds_chain, lds_all);
 }
 
+se_rt::SlicedShape se_rt::sliced_shape(const SlicedKernels& K, uint32_t W, uint32_t H, uint32_t n, uint32_t sub) {
+    SlicedShape s = sliced_one_tile(W, H, true);
+    if (s.nw) {
+        if (sub) s.max_sub = sub;
+        return s;
+    }
+    int kernel;
+    uint32_t deep;
+    sliced_choice(sliced_squares(W, H), K, &kernel, &deep);
+    if (deep < n && n <= 16) deep = 16;
+    return sliced_tiles(W, H, kernel, sub ? std::min(sub, deep) : deep);
+}
+
 // A launch of one sub-step and se_sl_brush take some 10 us and a pass over the packed
 // grid, a plain step 5 us and a pass over the ids, and it ends what is known of the
 // grids (us a call with a brush, plain step / packed: four materials 256^2 9 steps 35 / 42,
@@ -362,16 +369,7 @@ bool se_rt::sliced_takes_mods(const se_world* w, uint32_t n) {
 int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
     *done = false;
     const SlicedKernels& K = w->mod->sliced;
-    SlicedShape shape = sliced_one_tile(w->W, w->H, true);
-    if (!shape.nw) {
-        int kernel;
-        uint32_t deep;
-        sliced_choice(sliced_squares(w->W, w->H), K, &kernel, &deep);
-        if (deep < n && n <= 16) deep = 16;
-        shape = sliced_tiles(w->W, w->H, kernel, sub ? std::min(sub, deep) : deep);
-    } else if (sub) {
-        shape.max_sub = sub;
-    }
+    const SlicedShape shape = sliced_shape(K, w->W, w->H, n, sub);
     SlicedWorld one;
     SlicedGrid& g = one.g;
     sliced_geometry(shape, w->W, w->H, g);

@@ -56,6 +56,8 @@ SlicedShape sliced_one_tile(uint32_t W, uint32_t H, bool wide);
 SlicedShape sliced_tiles(uint32_t W, uint32_t H, int kernel, uint32_t max_sub);
 // Step kernel and depth of a launch for worlds of `few` 64 x 64 squares in all.
 void sliced_choice(size_t few, const SlicedKernels& K, int* kernel, uint32_t* deep);
+// What a run of n steps takes, in launches of up to `sub` (0: the choice).
+SlicedShape sliced_shape(const SlicedKernels& K, uint32_t W, uint32_t H, uint32_t n, uint32_t sub);
 inline size_t sliced_squares(uint32_t W, uint32_t H) { return (size_t)((W + 63) / 64) * ((H + 63) / 64); }
 // Fills the geometry fields of g for that shape.
 void sliced_geometry(const SlicedShape& s, uint32_t W, uint32_t H, SlicedGrid& g);
