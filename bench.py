@@ -36,9 +36,7 @@ WORKLOADS = {
     "single256": (256, "four_materials", 0, [0, 3, 4, 5], [50, 25, 15, 10], (0, 1), 0),
     "rich8k": (8192, "twelve_materials", 2, [0] + list(range(3, 15)), [40] + [5] * 12, (0, 1), 0),
 }
-# Step kernel and deepest launch of the sliced form, by the world's size and planes
-SLICED = {"single16k": ("se_sl_step_4x2", 12), "rich8k": ("se_sl_step_4x2s", 16), "single256": ("se_sl_step_2x2s", 32)}
-SLICED_PAYS = 9  # steps from which the default choice is the sliced kernels
+SLICED_STEP = ["se_sl_step_2x2", "se_sl_step_4x2", "se_sl_step_2x2s", "se_sl_step_4x2s"]  # as World.variant_info(4, n) counts
 BATCH = {
     # name: (n worlds, side range, step range, seed)
     "batch4096": (4096, (64, 1024), (100, 1000), 3),
@@ -346,11 +344,16 @@ def log(*a):
 
 
 def make_world(S, ctx, rs, wl):
-    side, _, seed, ids, pct, (num, den), stone = WORKLOADS[wl]
+    side = WORKLOADS[wl][0]
     w = S.World(ctx, rs, side, side)
+    seed_world(w, wl)
+    return w
+
+
+def seed_world(w, wl):
+    side, _, seed, ids, pct, (num, den), stone = WORKLOADS[wl]
     w.frame = 1  # the clearing frame has run; the seeded grid starts at frame 2
     w.fill_seeded(seed, ids, pct, stone_rows=(side * num) // den, stone_id=stone)
-    return w
 
 
 def time_path(S, w, mode, steps, warmup, sub):
@@ -361,18 +364,6 @@ def time_path(S, w, mode, steps, warmup, sub):
     gpu_ms = w.step_timed(steps, 0 if mode == "plain" else 1, sub)
     wall = time.perf_counter() - t0
     return wall, gpu_ms
-
-
-def sliced_variant(S, w):
-    """Index that names the sliced kernels (the last LDS index, without LDS), or None."""
-    last, found = 0, None
-    while True:
-        try:
-            if w.variant_info(3, last)[1] == 0:
-                found = last
-        except S.SandengineError:
-            return found
-        last += 1
 
 
 def latencies(w, mode, sub, n):
@@ -563,7 +554,7 @@ def main():
     log(f"copy reference: {copy_ms:.3f} ms per 2x{4 * cells / 2**30:.2f} GiB -> {copy_gbs:.0f} GB/s")
     for mode in args.paths.split(","):
         w = make_world(S, ctx, rs, args.workload)
-        if mode == "blocked_dense":  # tile sleeping off: LDS tiles are all loaded and stored
+        if mode == "blocked_dense":  # tile sleeping off: all tiles are stepped, loaded and stored
             w.set_sleep(False)
         sub, tune, lds_kernel = args.sub, None, None
         if mode == "blocked_tuned":  # the variant se_world_autotune picks for this run length (untimed)
@@ -574,14 +565,21 @@ def main():
             log(f"autotune for {args.steps} steps: variant {vi} {w.variant_info(1, vi)}, {sub} sub-steps per launch")
         sliced = False
         if mode.startswith("blocked"):
-            which = tune["variant"] if tune else w.variant_info(2, sub)[0]
-            tw, th, c = w.variant_info(1, which)
-            lds_kernel = f"se_step_lds_{tw}x{th}_h{c // 1000}_t{c % 1000}"
-            sl = sliced_variant(S, w)
-            sliced = sl is not None and (which == sl if tune else args.steps >= SLICED_PAYS)
+            takes, step_kernel, deep = w.variant_info(4, args.steps)
+            sliced = bool(takes)
             if sliced:
-                lds_kernel = SLICED[args.workload][0]
-                sub = min(sub, SLICED[args.workload][1])
+                lds_kernel = SLICED_STEP[step_kernel]
+                sub = min(sub, deep)
+                # These kernels' device memory is taken by the first run of each length, which a
+                # short warm-up is not: the same runs once untimed, then the seeded grid again
+                time_path(S, w, mode, args.steps, args.warmup, sub)
+                w.step_timed(2 * sub, 1, sub)
+                w.step_timed(sub * args.roofline_launches, 1, sub)
+                seed_world(w, args.workload)
+                w.sync()
+            else:
+                tw, th, c = w.variant_info(1, tune["variant"] if tune else w.variant_info(2, sub)[0])
+                lds_kernel = f"se_step_lds_{tw}x{th}_h{c // 1000}_t{c % 1000}"
         wall, gpu_ms = time_path(S, w, mode, args.steps, args.warmup, sub)
         launches = args.steps if mode == "plain" else -(-args.steps // sub)
         avg_launch_ms = gpu_ms / launches
