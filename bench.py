@@ -484,16 +484,17 @@ def binding_limit(path, traffic, launch_ms, valu):
     if hbm is None or v is None:
         return "unmeasured: no counter profile for this kernel in profiles/traffic.json"
     if v >= hbm:
-        return (f"valu: the block loop issues VALU at {v:.2f} of the 614 G/s peak, while the measured HBM traffic "
+        return (f"valu: the block loop issues VALU at {v:.2f} of the 614 G/s of VOP3 forms, while the measured HBM traffic "
                 f"(`traffic`) moves at {hbm:.2f} of 8 TB/s")
     return (f"hbm: the tile loads and stores move the measured traffic (`traffic`) at {hbm:.2f} of 8 TB/s, the "
-            f"block loop issues VALU at {v:.2f} of its peak")
+            f"block loop issues VALU at {v:.2f} of the 614 G/s of VOP3 forms")
 
 
 # One wave64 VALU instruction per cycle per CU (4 SIMD16 units), 256 CUs, 2.4 GHz: the
 # issue rate measured on the MI355X for the forms the block loop is made of (VOP3, SDWA,
 # 32-bit multiplies, VOP2 with a scalar or constant operand).  VOP2 ops with two VGPR
-# sources can issue faster, so this is the ceiling for this loop, not for every kernel.
+# sources can issue faster, so this is the ceiling for the LDS kernels' loop and not for every
+# kernel: the sliced ones mix in such forms, at a rate not measured, and reach 1.05 of it.
 VALU_PEAK_WAVE_INSTR_PER_S = 256 * 2.4e9
 
 

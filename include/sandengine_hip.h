@@ -225,8 +225,9 @@ int se_batch_clear(se_batch* b);
  * Its launch shape: mode 2 one workgroup per work item, mode 3 persistent (as
  * many workgroups as are resident, striding over the items), mode 1 the
  * autotuned shape (else one workgroup per item).
- * lds_variant -1 / k 0: the autotuned (else default) choice, which for longer
- * runs of rule sets with a sliced form is the sliced kernels (modes 1 and 2).
+ * lds_variant -1 / k 0: the autotuned (else default) choice; by default a group
+ * of a rule set with a sliced form takes the sliced kernels (modes 1 and 2) where
+ * its run is long enough for them to be the faster ones.
  * graph != 0 captures the LDS kernels' launches in a hipGraph and launches
  * that; rule sets that take the sliced kernels submit their few launches directly
  * beside it.

@@ -7,12 +7,12 @@
 //   * larger worlds advance in rounds of k sub-steps (k <= the tile halo): round
 //     r covers every world with more than r*k steps; worlds are ordered by step
 //     count (longest first) so the active set of a round is a prefix, and one
-//     persistent launch per round strides over all of their tiles.
-// Rule sets with a sliced form run these two lists with the sliced kernels instead
-// (SlicedPlan below).
+//     launch per round covers all of their tiles.
+// Groups of a rule set with a sliced form run these two lists with the sliced kernels
+// where that is estimated to be faster (SlicedPlan below).
 // The single-tile launch and the rounds of every group go to their own streams
-// and overlap on the device; the whole submission can be captured in one
-// hipGraph.  The reference has no batched mode: each Simulation is one world
+// and overlap on the device; these launches can be captured in one hipGraph, the sliced
+// plans' are submitted beside it.  The reference has no batched mode: each Simulation is one world
 // (sandengine-core/src/simulation.rs:97-126); the per-world step is the same.
 #include <algorithm>
 #include <cstdio>

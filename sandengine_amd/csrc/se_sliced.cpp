@@ -70,8 +70,8 @@ se_rt::SlicedShape se_rt::sliced_one_tile(uint32_t W, uint32_t H, bool wide) {
 // make.  While those leave SIMDs idle a launch is a serial chain of sub-steps: split
 // tiles, the small one first, and the deepest launch.  Beyond that the rows and
 // columns given up count (16 columns a side up to 16 sub-steps, 32 beyond), and
-// where one wavefront a tile has the registers for it, the barriers.  us a call
-// (2x2s 32 deep / 4x2s 32 / 2x2 16 / 4x2s 16, and from the third on 4x2 12):
+// where one wavefront a tile has the registers for it, the barriers.  us a call without
+// the seeded fill (2x2s 32 deep / 4x2s 32 / 2x2 16 / 4x2s 16, and from the third on 4x2 12):
 //   1000x700   200 steps  113 / 120 / 160 / 138
 //   2000x1900  200 steps  184 / 186 / 209 / 183 / 299
 //   4096^2     200 steps  544 / 476 / 445 / 455 / 511

@@ -842,13 +842,13 @@ __device__ __forceinline__ bool se_sl_sleeps(const se_slworld& v, int from, int 
                                  min(k, v.steps - done), v.side, v.halo, sh);                                      \
     }
 // By two and by four wavefronts: half the instructions in a sub-step's chain, which
-// is what a world of few tiles waits for (us a call, one wavefront for 2x2: 100x90 500
+// is what a world of few tiles waits for (us a call without the fill, one wavefront for 2x2: 100x90 500
 // steps 229 / 162, 1000x700 200 steps 141 / 113, twelve materials 800x800 150 steps
 // 201 / 152); the wider tile gives up a smaller share of its columns.
 SE_SL_STEP(1, 2, 2, 4, 1, 2x2s)
 SE_SL_STEP(1, 2, 4, 4, 1, 4x2s)
 // By one: no barriers, for worlds that fill the SIMDs many times over (16384^2, 100
-// steps: 1.37 ms with 4x2, 1.39 with 4x2s; 4096^2, 200 steps: 445 and 455 us).  With
+// steps without the fill: 1.37 ms with 4x2, 1.39 with 4x2s; 4096^2, 200 steps: 445 and 455 us).  With
 // four planes one wavefront's registers leave two or three a SIMD and the
 // split tiles are faster (8192^2, twelve materials, 64 steps: 646 us with 4x2s, 758).
 #if SE_SL_K <= 3
