@@ -36,7 +36,7 @@ WORKLOADS = {
     "single256": (256, "four_materials", 0, [0, 3, 4, 5], [50, 25, 15, 10], (0, 1), 0),
     "rich8k": (8192, "twelve_materials", 2, [0] + list(range(3, 15)), [40] + [5] * 12, (0, 1), 0),
 }
-SLICED_STEP = ["se_sl_step_2x2", "se_sl_step_4x2", "se_sl_step_2x2s", "se_sl_step_4x2s"]  # as World.variant_info(4, n) counts
+SLICED_STEP = [f"se_sl_step_{t}" for t in ("2x2", "4x2", "2x2s", "4x2s", "2x2z", "4x2z")]  # as World.variant_info(4, n) counts
 BATCH = {
     # name: (n worlds, side range, step range, seed)
     "batch4096": (4096, (64, 1024), (100, 1000), 3),

@@ -131,8 +131,8 @@ int se_world_step_blocked(se_world* w, uint32_t nsteps, uint32_t sub);
  * once on the device (the batch's persistent launch shape), b=its LDS bytes per
  * workgroup; kind 4: a=1 if se_world_step_blocked takes the sliced kernels for
  * `index` steps, by default or as chosen, b=their step kernel (0 to 3: tiles of
- * 2x2 and 4x2 words by one wavefront, 2x2 by two, 4x2 by four), c=its steps a
- * launch).  The last LDS index of a rule set with a sliced form (bit planes) names
+ * 2x2 and 4x2 words by one wavefront, 2x2 by two, 4x2 by four; 4 and 5: the last
+ * two where their tiles may sleep), c=its steps a launch).  The last LDS index of a rule set with a sliced form (bit planes) names
  * those kernels: LDS bytes 0. */
 int se_world_set_variant(se_world* w, int32_t plain_variant, int32_t lds_variant);
 /* Tile sleeping of se_world_step_blocked (no reference counterpart; on by
@@ -140,9 +140,9 @@ int se_world_set_variant(se_world* w, int32_t plain_variant, int32_t lds_variant
  * uniform 2x2 block no rule changes skips its sub-steps, and when it and its
  * eight neighbours were already so in the previous launch it also skips its
  * loads and stores (its output buffer already holds those cells).  The sliced
- * kernels, in worlds of some 4 M cells and more, do the same by tiles for the
- * sub-steps, and by squares of 64 x 64 cells for reading and writing the grid,
- * the latter only while the caller has not asked for the grid's address
+ * kernels do the same by tiles for the sub-steps in worlds of some 8 M cells and
+ * more, and from some 4 M on by squares of 64 x 64 cells for reading and writing
+ * the grid, the latter only while the caller has not asked for the grid's address
  * (se_world_device_ptr).  Results are identical either way; any other write to
  * the grids restarts the record. */
 int se_world_set_sleep(se_world* w, int enable);

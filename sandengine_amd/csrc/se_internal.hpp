@@ -109,6 +109,7 @@ struct SlicedKernels {
     hipFunction_t pack = nullptr, unpack = nullptr, hash = nullptr, brush = nullptr;
     hipFunction_t bpack = nullptr, bunpack = nullptr, bhash = nullptr;  // the worlds of a batch
     hipFunction_t step[4] = {};  // 2x2 and 4x2 tiles by one wavefront (up to three planes), 2x2 by two, 4x2 by four
+    hipFunction_t sleep_step[4] = {};  // those of large worlds, whose tiles sleep
 };
 
 }  // namespace se_rt

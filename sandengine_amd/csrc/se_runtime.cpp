@@ -433,6 +433,11 @@ int load_module(se_ctx* ctx, const std::string& src, const se::HipGenInfo& info,
         if (info.sliced.planes <= 3) {
             HIPCHECK(hipModuleGetFunction(&K.step[0], m->mod, "se_sl_step_2x2"));
             HIPCHECK(hipModuleGetFunction(&K.step[1], m->mod, "se_sl_step_4x2"));
+            K.sleep_step[0] = K.step[0];
+            K.sleep_step[1] = K.step[1];
+        } else {
+            HIPCHECK(hipModuleGetFunction(&K.sleep_step[2], m->mod, "se_sl_step_2x2z"));
+            HIPCHECK(hipModuleGetFunction(&K.sleep_step[3], m->mod, "se_sl_step_4x2z"));
         }
         HIPCHECK(hipModuleGetFunction(&K.bpack, m->mod, "se_sl_bpack"));
         HIPCHECK(hipModuleGetFunction(&K.bunpack, m->mod, "se_sl_bunpack"));
@@ -1079,7 +1084,8 @@ int se_variant_info(const se_world* w, int32_t kind, int32_t index, int32_t* a, 
                                                             : w->mod->lds[w->lds_variant].first.sliced);
         if (!takes) return put(0, 0, 0);
         const se_rt::SlicedShape s = se_rt::sliced_shape(K, w->W, w->H, (uint32_t)index, 0);
-        return put(1, s.kernel, (int32_t)std::min(s.max_sub, (uint32_t)index));
+        const bool own = se_rt::sliced_sleeps(w, s.kernel) && K.sleep_step[s.kernel] != K.step[s.kernel];
+        return put(1, own ? s.kernel + 2 : s.kernel, (int32_t)std::min(s.max_sub, (uint32_t)index));
     }
     if (index < 0 || index >= (int)w->mod->lds.size()) return fail(SE_ERR_ARG, "lds variant out of range");
     const se::LdsVariant& v = w->mod->lds[index].first;

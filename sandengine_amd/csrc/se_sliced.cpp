@@ -17,6 +17,7 @@ using se_rt::fail;
 namespace {
 
 constexpr size_t kKnownSquares = 1024;      // from so many 64 x 64 squares on a world keeps what is known of them
+constexpr size_t kFewSquares = 2048;        // up to so many a run is a chain of sub-steps, beyond its tiles can sleep
 constexpr size_t kHashBudget = 128u << 20;  // hash planes made ahead, unless one launch needs more
 
 struct Tile {
@@ -85,7 +86,7 @@ se_rt::SlicedShape se_rt::sliced_one_tile(uint32_t W, uint32_t H, bool wide) {
 // launch and not in two (settled 16384^2: 201 us a call, 236 in two).
 void se_rt::sliced_choice(size_t few, const SlicedKernels& K, int* kernel, uint32_t* deep) {
     const bool one_wave = K.step[0] != nullptr;
-    if (few <= 2048) {
+    if (few <= kFewSquares) {
         *kernel = few <= 256 ? 2 : 3;
         *deep = 32;
     } else if (few <= 8192) {
@@ -360,10 +361,15 @@ se_rt::SlicedShape se_rt::sliced_shape(const SlicedKernels& K, uint32_t W, uint3
 
 // A launch of one sub-step and se_sl_brush take some 10 us and a pass over the packed
 // grid, a plain step 5 us and a pass over the ids, and it ends what is known of the
-// grids (us a call with a brush, plain step / packed: four materials 256^2 9 steps 35 / 42,
-// 1024^2 39 / 44, settled 4096^2 92 / 62, 16384^2 829 / 171).
+// grids (us a call of 12 steps with a brush, plain step / packed, dense worlds: twelve materials
+// 2304x2112 54 / 58, 2816x2880 73 / 74, 4096^2 115 / 105, 8192^2 292 / 236; feature rules 62 / 65,
+// 85 / 85, 131 / 121, 301 / 247; settled four materials 40 / 39, 52 / 45, 84 / 57, 222 / 87).
 bool se_rt::sliced_takes_mods(const se_world* w, uint32_t n) {
     return n > 1 && sliced_squares(w->W, w->H) >= kKnownSquares;
+}
+
+bool se_rt::sliced_sleeps(const se_world* w, int kernel) {
+    return w->sleep_enabled && sliced_squares(w->W, w->H) > kFewSquares && w->mod->sliced.sleep_step[kernel];
 }
 
 int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
@@ -381,15 +387,16 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
 
     const int ptiles = sliced_pack_tiles(g), pcols = ptiles / (g.rows / 64);
     const int ucols = sliced_unpack_columns(g), utiles = ucols * (g.rows / 64);
-    // Sleeping, from some 4 M cells on (below, a call is a chain of launches and steps that
-    // a settled tile does not shorten): settled tiles are only written, known squares are
-    // not packed or unpacked.  us a call of 12 steps of a settled world (stone below, nothing
-    // above), sleeping LDS tiles / sliced kernels without / with this: four materials 4096^2
-    // 61 / 76 / 57, 8192^2 88 / 166 / 80, 16384^2 174 / 540 / 139, twelve at 16384^2 312 / 748
-    // / 240; a dense world pays up to 1 % (8192^2 twelve 749 / 755).
+    // From some 4 M cells on known squares are not packed or unpacked, and from twice that on
+    // settled tiles are only written (below, a call is a chain of launches and steps that a
+    // settled tile does not shorten).  us a call of 12 steps of a settled world (stone below,
+    // nothing above), sleeping LDS tiles / sliced kernels without / with this: four materials
+    // 2816x2880 46 / 41 / 35, 4096^2 61 / 76 / 57, 8192^2 88 / 166 / 80, 16384^2 174 / 540 / 139,
+    // twelve at 16384^2 312 / 748 / 240; a dense world pays up to 1 % (8192^2 twelve 749 / 756).
     // A caller who holds a grid's address may write it between two calls: nothing is known
     // from one to the next then.
     SlicedKnown known;
+    hipFunction_t step = K.step[shape.kernel];
     const int variant = (int)w->mod->lds.size() - 1, layout = (g.xpad << 8 | g.ypad) << 16 | pcols;
     const size_t each = ((size_t)ptiles + 255) & ~(size_t)255;  // calm is read by whole words
     if (w->sleep_enabled && sliced_squares(w->W, w->H) >= kKnownSquares && sleep_room(w, 2 * each) == SE_OK) {
@@ -397,9 +404,12 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
         known.was = w->d_sleep[1];
         known.calm = w->d_sleep[1] + each;
         known.valid = known.same && w->sleep_variant == variant && w->sleep_layout == layout;
-        one.stable = K.stable;
-        one.calm = known.calm;
-        one.calm_cols = pcols;
+        if (sliced_sleeps(w, shape.kernel)) {
+            step = K.sleep_step[shape.kernel];
+            one.stable = K.stable;
+            one.calm = known.calm;
+            one.calm_cols = pcols;
+        }
     }
 
     // The scratch belongs to the context: its worlds share one stream, and the
@@ -448,7 +458,7 @@ int se_rt::sliced_steps(se_world* w, uint32_t n, uint32_t sub, bool* done) {
                                               (nf - d - m + shape.max_sub - 1) / shape.max_sub)
                 m -= lead;
             if (at + d == 0 && mods.n > 0) m = 1;  // modifications follow the first step
-            rc = launch2(K.step[shape.kernel], (unsigned)(shape.tiles_x * shape.tiles_y), 1, shape.threads, w->stream, one,
+            rc = launch2(step, (unsigned)(shape.tiles_x * shape.tiles_y), 1, shape.threads, w->stream, one,
                          (const SlicedWorld*)nullptr, (const int*)nullptr, 0, (const SlicedGrid*)nullptr, from,
                          (int)(at + d), (int)m);
             from ^= 1;

@@ -813,7 +813,7 @@ __device__ __forceinline__ bool se_sl_sleeps(const se_slworld& v, int from, int 
 
 // Steps [done, done + k) of `one` (n = 0), or of worlds [0, n) (longest first, their
 // tiles counted by prefix); one workgroup per tile.
-#define SE_SL_STEP(NW, R, S, AHEAD, WAVES, NAME)                                                                              \
+#define SE_SL_STEP(NW, R, S, AHEAD, WAVES, SLEEP, NAME)                                                                       \
     extern "C" __global__ __launch_bounds__(64 * S, WAVES) void se_sl_step_##NAME(                                 \
         se_slworld one, const se_slworld* __restrict__ worlds, const int* __restrict__ prefix, int n,          \
         const se_slgrid* __restrict__ groups, int from, int done, int k) {                                     \
@@ -823,7 +823,7 @@ __device__ __forceinline__ bool se_sl_sleeps(const se_slworld& v, int from, int 
         int tile;                                                                                              \
         if (n == 0) {                                                                                          \
             tile = se_xcd_tile((int)blockIdx.x, (int)gridDim.x);                                               \
-            if (one.stable != 0u &&                                                                            \
+            if (SLEEP && one.stable != 0u &&                                                                   \
                 se_sl_sleeps<NW, R, S>(one, from, tile % one.tiles_x, tile / one.tiles_x, done)) return;       \
         } else {                                                                                               \
             const int w = se_owner(prefix, n, (int)blockIdx.x);                                                \
@@ -845,15 +845,21 @@ __device__ __forceinline__ bool se_sl_sleeps(const se_slworld& v, int from, int 
 // is what a world of few tiles waits for (us a call without the fill, one wavefront for 2x2: 100x90 500
 // steps 229 / 162, 1000x700 200 steps 141 / 113, twelve materials 800x800 150 steps
 // 201 / 152); the wider tile gives up a smaller share of its columns.
-SE_SL_STEP(1, 2, 2, 4, 1, 2x2s)
-SE_SL_STEP(1, 2, 4, 4, 1, 4x2s)
+SE_SL_STEP(1, 2, 2, 4, 1, false, 2x2s)
+SE_SL_STEP(1, 2, 4, 4, 1, false, 4x2s)
 // By one: no barriers, for worlds that fill the SIMDs many times over (16384^2, 100
 // steps without the fill: 1.37 ms with 4x2, 1.39 with 4x2s; 4096^2, 200 steps: 445 and 455 us).  With
 // four planes one wavefront's registers leave two or three a SIMD and the
 // split tiles are faster (8192^2, twelve materials, 64 steps: 646 us with 4x2s, 758).
+// Only the kernels of large worlds sleep: with se_sl_sleeps in them the split tiles' main
+// loops came out with other registers and moves (us a call, split tiles with / without: feature
+// rules 1296x67 557 steps 417 / 409, 618x119 107 steps 104 / 103).
 #if SE_SL_K <= 3
-SE_SL_STEP(2, 2, 1, 4, 3, 2x2)
-SE_SL_STEP(4, 2, 1, 2, 3, 4x2)
+SE_SL_STEP(2, 2, 1, 4, 3, true, 2x2)
+SE_SL_STEP(4, 2, 1, 2, 3, true, 4x2)
+#else
+SE_SL_STEP(1, 2, 2, 4, 1, true, 2x2z)
+SE_SL_STEP(1, 2, 4, 4, 1, true, 4x2z)
 #endif
 
 // ---------------------------------------------------------------------------

@@ -92,6 +92,8 @@ int sliced_unpack_columns(const SlicedGrid& g);
 // Do the modifications of a run's first step go into the packed grid (else that step is
 // for the plain kernel)?
 bool sliced_takes_mods(const se_world* w, uint32_t n);
+// Do the step kernel's tiles sleep (K.sleep_step in place of K.step)?
+bool sliced_sleeps(const se_world* w, int kernel);
 // Advances w by n steps (no clearing frame among them; queued modifications follow the
 // first), launches of up to `sub` sub-steps.  *done = false and nothing enqueued
 // when the scratch memory cannot be had.
