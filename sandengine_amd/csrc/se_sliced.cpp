@@ -365,7 +365,7 @@ se_rt::SlicedShape se_rt::sliced_shape(const SlicedKernels& K, uint32_t W, uint3
 // 2304x2112 54 / 58, 2816x2880 73 / 74, 4096^2 115 / 105, 8192^2 292 / 236; feature rules 62 / 65,
 // 85 / 85, 131 / 121, 301 / 247; settled four materials 40 / 39, 52 / 45, 84 / 57, 222 / 87).
 bool se_rt::sliced_takes_mods(const se_world* w, uint32_t n) {
-    return n > 1 && sliced_squares(w->W, w->H) >= kKnownSquares;
+    return n > 1 && sliced_squares(w->W, w->H) > kFewSquares;
 }
 
 bool se_rt::sliced_sleeps(const se_world* w, int kernel) {

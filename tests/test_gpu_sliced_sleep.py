@@ -137,8 +137,8 @@ def test_a_caller_with_the_grids_address_writes_between_runs():
 @pytest.mark.parametrize("name", ["four_materials", "features"])
 @pytest.mark.parametrize("size", [(1, 1), (124, 126), (700, 333), (70001, 3), (3, 70001), (2081, 2047)], ids=lambda s: f"{s[0]}x{s[1]}")
 def test_modifications_of_the_first_step(name, size):
-    """Worlds whose first step is a plain one and worlds that take them into the packed grid
-    (from 1024 squares on), against the oracle: lists that travel by value and lists that do not, overlapping
+    """Worlds whose first step is a plain one, and beyond 2048 squares worlds that take them into
+    the packed grid, against the oracle: lists that travel by value and lists that do not, overlapping
     boxes, later entries over earlier ones, NULL materials that hide them, a list cut at
     size 0, boxes larger than the world, beside it and across its sides."""
     W, H = size

@@ -23,3 +23,10 @@ def test_kernels_whose_tiles_sleep_are_named():
         w.set_sleep(False)
         assert w.variant_info(4, 24)[:2] == (1, dense)
         w.close()
+
+
+@pytest.mark.parametrize("name", ["four_materials", "features"])
+@pytest.mark.parametrize("size", [(2049, 4097), (32801, 257)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_modifications_of_the_first_step(name, size):
+    """Lists that go into the packed grid."""
+    Z.test_modifications_of_the_first_step(name, size)
